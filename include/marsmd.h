@@ -520,8 +520,9 @@ marsmd_status marsmd_patch_autotune(marsmd_patch* p, const marsmd_run_params* pa
                                     marsmd_stream stream);
 /* Cell configuration of the Patch's pairlist walk: home cells (one wave's tile of home
  * particles) of the finest Morton level that holds home_target particles on average
- * (1 .. 4096, default 24), candidate cells fine_offset levels below (1 .. 4, default
- * 2). The pair set does not depend on it; the order of neighbours in a row, and so the
+ * (1 .. 4096), candidate cells fine_offset levels below (1 .. 4). Until it is set or
+ * tuned the library chooses the cells from the particle count (and get_cells reports 24
+ * and 2). The pair set does not depend on it; the order of neighbours in a row, and so the
  * FP32 summation order of the forces, does. Applies from the next build. No
  * counterpart in the reference (its cell grid is select_cell_grid's,
  * ZOrderPairlist.cpp:24-81). */
@@ -623,7 +624,8 @@ marsmd_status marsmd_batch_autotune(marsmd_batch* b, const marsmd_run_params* pa
  * are the finest Morton cells that still hold home_target[b] particles on average,
  * the candidate cells lie fine_offset[b] Morton levels below them. The pair set does
  * not depend on it; the order of neighbours in a row, and so the FP32 summation order
- * of the forces, does. Defaults: 24 and 2. No counterpart in the reference (its cell
+ * of the forces, does. A bucket left at 24 and 2, the defaults, has its cells chosen by
+ * the library from the particle counts. No counterpart in the reference (its cell
  * grid is ZOrderPairlist::select_cell_grid's, ZOrderPairlist.cpp:24-81). */
 #define MARSMD_BATCH_BUCKETS 32
 typedef struct marsmd_batch_cells {

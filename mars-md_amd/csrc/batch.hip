@@ -279,12 +279,10 @@ __global__ void k_b_gather(const uint32_t* __restrict__ old_slot, uint64_t total
 }
 
 // Fine and home cell ranges of every replica (BuildCellRangesKernel, ZOrderNeighbor.h:27-43,
-// per replica), in global slots.
+// per replica) as {begin, end} in global slots.
 __global__ void k_b_cell_ranges(const uint32_t* __restrict__ codes, uint64_t total,
 								const uint32_t* __restrict__ rep_of_slot, const RepGeom* __restrict__ geom,
-								uint32_t* __restrict__ fine_begin, uint32_t* __restrict__ fine_end,
-								uint32_t* __restrict__ home_begin, uint32_t* __restrict__ home_end,
-								uint32_t* __restrict__ flags) {
+								uint2* __restrict__ fine, uint2* __restrict__ home, uint32_t* __restrict__ flags) {
 	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
 	if (i >= total)
 		return;
@@ -292,41 +290,36 @@ __global__ void k_b_cell_ranges(const uint32_t* __restrict__ codes, uint64_t tot
 	const bool first = i == G.slot0;
 	const bool last = i + 1 == uint64_t(G.slot0) + G.n;
 	const uint32_t c = codes[i];
+	const uint32_t cp = first ? ~c : codes[i - 1], cn = last ? ~c : codes[i + 1];
 	// the gather recomputes each code from the position it moves: codes out of order
 	// within a replica (a mismatch with the sort's keys) would give wrong cell ranges
-	if (!first && codes[i - 1] > c && flags)
+	if (!first && cp > c && flags)
 		atomicOr(flags, 2u);
 	const int fs = 3 * (10 - G.mf), hs = 3 * (10 - G.h);
 	const uint32_t fc = c >> fs, hc = c >> hs;
-	if (first || (codes[i - 1] >> fs) != fc)
-		fine_begin[G.fine_off + fc] = uint32_t(i);
-	if (last || (codes[i + 1] >> fs) != fc)
-		fine_end[G.fine_off + fc] = uint32_t(i + 1);
-	if (first || (codes[i - 1] >> hs) != hc)
-		home_begin[G.home_off + hc] = uint32_t(i);
-	if (last || (codes[i + 1] >> hs) != hc)
-		home_end[G.home_off + hc] = uint32_t(i + 1);
+	if (first || (cp >> fs) != fc)
+		fine[G.fine_off + fc].x = uint32_t(i);
+	if (last || (cn >> fs) != fc)
+		fine[G.fine_off + fc].y = uint32_t(i + 1);
+	if (first || (cp >> hs) != hc)
+		home[G.home_off + hc].x = uint32_t(i);
+	if (last || (cn >> hs) != hc)
+		home[G.home_off + hc].y = uint32_t(i + 1);
 }
 
 // The home-cell walk over the work items of all replicas (item_off[r] = first item of
-// replica r, one item per home cell), at 6 waves per SIMD (80 VGPRs) as the Patch's walk:
-// more waves hide the per-home-particle LDS reads.
+// replica r, one item per home cell).
 __global__ __launch_bounds__(256, 6) void k_b_walk(const RepGeom* __restrict__ geom, const uint32_t* __restrict__ item_off,
 												uint32_t R, uint32_t num_items, const float4* __restrict__ spos,
-												const uint32_t* __restrict__ home_begin,
-												const uint32_t* __restrict__ home_end,
-												const uint32_t* __restrict__ fine_begin,
-												const uint32_t* __restrict__ fine_end, float rc2, uint32_t cap,
-												const int4* __restrict__ stencils, uint32_t* __restrict__ counts,
+												const uint2* __restrict__ home, const uint2* __restrict__ fine,
+												float rc2, uint32_t cap, const uint32_t* __restrict__ stencils,
+												uint32_t* __restrict__ counts,
 												uint32_t* __restrict__ nbr) {
-	__shared__ uint32_t seg_b[kHomeWaves][kSegMax];
-	__shared__ uint32_t seg_pre[kHomeWaves][kSegMax + 1];
-	__shared__ float4 home_pos[kHomeWaves][kHomeLds];
-	__shared__ uint32_t keep[kHomeWaves][kHomeKeep];
+	__shared__ WalkLds lds[kHomeWaves];
 	const int wv = threadIdx.x >> 6;
 	const TileRange TR = xcd_tiles((num_items + kHomeWaves - 1) / kHomeWaves);
 	for (uint32_t gidx = TR.tile; gidx < TR.end; gidx += TR.stride) {
-		const uint32_t item = gidx * kHomeWaves + uint32_t(wv);
+		const uint32_t item = uint32_t(__builtin_amdgcn_readfirstlane(int(gidx * kHomeWaves + uint32_t(wv))));
 		if (item >= num_items)
 			continue;
 		uint32_t lo = 0, hi = R; // item_off[lo] <= item < item_off[hi]
@@ -341,10 +334,8 @@ __global__ __launch_bounds__(256, 6) void k_b_walk(const RepGeom* __restrict__ g
 		const RepGeom& G = geom[r];
 		HomeParams P{};
 		P.spos = spos;
-		P.home_begin = home_begin + G.home_off;
-		P.home_end = home_end + G.home_off;
-		P.fine_begin = fine_begin + G.fine_off;
-		P.fine_end = fine_end + G.fine_off;
+		P.home = home + G.home_off;
+		P.fine = fine + G.fine_off;
 		P.num_home = uint32_t(1) << (3 * G.h);
 		P.h = G.h;
 		P.s = G.mf - G.h;
@@ -370,9 +361,16 @@ __global__ __launch_bounds__(256, 6) void k_b_walk(const RepGeom* __restrict__ g
 		P.pre = G.pre;
 		P.pre_lo2 = G.pre_lo2;
 		P.pre_hi2 = G.pre_hi2;
-		P.stencil = G.stencil_n ? stencils + G.stencil_off : nullptr;
+		P.stencil_code = G.stencil_n ? stencils + G.stencil_off : nullptr;
 		P.stencil_n = G.stencil_n;
-		walk_home_cell<true>(P, item - item_off[r], seg_b[wv], seg_pre[wv], home_pos[wv], keep[wv], counts, nbr);
+		const uint32_t cell = item - item_off[r];
+		const uint2 hr = P.home[cell];
+		const uint32_t from = uint32_t(__builtin_amdgcn_readfirstlane(int(hr.x)));
+		const uint32_t to = uint32_t(__builtin_amdgcn_readfirstlane(int(hr.y)));
+		if (walk_mode(P) == kWalkPlain)
+			walk_home_cell<kWalkPlain>(P, cell, from, to, lds[wv], counts, nbr);
+		else
+			walk_home_cell<kWalkGeneral>(P, cell, from, to, lds[wv], counts, nbr);
 	}
 }
 
@@ -848,11 +846,11 @@ void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<ui
 		int m = 0;
 		while (m < 10 && (uint64_t(1) << (3 * (m + 1))) <= 2 * std::max<uint64_t>(n, 1))
 			++m;
-		int h = 0;
-		while (h + 1 <= m - 1 && (n >> (3 * (h + 1))) >= target)
-			++h;
+		const WalkLevel lv = walk_level(n, m, cells_auto[size_t(bucket)] ? 0 : int(target), cell_fine[size_t(bucket)],
+										kWalkFill * double(n) / double(total));
+		const int h = lv.h;
 		g.h = h;
-		g.mf = std::min(10, h + std::max(1, cell_fine[size_t(bucket)]));
+		g.mf = std::min(10, h + lv.s);
 		const int fine_cells = 1 << g.mf;
 		const int span = 1 << (g.mf - h);
 		const int k = 1024 / fine_cells;
@@ -894,7 +892,8 @@ void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<ui
 		if (it == stencil_index.end()) {
 			const std::vector<int4> st = home_stencil(h, g.mf - h, g.reach, g.full, g.cw, g.margin, rc2, 8192);
 			it = stencil_index.emplace(key, std::make_pair(uint32_t(stencils_host.size()), uint32_t(st.size()))).first;
-			stencils_host.insert(stencils_host.end(), st.begin(), st.end());
+			for (const int4& o : st)
+				stencils_host.push_back(stencil_offset_code(o, g.mf));
 		}
 		g.stencil_off = it->second.first;
 		g.stencil_n = it->second.second;
@@ -910,7 +909,7 @@ void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<ui
 		raise(MARSMD_ERR_VALUE, "batch: cell tables exceed 2^32 entries");
 	if (stencils_host.size() > stencils_uploaded) { // new geometries (a synchronous upload, rare)
 		stencils.resize(stencils_host.size());
-		MMD_HIP(hipMemcpy(stencils.data(), stencils_host.data(), sizeof(int4) * stencils_host.size(),
+		MMD_HIP(hipMemcpy(stencils.data(), stencils_host.data(), sizeof(uint32_t) * stencils_host.size(),
 						  hipMemcpyHostToDevice));
 		stencils_uploaded = stencils_host.size();
 	}
@@ -923,7 +922,7 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 	// the plan depends on the cutoff, the cell configuration and the pair bookkeeping
 	// (boxes and sizes are fixed): planned again only when one of them changed, which
 	// keeps it off the GPU's idle time when a run starts with a rebuild
-	if (!(plan.valid && plan.rc == rc && plan.target == cell_target && plan.fine == cell_fine &&
+	if (!(plan.valid && plan.rc == rc && plan.target == cell_target && plan.fine == cell_fine && plan.own == cells_auto &&
 		  plan.ref == ref_max_pairs)) {
 		plan.valid = false; // until planned whole
 		plan_geometry(rc, geom_host, items, plan.fine_total, plan.home_total);
@@ -931,6 +930,7 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 		plan.rc = rc;
 		plan.target = cell_target;
 		plan.fine = cell_fine;
+		plan.own = cells_auto;
 		plan.ref = ref_max_pairs;
 	}
 	const uint64_t fine_total = plan.fine_total, home_total = plan.home_total;
@@ -988,17 +988,12 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 	ids.swap(ids_tmp);
 	slot_of_canon.swap(slot_of_canon_tmp);
 	// cell tables
-	fine_begin.resize(num_fine);
-	fine_end.resize(num_fine);
-	home_begin.resize(num_home);
-	home_end.resize(num_home);
-	fill_u32(fine_begin.data(), 0u, num_fine, s);
-	fill_u32(fine_end.data(), 0u, num_fine, s);
-	fill_u32(home_begin.data(), 0u, num_home, s);
-	fill_u32(home_end.data(), 0u, num_home, s);
-	k_b_cell_ranges<<<grid_for(total, 256), 256, 0, s>>>(codes.data(), total, rep_of_slot.data(), gd,
-														 fine_begin.data(), fine_end.data(), home_begin.data(),
-														 home_end.data(), scalars.data());
+	cells.resize(num_fine + num_home);
+	uint2* const fine = cells.data();
+	uint2* const home = fine + num_fine;
+	fill_u32(reinterpret_cast<uint32_t*>(fine), 0u, 2 * (num_fine + num_home), s);
+	k_b_cell_ranges<<<grid_for(total, 256), 256, 0, s>>>(codes.data(), total, rep_of_slot.data(), gd, fine, home,
+														 scalars.data());
 	MMD_LAUNCH_CHECK();
 	// walk with uniform rows of `cap` entries; once more with larger rows if needed
 	const uint64_t tiles = (total + 63) / 64;
@@ -1022,8 +1017,7 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 		k_b_uniform_tile_base<<<grid_for(tiles + 1, 256), 256, 0, s>>>(tile_base.data(), tiles, 64u * cap);
 		MMD_LAUNCH_CHECK();
 		k_b_walk<<<grid, 256, 0, s>>>(gd, item_off.data(), uint32_t(R), uint32_t(num_items), pos[cur].data(),
-									  home_begin.data(), home_end.data(), fine_begin.data(), fine_end.data(), rc2,
-									  cap, stencils.data(), counts.data(), nbr.data());
+									  home, fine, rc2, cap, stencils.data(), counts.data(), nbr.data());
 		MMD_LAUNCH_CHECK();
 		fill_u32(scalars.data() + 2, 0u, 4, s);
 		k_b_count_stats<<<std::min<unsigned>(grid_for(total, 256), 240), 256, 0, s>>>(
@@ -1325,6 +1319,9 @@ void BatchImpl::set_cells(const marsmd_batch_cells& c) {
 			raise(MARSMD_ERR_VALUE, "batch: fine_offset must be in [1, 4]");
 	}
 	for (int b = 0; b < kBatchBuckets; ++b) {
+		// a bucket set to what it already says keeps the library's own choice
+		cells_auto[size_t(b)] = cells_auto[size_t(b)] && cell_target[size_t(b)] == c.home_target[b] &&
+								cell_fine[size_t(b)] == c.fine_offset[b];
 		cell_target[size_t(b)] = c.home_target[b];
 		cell_fine[size_t(b)] = c.fine_offset[b];
 	}
@@ -1346,10 +1343,9 @@ double BatchImpl::walk_ms(hipStream_t s) {
 	MMD_HIP(hipMemcpyAsync(t_geom.data(), gh.data(), R * sizeof(RepGeom), hipMemcpyHostToDevice, s));
 	t_items.resize(R + 1);
 	MMD_HIP(hipMemcpyAsync(t_items.data(), items.data(), 4 * (R + 1), hipMemcpyHostToDevice, s));
-	t_fine_begin.resize(ft);
-	t_fine_end.resize(ft);
-	t_home_begin.resize(ht);
-	t_home_end.resize(ht);
+	t_cells.resize(ft + ht);
+	uint2* const fine = t_cells.data();
+	uint2* const home = fine + ft;
 	t_counts.resize(total);
 	const uint64_t storage = (total + 63) / 64 * 64 * uint64_t(cap);
 	t_nbr.resize(std::max<uint64_t>(storage, 1));
@@ -1362,16 +1358,11 @@ double BatchImpl::walk_ms(hipStream_t s) {
 	const unsigned groups = unsigned((nitems + kHomeWaves - 1) / kHomeWaves);
 	const unsigned grid = std::max(8u, (groups + 7u) / 8u * 8u);
 	MMD_HIP(hipEventRecord(t_events[0], s));
-	fill_u32(t_fine_begin.data(), 0u, ft, s);
-	fill_u32(t_fine_end.data(), 0u, ft, s);
-	fill_u32(t_home_begin.data(), 0u, ht, s);
-	fill_u32(t_home_end.data(), 0u, ht, s);
-	k_b_cell_ranges<<<grid_for(total, 256), 256, 0, s>>>(codes.data(), total, rep_of_slot.data(), gd,
-														 t_fine_begin.data(), t_fine_end.data(), t_home_begin.data(),
-														 t_home_end.data(), nullptr);
+	fill_u32(reinterpret_cast<uint32_t*>(fine), 0u, 2 * (ft + ht), s);
+	k_b_cell_ranges<<<grid_for(total, 256), 256, 0, s>>>(codes.data(), total, rep_of_slot.data(), gd, fine, home,
+														 nullptr);
 	MMD_LAUNCH_CHECK();
-	k_b_walk<<<grid, 256, 0, s>>>(gd, t_items.data(), uint32_t(R), uint32_t(nitems), snap.data(), t_home_begin.data(),
-								  t_home_end.data(), t_fine_begin.data(), t_fine_end.data(),
+	k_b_walk<<<grid, 256, 0, s>>>(gd, t_items.data(), uint32_t(R), uint32_t(nitems), snap.data(), home, fine,
 								  built_cutoff * built_cutoff, cap, stencils.data(), t_counts.data(), t_nbr.data());
 	MMD_LAUNCH_CHECK();
 	MMD_HIP(hipEventRecord(t_events[1], s));
@@ -1411,9 +1402,11 @@ void BatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, 
 	// one bucket at a time, the others held; a candidate must beat the incumbent by 1%
 	for (int b : present) {
 		int bt = cell_target[size_t(b)], bf = cell_fine[size_t(b)];
+		bool own = cells_auto[size_t(b)]; // the library's own choice, until a candidate beats it
+		cells_auto[size_t(b)] = false;
 		for (int t : targets)
 			for (int f : fines) {
-				if (t == bt && f == bf)
+				if (!own && t == bt && f == bf)
 					continue;
 				cell_target[size_t(b)] = t;
 				cell_fine[size_t(b)] = f;
@@ -1422,10 +1415,12 @@ void BatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, 
 					best = ms;
 					bt = t;
 					bf = f;
+					own = false;
 				}
 			}
 		cell_target[size_t(b)] = bt;
 		cell_fine[size_t(b)] = bf;
+		cells_auto[size_t(b)] = own;
 	}
 	*walk_out = best < 1e300 ? best : 0.0;
 	if (step < first_step + num_steps)

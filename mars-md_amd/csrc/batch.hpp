@@ -33,7 +33,8 @@ struct BatchImpl {
 	// rebuild
 	DevArray<uint32_t> keys, vals, keys_s, vals_s, rkeys, rvals, rkeys_s, rvals_s, codes, perm;
 	DevArray<uint8_t> sort_scratch, geom;
-	DevArray<uint32_t> fine_begin, fine_end, home_begin, home_end, item_off;
+	DevArray<uint2> cells; // every replica's fine cells, then home cells: {begin, end}
+	DevArray<uint32_t> item_off;
 	DevArray<uint32_t> counts, tile_base, nbr, scalars;
 	DevArray<int32_t> pairs;
 	DevArray<uint32_t> half_counts, half_offsets;
@@ -44,14 +45,15 @@ struct BatchImpl {
 	// fine-cell stencils of the home walk, one per distinct replica geometry (key: the
 	// walk parameters it depends on; value: offset and count in stencils)
 	std::map<std::vector<float>, std::pair<uint32_t, uint32_t>> stencil_index;
-	std::vector<int4> stencils_host;
-	DevArray<int4> stencils;
+	std::vector<uint32_t> stencils_host; // Morton codes of the offsets
+	DevArray<uint32_t> stencils;
 	size_t stencils_uploaded = 0;
 	std::vector<uint32_t> items_host;
 	struct Plan { // what geom_host and items_host were planned from
 		bool valid = false;
 		float rc = 0.0f;
 		std::vector<int> target, fine;
+		std::vector<uint8_t> own;
 		std::vector<uint64_t> ref;
 		uint64_t fine_total = 0, home_total = 0;
 	} plan;
@@ -85,9 +87,12 @@ struct BatchImpl {
 	// cell_target particles on average; its fine cells lie cell_fine levels below
 	std::vector<int> cell_target = std::vector<int>(size_t(kBatchBuckets), 24);
 	std::vector<int> cell_fine = std::vector<int>(size_t(kBatchBuckets), 2);
+	// buckets neither set nor tuned, whose cells walk_level chooses
+	std::vector<uint8_t> cells_auto = std::vector<uint8_t>(size_t(kBatchBuckets), 1);
 	// scratch of the walk timing (the live list is untouched)
 	DevArray<uint8_t> t_geom;
-	DevArray<uint32_t> t_items, t_fine_begin, t_fine_end, t_home_begin, t_home_end, t_counts, t_nbr;
+	DevArray<uint32_t> t_items, t_counts, t_nbr;
+	DevArray<uint2> t_cells;
 	hipEvent_t t_events[2] = {nullptr, nullptr};
 
 	explicit BatchImpl(const marsmd_batch_desc& d);

@@ -13,14 +13,9 @@ namespace mmd {
 
 namespace {
 
-// Canonical pair predicate of ZOrderCellNeighborKernel for sorted lo < hi
-// (ZOrderNeighbor.h:204-221): wrap_diff(pos_hi - pos_lo)^2 <= rc^2, not excluded by
-// lo's CSR row or a shared rigid body.
-__device__ __forceinline__ bool pair_predicate(const DevBox& box, float rc2, const marsmd_exclusion_view& ex,
-											   const float4& plo, const float4& phi) {
-	const float3 dr = wrap_diff(box, sub3(phi, plo));
-	if (!(len2(dr) <= rc2))
-		return false;
+// Not excluded by lo's CSR row or a shared rigid body.
+__device__ __forceinline__ bool pair_unexcluded(const marsmd_exclusion_view& ex, const float4& plo,
+												const float4& phi) {
 	const int a = int(meta_canon(__float_as_uint(plo.w)));
 	const int b = int(meta_canon(__float_as_uint(phi.w)));
 	if (ex.rigid_body_id) {
@@ -37,45 +32,44 @@ __device__ __forceinline__ bool pair_predicate(const DevBox& box, float rc2, con
 	return true;
 }
 
-// pair_predicate for a home particle pi (slot ti) and a candidate q (slot j != ti),
-// oriented by slot: the difference phi - plo is q - pi or its exact negation (rounding
-// is sign-symmetric), so the orientation costs three selects; the metadata of the two
-// ends is only looked at when exclusions or rigid bodies are given.
-__device__ __forceinline__ bool pair_predicate_home(const DevBox& box, float rc2, const marsmd_exclusion_view& ex,
-													const float4& pi, uint32_t ti, const float4& q, uint32_t j) {
-	const bool t_lo = j > ti;
-	const float dx = q.x - pi.x, dy = q.y - pi.y, dz = q.z - pi.z;
-	const float3 dr = wrap_diff(box, t_lo ? make_float3(dx, dy, dz) : make_float3(-dx, -dy, -dz));
-	if (!(len2(dr) <= rc2))
-		return false;
-	if (!ex.rigid_body_id && !ex.offsets)
-		return true;
-	return pair_predicate(box, rc2, ex, t_lo ? pi : q, t_lo ? q : pi);
+// Canonical pair predicate of ZOrderCellNeighborKernel for sorted lo < hi
+// (ZOrderNeighbor.h:204-221): wrap_diff(pos_hi - pos_lo)^2 <= rc^2, and not excluded.
+__device__ __forceinline__ bool pair_predicate(const DevBox& box, float rc2, const marsmd_exclusion_view& ex,
+											   const float4& plo, const float4& phi) {
+	const float3 dr = wrap_diff(box, sub3(phi, plo));
+	return len2(dr) <= rc2 && pair_unexcluded(ex, plo, phi);
 }
+
 // ------------------------------------------------------------ home-cell walk
 // One wave per home cell: a Morton cell of the home level h, whose particles are
 // contiguous in sorted order. The wave enumerates the fine cells (level m = h + s)
-// within `reach` fine cells of the home cell, keeps those whose box can lie within rc
-// of the home cell's box (both widened by the quantisation margin, so the test is
-// conservative across the periodic seam), stores their particle ranges as segments
-// in LDS, then streams the candidates 64 at a time (one coalesced load per lane) and
-// tests them against the wave's home particles, which are broadcast from LDS.
+// within `reach` fine cells of the home cell whose box can lie within rc of the home
+// cell's box (both widened by the quantisation margin, so the test is conservative
+// across the periodic seam), 64 cells at a time, spreads their particles over its lanes,
+// drops those farther than rc from the bounding box of the home particles, queues the
+// rest in LDS and tests each full queue of 64 against the home particles one by one (a
+// home particle is wave-uniform: scalar loads). The hits of a home particle are one
+// 64-bit mask; each hit lane writes its slot at the row's end plus its rank in the mask.
 // Predicate and orientation are k_walk's (the reference's), so the pair set is the
 // same; a particle's list is in candidate order. Entries past `cap` are not written
 // (the host sees the count and walks again with a larger cap).
+//
+// What bounds it: with thousands of cells per SIMD the VALU instructions of the tests
+// (17 a home particle and 64 candidates), with few the chain of one wave: cell ranges ->
+// positions -> queue -> tests. Both want cells with few particles while the chip is not
+// full (walk_level), and no search per candidate: the earlier form kept the cells of the
+// whole stencil as LDS segments, found each candidate's by bisection (9 dependent LDS
+// reads) and appended each home particle's hits in a per-lane loop.
 constexpr int kHomeWaves = 4;
-constexpr int kSegMax = 448;
-// LDS per wave for the home particles: 64 positions, then 64 candidate slots
-constexpr int kHomeLds = 64 + 16;
-// LDS per wave for the queue of candidates kept by the bounding-box test
-constexpr int kHomeKeep = 128;
+// home cells that occupy the chip: four waves on each of its 1024 SIMDs
+constexpr double kWalkFill = 4096.0;
+// candidates of one 64-cell step mapped to lanes at a time (start bits in LDS)
+constexpr uint32_t kWalkWindow = 1024;
 
 struct HomeParams {
 	const float4* spos;
-	const uint32_t* home_begin;
-	const uint32_t* home_end;
-	const uint32_t* fine_begin;
-	const uint32_t* fine_end;
+	const uint2* home; // {begin, end} of every home cell
+	const uint2* fine; // {begin, end} of every fine cell
 	uint32_t num_home;
 	int h;         // home level
 	int s;         // fine level m = h + s
@@ -86,6 +80,10 @@ struct HomeParams {
 	float rc2;
 	DevBox box;
 	marsmd_exclusion_view ex;
+	// the sorted slot of every canonical index, when the exclusion rows are symmetric (a
+	// in b's row exactly when b is in a's): a home particle's own row then decides all of
+	// its pairs and is read once, as slots; null: each pair looks at its lower end's row
+	const uint32_t* ex_slot;
 	uint32_t cap;  // entries per slot the uniform tile rows hold
 	// When the reference cell grid misses pairs at the periodic seam, only the pairs its
 	// stencil reaches are kept: cells (quantised coordinate >> ref_shift) within
@@ -104,19 +102,22 @@ struct HomeParams {
 	// for that move to give the minimum image of every pair within the cutoff.
 	int pre;
 	float pre_lo2, pre_hi2;
-	// The fine cells the walk enumerates, when given: per entry the cell offset from the
-	// home cell's first fine cell on each axis (the absolute cell on an axis enumerated
-	// whole), in enumeration order, for the cells that pass the gap test; null: every
-	// cell of the reach is enumerated and gap-tested per home cell.
+	// The fine cells the walk enumerates, when given: their offsets from the home cell's
+	// first fine cell (the absolute cell on an axis enumerated whole) that pass the gap
+	// test, in enumeration order. In a box periodic on every axis an offset is the Morton
+	// code of its three components modulo the cells (stencil_code, added to the home
+	// cell's code axis by axis on the interleaved bits, which wraps by itself); else three
+	// integers (stencil). Neither: every cell of the reach is enumerated and gap-tested.
+	const uint32_t* stencil_code;
 	const int4* stencil;
 	uint32_t stencil_n;
 };
 
 // The fine cells of the walk's enumeration that pass its gap test, as offsets (see
-// HomeParams::stencil), in its order (x fastest); empty when there are more than
-// max_cells of them. The test is the walk's own: per axis not enumerated whole, the
-// number of cells between the cell and the home cell's span times the cell width, less
-// twice the margin, floored at 0, squared and summed, against rc^2.
+// HomeParams::stencil); empty when there are more than max_cells of them. The test is
+// the walk's own: per axis not enumerated whole, the number of cells between the cell
+// and the home cell's span times the cell width, less twice the margin, floored at 0,
+// squared and summed, against rc^2.
 inline std::vector<int4> home_stencil(int h, int s, const int reach[3], const int full[3], const float cw[3],
 									  const float margin[3], float rc2, size_t max_cells) {
 	const int fine_cells = 1 << (h + s), span = 1 << s;
@@ -145,7 +146,7 @@ inline std::vector<int4> home_stencil(int h, int s, const int reach[3], const in
 				}
 			}
 	// Morton order of the offsets: 64 consecutive candidates then come from a compact
-	// cluster of cells, which a home particle's cutoff sphere often misses as a whole
+	// cluster of cells
 	auto key = [](const int4& c) {
 		uint64_t k = 0;
 		const uint32_t v[3] = {uint32_t(c.x + 1024), uint32_t(c.y + 1024), uint32_t(c.z + 1024)};
@@ -156,6 +157,36 @@ inline std::vector<int4> home_stencil(int h, int s, const int reach[3], const in
 	};
 	std::stable_sort(out.begin(), out.end(), [&](const int4& a, const int4& b) { return key(a) < key(b); });
 	return out;
+}
+// The walk's home level h and its fine cells' depth s below it. target > 0: the finest
+// level holding `target` particles per home cell on average, and `offset`. Else the
+// library's own choice for n particles (fine cells = home cells, which the candidates'
+// bounding-box test prunes more cheaply than a larger stencil does): a level finer while
+// its cells hold 5 particles on average, or (`fill`: home cells that occupy the chip) 1
+// while there are fewer cells than that. Walk times (us; one beads type, cutoff 35):
+// 10k beads at 6.4e-4 per A^3: level 2 (156 a cell) 642, 3 (20) 54, 4 (2.4) 21; 60k at
+// 1.25e-4: 3 (117) 240, 4 (15) 31, 5 (1.8) 44; 250k: 4 (61) 150, 5 (7.6) 67; 1M: 5 (30)
+// 261, 6 (3.8) 375.
+struct WalkLevel {
+	int h, s;
+};
+inline WalkLevel walk_level(uint64_t n, int m, int target, int offset, double fill, uint64_t per_cell = 4) {
+	int h = 0;
+	if (target > 0) {
+		while (h + 1 <= m && (n >> (3 * (h + 1))) >= uint64_t(target))
+			++h;
+		return WalkLevel{h, offset};
+	}
+	while (h + 1 <= m && ((n >> (3 * (h + 1))) >= per_cell || double(uint64_t(1) << (3 * h)) < fill))
+		++h;
+	return WalkLevel{h, 0};
+}
+
+// An offset of home_stencil as the Morton code of its components modulo 2^level cells.
+inline uint32_t stencil_offset_code(const int4& o, int level) {
+	const uint32_t mask = (1u << level) - 1u;
+	return split_by3(uint32_t(o.z) & mask) | (split_by3(uint32_t(o.y) & mask) << 1) |
+		   (split_by3(uint32_t(o.x) & mask) << 2);
 }
 
 // The prefilter's band for a domain [lo, hi) whose home cells (level h) have width
@@ -206,21 +237,48 @@ __device__ __forceinline__ bool in_reference_stencil(const HomeParams& P, const 
 	return true;
 }
 
-__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
-	const int lane = threadIdx.x & 63;
-#pragma unroll
-	for (int o = 1; o < 64; o <<= 1) {
-		const uint32_t t = __shfl_up(v, o, 64);
-		if (lane >= o)
-			v += t;
-	}
-	return v;
+// Wave-wide scans and reductions on the DPP crossbar: row shifts within 16 lanes, then
+// the row broadcasts (lane 15 of rows 0 and 2 into the next row, lane 31 into rows 2 and 3).
+template<int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_add(uint32_t v) {
+	return v + uint32_t(__builtin_amdgcn_update_dpp(0, int(v), CTRL, ROWS, 0xf, false));
 }
-__device__ __forceinline__ uint32_t bcast_u32(uint32_t v, uint32_t lane) {
-	return uint32_t(__builtin_amdgcn_readlane(int(v), int(lane)));
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
+	v = dpp_add<0x111, 0xf>(v); // row_shr:1
+	v = dpp_add<0x112, 0xf>(v);
+	v = dpp_add<0x114, 0xf>(v);
+	v = dpp_add<0x118, 0xf>(v);
+	v = dpp_add<0x142, 0xa>(v); // row_bcast:15 into rows 1 and 3
+	return dpp_add<0x143, 0xc>(v); // row_bcast:31 into rows 2 and 3
 }
 __device__ __forceinline__ float bcast_f32(float v, uint32_t lane) {
 	return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), int(lane)));
+}
+template<int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_min(float v) {
+	const int x = __float_as_int(v);
+	return fminf(v, __int_as_float(__builtin_amdgcn_update_dpp(x, x, CTRL, ROWS, 0xf, false)));
+}
+__device__ __forceinline__ float wave_min(float v) {
+	v = dpp_min<0x111, 0xf>(v);
+	v = dpp_min<0x112, 0xf>(v);
+	v = dpp_min<0x114, 0xf>(v);
+	v = dpp_min<0x118, 0xf>(v);
+	v = dpp_min<0x142, 0xa>(v);
+	v = dpp_min<0x143, 0xc>(v);
+	return bcast_f32(v, 63);
+}
+__device__ __forceinline__ float wave_max(float v) { return -wave_min(-v); }
+__device__ __forceinline__ uint32_t bcast_u32(uint32_t v, uint32_t lane) {
+	return uint32_t(__builtin_amdgcn_readlane(int(v), int(lane)));
+}
+// Number of set bits of the wave-uniform mask m below this lane.
+__device__ __forceinline__ uint32_t bits_below(uint64_t m) {
+	return uint32_t(__builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u)));
+}
+// Lane i (wave-uniform) of v takes the wave-uniform x.
+__device__ __forceinline__ void set_lane(uint32_t& v, uint32_t x, uint32_t i) {
+	asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(x), "{m0}"(i));
 }
 // LDS written by some lanes of this wave and read by others: order the accesses.
 __device__ __forceinline__ void wave_lds_sync() {
@@ -229,349 +287,345 @@ __device__ __forceinline__ void wave_lds_sync() {
 	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The hits of the wave's nh home particles (visited one by one from LDS, the next one
-// read ahead) among one block of up to 64 candidates (lane: slot j, position q) by the
-// reference's predicate: the mask over the block's lanes of home particle i, in lane i.
-// Lane i (< 64, wave-uniform) of the 64-bit per-lane mask {lo, hi} takes the wave-uniform
-// mask m: one v_writelane per half, the lane in M0 (a select over lanes would take a
-// compare, two moves of the mask into vector registers and two selects).
-__device__ __forceinline__ void set_lane_mask(int& lo, int& hi, uint64_t m, uint32_t i) {
-	const uint32_t mlo = uint32_t(m), mhi = uint32_t(m >> 32);
-	asm("v_writelane_b32 %0, %1, %2" : "+v"(lo) : "s"(mlo), "{m0}"(i));
-	asm("v_writelane_b32 %0, %1, %2" : "+v"(hi) : "s"(mhi), "{m0}"(i));
-}
-__device__ __forceinline__ uint64_t lane_mask(int lo, int hi) {
-	return uint64_t(uint32_t(lo)) | (uint64_t(uint32_t(hi)) << 32);
+// LDS of one wave of the walk.
+struct WalkLds {
+	float4 keep[128];                    // queued candidates {position, slot}
+	uint32_t delta[64];                  // slot less index of each nonempty cell's candidates
+	uint32_t start[kWalkWindow / 32];    // bit q: a cell's candidates start at index q of the window
+};
+
+typedef float walk_f4 __attribute__((ext_vector_type(4)));
+
+// The distance part of the reference's predicate for home particle pi (slot ti) and this
+// lane's candidate j: the difference of the higher slot's position less the lower's is
+// q - pi or its exact negation (rounding is sign-symmetric).
+__device__ __forceinline__ bool pair_within(const HomeParams& P, const walk_f4& pi, uint32_t ti, uint32_t j,
+											const float4& q) {
+	const float dx = q.x - pi.x, dy = q.y - pi.y, dz = q.z - pi.z;
+	return len2(wrap_diff(P.box, j > ti ? make_float3(dx, dy, dz) : make_float3(-dx, -dy, -dz))) <= P.rc2;
 }
 
-__device__ __forceinline__ uint64_t exact_hit_masks(const HomeParams& P, const float4* home_pos, uint32_t nh,
-													 uint32_t c0s, bool live, uint32_t j, const float4& q) {
-	int mine_lo = 0, mine_hi = 0;
-	float4 pn = home_pos[0];
-	for (uint32_t i = 0; i < nh; ++i) {
-		const float4 pi = pn;
-		pn = home_pos[(i + 1u) & 63u];
-		const uint32_t ti = c0s + i;
-		bool in = live && j != ti && pair_predicate_home(P.box, P.rc2, P.ex, pi, ti, q, j);
-		if (in && P.ref_filter)
-			in = in_reference_stencil(P, pi, q); // symmetric in its two ends
-		set_lane_mask(mine_lo, mine_hi, __ballot(in), i);
-	}
-	return lane_mask(mine_lo, mine_hi);
+// The pairs of home particle i with the candidates of one block that pass everything but
+// the distance: exclusions and rigid bodies by the lower end's row, the reference's stencil.
+__device__ __forceinline__ bool pair_allowed(const HomeParams& P, uint32_t ti, uint32_t j) {
+	const float4 pi = P.spos[ti], q = P.spos[j];
+	if ((P.ex.rigid_body_id || P.ex.offsets) && !pair_unexcluded(P.ex, j > ti ? pi : q, j > ti ? q : pi))
+		return false;
+	return !P.ref_filter || in_reference_stencil(P, pi, q); // symmetric in its two ends
 }
 
-// The same masks from the home-frame prefilter (the candidate moved into the home frame
-// as qx, qy, qz; +inf on lanes without a candidate): a pair with d2' <= pre_lo2 is in,
-// one with d2' > pre_hi2 out. A home particle's own slot among the candidates is not
-// excluded here (the caller skips it). When any pair of the block falls between the two
-// bounds the block is decided again by exact_hit_masks.
-__device__ __forceinline__ uint64_t home_frame_hit_masks(const HomeParams& P, const float4* home_pos, uint32_t nh,
-														 uint32_t c0s, bool live, uint32_t j, const float4& q,
-														 float qx, float qy, float qz) {
-	int mine_lo = 0, mine_hi = 0;
-	uint64_t band = 0;
-	float4 pn = home_pos[0];
-	for (uint32_t i = 0; i < nh; ++i) {
-		const float4 pi = pn;
-		pn = home_pos[(i + 1u) & 63u];
-		const float dx = qx - pi.x, dy = qy - pi.y, dz = qz - pi.z;
-		const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-		const uint64_t hits = __ballot(d2 <= P.pre_lo2);
-		band |= __ballot(d2 <= P.pre_hi2) & ~hits;
-		set_lane_mask(mine_lo, mine_hi, hits, i);
+// The exclusion row of this lane's home particle as slots, the first four in registers.
+struct HomeExcl {
+	uint32_t begin, count, slot[4];
+};
+__device__ __forceinline__ HomeExcl home_exclusions(const HomeParams& P, bool valid, const float4& p) {
+	HomeExcl x{0u, 0u, {0u, 0u, 0u, 0u}};
+	const uint32_t c = meta_canon(__float_as_uint(p.w));
+	if (valid && c < P.ex.num_particles) {
+		x.begin = uint32_t(P.ex.offsets[c]);
+		x.count = uint32_t(P.ex.offsets[c + 1]) - x.begin;
 	}
-	uint64_t mine = lane_mask(mine_lo, mine_hi);
-	if (band)
-		mine = exact_hit_masks(P, home_pos, nh, c0s, live, j, q);
-	return mine;
-}
-
-// One block of candidates against the wave's home particles: the hit masks (lane i:
-// home particle i's hits over the block's lanes), then every home lane appends its hits
-// to its row in lane (candidate) order, reading their slots from `cand` (LDS).
-template<bool FAST, bool FILL>
-__device__ __forceinline__ void test_candidate_block(const HomeParams& P, const float4* home_pos, uint32_t* cand,
-													 uint32_t nh, uint32_t c0, bool live, uint32_t j, const float4& q,
-													 float qx, float qy, float qz, uint32_t& cnt,
-													 uint32_t* __restrict__ nbr) {
-	const uint32_t lane = threadIdx.x & 63u;
-	const uint32_t c0s = uint32_t(__builtin_amdgcn_readfirstlane(int(c0))); // wave-uniform
-	cand[lane] = j;
-	wave_lds_sync();
-	const uint64_t mine = FAST ? home_frame_hit_masks(P, home_pos, nh, c0s, live, j, q, qx, qy, qz)
-							   : exact_hit_masks(P, home_pos, nh, c0s, live, j, q);
-	if (lane < nh) {
-		const uint32_t t = c0s + lane;
-		uint32_t* __restrict__ row = nbr + (uint64_t(t) >> 6) * 64u * P.cap + (t & 63u) * 4u;
-		uint64_t m = mine;
-		while (m) {
-			const uint32_t b = uint32_t(__builtin_ctzll(m));
-			m &= m - 1;
-			const uint32_t jb = cand[b];
-			if (FAST && jb == t) // never a pair with itself
-				continue;
-			if (FILL && cnt < P.cap) // entry cnt of slot t (nbr_slot_index)
-				row[(cnt >> 2) * 256u + (cnt & 3u)] = jb;
-			++cnt;
-		}
-	}
-	wave_lds_sync();
-}
-
-// The home-frame coordinates of a candidate at q (see candidate_at).
-__device__ __forceinline__ void home_frame(const HomeParams& P, bool live, bool frame, const float4& p0,
-										   const float4& q, float& qx, float& qy, float& qz) {
-	if (!frame) {
-		qx = q.x;
-		qy = q.y;
-		qz = q.z;
-		return;
-	}
-	qx = qy = qz = INFINITY;
-	if (live) {
-		qx = P.box.periodic[0] ? q.x - P.box.L[0] * rintf((q.x - p0.x) * P.box.inv_L[0]) : q.x;
-		qy = P.box.periodic[1] ? q.y - P.box.L[1] * rintf((q.y - p0.y) * P.box.inv_L[1]) : q.y;
-		qz = P.box.periodic[2] ? q.z - P.box.L[2] * rintf((q.z - p0.z) * P.box.inv_L[2]) : q.z;
-	}
-}
-
-// Candidate qi of segments [0, nseg) (ntot particles): its slot j and position q, and q
-// in the home frame (moved by whole box lengths next to the anchor p0, so the image is
-// exact; +inf on lanes without a candidate) when `frame`.
-__device__ __forceinline__ void candidate_at(const HomeParams& P, const uint32_t* seg_b, const uint32_t* seg_pre,
-											 uint32_t nseg, uint32_t qi, bool live, bool frame, const float4& p0,
-											 uint32_t& j, float4& q, float& qx, float& qy, float& qz) {
-	j = 0xFFFFFFFFu;
-	q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-	if (live) {
-		uint32_t lo = 0, hi = nseg; // seg_pre[lo] <= qi < seg_pre[hi]
-		while (hi - lo > 1) {
-			const uint32_t mid = (lo + hi) >> 1;
-			if (seg_pre[mid] <= qi)
-				lo = mid;
-			else
-				hi = mid;
-		}
-		j = seg_b[lo] + (qi - seg_pre[lo]);
-		q = P.spos[j];
-	}
-	home_frame(P, live, frame, p0, q, qx, qy, qz);
-}
-
-__device__ __forceinline__ float wave_min(float v) {
-	for (int o = 32; o > 0; o >>= 1)
-		v = fminf(v, __shfl_xor(v, o));
-	return v;
-}
-__device__ __forceinline__ float wave_max(float v) {
-	for (int o = 32; o > 0; o >>= 1)
-		v = fmaxf(v, __shfl_xor(v, o));
-	return v;
-}
-
-// Tests the candidates of segments [0, nseg) (ntot particles) against the wave's home
-// particles (lane l holds home particle t = c0 + l when valid, with its count) and
-// records the hits. The candidates are spread over the lanes, 64 at a time, and the
-// home particles are visited one by one from LDS: each (home particle, candidate) pair
-// is evaluated by exactly one lane, so a wave whose home cell holds fewer than 64
-// particles does not idle lanes on every test. Every row lists its neighbours in
-// candidate order.
-// With the home-frame prefilter, a candidate whose squared distance to the bounding box
-// of the home particles exceeds pre_hi2 is dropped first (the fine cells of the stencil
-// reach past that box: at 1M beads most candidates are dropped): that distance is at
-// most d2' to every home particle, computed with the same monotone operations, so each
-// dropped candidate is one the prefilter would decide "out" for every home particle.
-// The kept ones (in candidate order, through a 128-entry LDS queue `keep`) are tested
-// 64 at a time, so the pair set and each row's order are unchanged.
-template<bool FILL>
-__device__ __forceinline__ void home_test_segments(const HomeParams& P, const uint32_t* seg_b, uint32_t* seg_pre,
-												   uint32_t nseg, uint32_t ntot, bool valid, uint32_t t,
-												   const float4& p, uint32_t& cnt, uint32_t* __restrict__ nbr,
-												   float4* home_pos, uint32_t* keep) {
-	const uint32_t lane = threadIdx.x & 63u;
-	if (lane == 0)
-		seg_pre[nseg] = ntot;
-	home_pos[lane] = p;
-	wave_lds_sync();
-	uint32_t* cand = reinterpret_cast<uint32_t*>(home_pos + 64); // the block's candidate slots
-	const uint32_t c0 = t - lane;                       // first home slot of this chunk
-	const uint32_t nh = uint32_t(__popcll(__ballot(valid))); // valid lanes are a prefix
-	const float4 p0 = home_pos[0];                       // the home frame's anchor
-	const bool fast = P.pre && !P.ref_filter && !P.ex.rigid_body_id && !P.ex.offsets;
-	if (!fast) {
-		for (uint32_t q0 = 0; q0 < ntot; q0 += 64) {
-			const bool live = q0 + lane < ntot;
-			uint32_t j;
-			float4 q;
-			float qx, qy, qz;
-			candidate_at(P, seg_b, seg_pre, nseg, q0 + lane, live, false, p0, j, q, qx, qy, qz);
-			test_candidate_block<false, FILL>(P, home_pos, cand, nh, c0, live, j, q, qx, qy, qz, cnt, nbr);
-		}
-		wave_lds_sync();
-		return;
-	}
-	const float lox = wave_min(valid ? p.x : INFINITY), hix = wave_max(valid ? p.x : -INFINITY);
-	const float loy = wave_min(valid ? p.y : INFINITY), hiy = wave_max(valid ? p.y : -INFINITY);
-	const float loz = wave_min(valid ? p.z : INFINITY), hiz = wave_max(valid ? p.z : -INFINITY);
-	const uint64_t lt = (uint64_t(1) << lane) - 1;
-	uint32_t nk = 0; // queued candidates (wave-uniform), fewer than 64 between blocks
-	for (uint32_t q0 = 0; q0 < ntot; q0 += 64) {
-		const bool live = q0 + lane < ntot;
-		uint32_t j;
-		float4 q;
-		float qx, qy, qz;
-		candidate_at(P, seg_b, seg_pre, nseg, q0 + lane, live, true, p0, j, q, qx, qy, qz);
-		const float ax = fmaxf(fmaxf(lox - qx, qx - hix), 0.0f);
-		const float ay = fmaxf(fmaxf(loy - qy, qy - hiy), 0.0f);
-		const float az = fmaxf(fmaxf(loz - qz, qz - hiz), 0.0f);
-		const bool kept = live && !(fmaf(ax, ax, fmaf(ay, ay, az * az)) > P.pre_hi2);
-		const uint64_t km = __ballot(kept);
-		if (kept)
-			keep[nk + uint32_t(__popcll(km & lt))] = j;
-		nk += uint32_t(__popcll(km));
-		if (nk >= 64) {
-			wave_lds_sync();
-			{
-				const uint32_t jb = keep[lane];
-				const float4 qb = P.spos[jb];
-				float bx, by, bz;
-				home_frame(P, true, true, p0, qb, bx, by, bz);
-				test_candidate_block<true, FILL>(P, home_pos, cand, nh, c0, true, jb, qb, bx, by, bz, cnt, nbr);
-			}
-			const uint32_t rest = nk - 64;
-			const uint32_t v = lane < rest ? keep[64 + lane] : 0u;
-			wave_lds_sync();
-			if (lane < rest)
-				keep[lane] = v;
-			nk = rest;
-			wave_lds_sync();
-		}
-	}
-	if (nk > 0) {
-		wave_lds_sync();
-		const bool live = lane < nk;
-		const uint32_t jb = live ? keep[lane] : 0xFFFFFFFFu;
-		const float4 qb = live ? P.spos[jb] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-		float bx, by, bz;
-		home_frame(P, live, true, p0, qb, bx, by, bz);
-		test_candidate_block<true, FILL>(P, home_pos, cand, nh, c0, live, jb, qb, bx, by, bz, cnt, nbr);
-	}
-	wave_lds_sync();
-}
-
-template<bool FILL>
-__device__ void walk_home_cell(const HomeParams& P, uint32_t home, uint32_t* seg_b, uint32_t* seg_pre, float4* home_pos,
-							   uint32_t* keep, uint32_t* __restrict__ counts, uint32_t* __restrict__ nbr) {
-	const int lane = threadIdx.x & 63;
-	const uint32_t hb = P.home_begin[home], he = P.home_end[home];
-	if (hb >= he)
-		return;
-	const int hc[3] = {int(compact_by3(home >> 2)), int(compact_by3(home >> 1)), int(compact_by3(home))};
-	const int fine_cells = 1 << (P.h + P.s);
-	const int span = 1 << P.s;
-	int lo[3], nax[3];
+	uint32_t e[4];
 #pragma unroll
-	for (int a = 0; a < 3; ++a) {
-		if (P.full[a]) {
-			lo[a] = 0;
-			nax[a] = fine_cells;
+	for (uint32_t k = 0; k < 4; ++k)
+		e[k] = k < x.count ? uint32_t(P.ex.excluded[x.begin + k]) : 0u;
+#pragma unroll
+	for (uint32_t k = 0; k < 4; ++k)
+		x.slot[k] = k < x.count ? P.ex_slot[e[k]] : 0u;
+	return x;
+}
+
+// The walk's instances. Fast ones: a box periodic on every axis, the prefilter, the
+// stencil as codes, no rigid bodies and no reference stencil, without exclusions or with
+// symmetric rows (ex_slot); the parameters of the rest would otherwise hold, and spill,
+// scalar registers throughout.
+constexpr int kWalkPlain = 0, kWalkOwnRows = 1, kWalkGeneral = 2;
+__host__ __device__ inline int walk_mode(const HomeParams& P) {
+	if (!P.pre || !P.stencil_code || P.ref_filter || P.ex.rigid_body_id || (P.ex.offsets && !P.ex_slot))
+		return kWalkGeneral;
+	return P.ex.offsets ? kWalkOwnRows : kWalkPlain;
+}
+
+// One block of up to 64 candidates (slot j, position q: in the home frame with the
+// prefilter; dead lanes have j = ~0 and, with the prefilter, q = +inf) against the wave's
+// nh home particles, the first at slot c0: each one's hits go to the end of its row
+// (cnt: this lane's home particle's entries so far).
+template<int MODE>
+__device__ __forceinline__ void test_block(const HomeParams& P, uint32_t c0, uint32_t nh, uint32_t j, float qx,
+										   float qy, float qz, const HomeExcl& X, bool own_rows, bool filter,
+										   uint32_t& cnt, uint32_t* __restrict__ nbr) {
+	const walk_f4 MMD_CONST_AS* home = (const walk_f4 MMD_CONST_AS*)(uint64_t(P.spos) + 16ull * c0);
+	const uint32_t self = j - c0; // this candidate's index among the home particles
+	// rows: slot t's entries lie 16 t bytes into its tile of 64 slots, the home particles in
+	// at most two tiles (byte offsets from the first one's fit 32 bits: a tile's rows do)
+	char* const rows = reinterpret_cast<char*>(nbr + uint64_t(c0 >> 6) * 64u * P.cap);
+	const uint64_t alive = __ballot(j != ~0u);
+	walk_f4 hp[4], hn[4];
+#pragma unroll
+	for (uint32_t u = 0; u < 4; ++u)
+		hn[u] = home[min(u, nh - 1u)];
+	for (uint32_t i0 = 0; i0 < nh; i0 += 4) {
+#pragma unroll
+		for (uint32_t u = 0; u < 4; ++u) {
+			hp[u] = hn[u];
+			hn[u] = home[min(i0 + 4u + u, nh - 1u)]; // the next four, in flight
+		}
+#pragma unroll
+		for (uint32_t u = 0; u < 4; ++u) {
+			const uint32_t i = i0 + u, ti = c0 + i;
+			// keeps the unused fourth word of each load alive: its register would otherwise be
+			// taken at once, with a wait for the load in flight
+			asm volatile("" ::"s"(hp[u].w));
+			if (i < nh) {
+				const uint64_t other = __ballot(self != i);
+				uint64_t hits;
+				if (MODE != kWalkGeneral || P.pre) {
+					const float dx = qx - hp[u].x, dy = qy - hp[u].y, dz = qz - hp[u].z;
+					const float d2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+					hits = __ballot(d2 <= P.pre_lo2) & other;
+					// between the two bounds the reference's predicate decides
+					if ((__ballot(d2 <= P.pre_hi2) & other) != hits)
+						hits = __ballot(j != ~0u && pair_within(P, hp[u], ti, j, P.spos[j])) & other;
+				} else {
+					hits = __ballot(pair_within(P, hp[u], ti, j, make_float4(qx, qy, qz, 0.0f))) & other & alive;
+				}
+				if (own_rows) {
+					const uint32_t nx = bcast_u32(X.count, i);
+#pragma unroll
+					for (uint32_t k = 0; k < 4; ++k)
+						if (k < nx)
+							hits &= ~__ballot(j == bcast_u32(X.slot[k], i));
+					for (uint32_t k = 4; k < nx; ++k)
+						hits &= ~__ballot(j == P.ex_slot[P.ex.excluded[bcast_u32(X.begin, i) + k]]);
+				}
+				if (filter)
+					hits = __ballot(__builtin_amdgcn_inverse_ballot_w64(hits) && pair_allowed(P, ti, j));
+				const uint32_t base = bcast_u32(cnt, i);
+				// this home particle's rows: entry e of slot t (nbr_slot_index)
+				const uint32_t at = ((ti >> 6) - (c0 >> 6)) * 256u * P.cap + (ti & 63u) * 16u;
+				if (__builtin_amdgcn_inverse_ballot_w64(hits)) {
+					const uint32_t e = uint32_t(__builtin_amdgcn_mbcnt_hi(
+						uint32_t(hits >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(hits), base)));
+					const uint32_t off = ((e << 8) & ~1023u) | ((e & 3u) << 2);
+					if (e < P.cap)
+						*reinterpret_cast<uint32_t*>(rows + (off + at)) = j;
+				}
+				set_lane(cnt, base + uint32_t(__popcll(hits)), i);
+			}
+		}
+	}
+}
+
+// Fine cell k of the enumeration around home cell `home` (its particle range; empty when
+// there is none or the gap test drops it).
+template<int MODE>
+struct WalkCells {
+	const HomeParams& P;
+	uint32_t home, total;
+	uint32_t base[3], mask[3]; // home code with every bit outside the axis set, axis bits
+	int hc[3], lo[3], nax[3];
+	__device__ __forceinline__ WalkCells(const HomeParams& P_, uint32_t home_) : P(P_), home(home_) {
+		const uint32_t all = uint32_t((uint64_t(1) << (3 * (P.h + P.s))) - 1u);
+		const uint32_t code = home << (3 * P.s);
+#pragma unroll
+		for (int a = 0; a < 3; ++a) {
+			mask[a] = (0x24924924u >> a) & all;
+			base[a] = (P.full[a] ? 0u : code & mask[a]) | ~mask[a];
+		}
+		total = P.stencil_n;
+		if (MODE == kWalkGeneral && !P.stencil_code) {
+			const int fine_cells = 1 << (P.h + P.s), span = 1 << P.s;
+			hc[0] = int(compact_by3(home >> 2));
+			hc[1] = int(compact_by3(home >> 1));
+			hc[2] = int(compact_by3(home));
+#pragma unroll
+			for (int a = 0; a < 3; ++a) {
+				lo[a] = P.full[a] ? 0 : hc[a] * span - P.reach[a];
+				int hgh = P.full[a] ? fine_cells - 1 : hc[a] * span + span - 1 + P.reach[a];
+				if (!P.full[a] && !P.box.periodic[a]) { // open axis: only cells that exist (the reach
+					lo[a] = max(lo[a], 0);               // can be huge when the extent is degenerate)
+					hgh = min(hgh, fine_cells - 1);
+				}
+				nax[a] = hgh - lo[a] + 1;
+			}
+			if (!P.stencil)
+				total = uint32_t(nax[0] * nax[1] * nax[2]);
+		}
+	}
+	__device__ __forceinline__ uint32_t offset(uint32_t k) const { // the stencil word, loaded ahead
+		return (MODE != kWalkGeneral || P.stencil_code) && k < total ? P.stencil_code[k] : 0u;
+	}
+	__device__ __forceinline__ uint2 range(uint32_t k, uint32_t off) const {
+		uint2 none = make_uint2(0u, 0u);
+		if (k >= total)
+			return none;
+		uint32_t code = 0;
+		if (MODE != kWalkGeneral || P.stencil_code) {
+#pragma unroll
+			for (int a = 0; a < 3; ++a)
+				code |= (base[a] + (off & mask[a])) & mask[a];
+			return P.fine[code];
+		}
+		const int fine_cells = 1 << (P.h + P.s), span = 1 << P.s;
+		int iv[3];
+		if (P.stencil) {
+			const int4 o = P.stencil[k];
+			iv[0] = o.x;
+			iv[1] = o.y;
+			iv[2] = o.z;
+#pragma unroll
+			for (int a = 0; a < 3; ++a)
+				iv[a] += P.full[a] ? 0 : hc[a] * span;
 		} else {
-			int l = hc[a] * span - P.reach[a];
-			int hgh = hc[a] * span + span - 1 + P.reach[a];
-			if (!P.box.periodic[a]) { // open axis: only cells that exist (the reach can be huge
-				l = max(l, 0);        // when the extent is degenerate)
-				hgh = min(hgh, fine_cells - 1);
-			}
-			lo[a] = l;
-			nax[a] = hgh - l + 1;
+			iv[0] = lo[0] + int(k) % nax[0];
+			iv[1] = lo[1] + (int(k) / nax[0]) % nax[1];
+			iv[2] = lo[2] + int(k) / (nax[0] * nax[1]);
 		}
+		float gap2 = 0.0f;
+#pragma unroll
+		for (int a = 0; a < 3; ++a) {
+			int u = iv[a];
+			if (!P.full[a]) {
+				const int h0 = hc[a] * span;
+				const int apart = u < h0 ? h0 - u - 1 : (u >= h0 + span ? u - h0 - span : 0);
+				const float g = fmaxf(0.0f, float(apart) * P.cw[a] - 2.0f * P.margin[a]);
+				gap2 += g * g;
+				if (P.box.periodic[a])
+					u = (u + fine_cells) & (fine_cells - 1);
+				else if (u < 0 || u >= fine_cells)
+					return none;
+			}
+			code |= split_by3(uint32_t(u) & 1023u) << (2 - a);
+		}
+		return gap2 <= P.rc2 ? P.fine[code] : none;
 	}
-	const int total = P.stencil ? int(P.stencil_n) : nax[0] * nax[1] * nax[2];
-	const uint64_t lt_mask = (uint64_t(1) << lane) - 1;
-	// The segments do not depend on the chunk of home particles: when the first chunk's
-	// enumeration fits LDS whole, the later chunks test the same segments.
-	uint32_t nseg = 0, ntot = 0; // wave-uniform
-	bool cached = false;
-	for (uint32_t c0 = hb; c0 < he; c0 += 64) {
-		const uint32_t t = c0 + uint32_t(lane);
-		const bool valid = t < he;
-		const float4 p = valid ? P.spos[t] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+};
+
+// A candidate at q moved by whole box lengths next to the home frame's anchor (so the
+// image is exact).
+template<int MODE>
+__device__ __forceinline__ float frame_axis(const HomeParams& P, int a, float q, float p0) {
+	return MODE != kWalkGeneral || P.box.periodic[a] ? q - P.box.L[a] * rintf((q - p0) * P.box.inv_L[a]) : q;
+}
+
+// Particles [from, to) of home cell `home`, 64 at a time.
+template<int MODE>
+__device__ __forceinline__ void walk_home_cell(const HomeParams& P, uint32_t home, uint32_t from, uint32_t to,
+											   WalkLds& S, uint32_t* __restrict__ counts, uint32_t* __restrict__ nbr) {
+	const uint32_t lane = threadIdx.x & 63u;
+	const WalkCells<MODE> cells(P, home);
+	const bool own_rows = MODE == kWalkOwnRows || (MODE == kWalkGeneral && P.ex_slot);
+	const bool filter = MODE == kWalkGeneral && (P.ref_filter || P.ex.rigid_body_id || (P.ex.offsets && !own_rows));
+	for (uint32_t c0 = from; c0 < to; c0 += 64) {
+		const uint32_t nh = min(to - c0, 64u);
+		const bool valid = lane < nh;
+		const float4 p = P.spos[c0 + min(lane, nh - 1u)];
+		HomeExcl X{};
+		if (own_rows)
+			X = home_exclusions(P, valid, p);
+		const float ox = bcast_f32(p.x, 0), oy = bcast_f32(p.y, 0), oz = bcast_f32(p.z, 0); // the frame's anchor
+		// (lanes past the end repeat the last home particle)
+		const float lox = wave_min(p.x), hix = wave_max(p.x);
+		const float loy = wave_min(p.y), hiy = wave_max(p.y);
+		const float loz = wave_min(p.z), hiz = wave_max(p.z);
 		uint32_t cnt = 0;
-		if (!cached) {
-			nseg = 0;
-			ntot = 0;
-		}
-		bool flushed = false;
-		for (int cb = cached ? total : 0; cb < total; cb += 64) {
-			const int k = cb + lane;
-			uint32_t b = 0, e = 0;
-			if (P.stencil && k < total) {
-				const int4 o = P.stencil[k];
-				const int off[3] = {o.x, o.y, o.z};
-				bool keep = true;
-				uint32_t code = 0;
-#pragma unroll
-				for (int a = 0; a < 3; ++a) {
-					int u = P.full[a] ? off[a] : hc[a] * span + off[a];
-					if (P.box.periodic[a])
-						u = (u + fine_cells) & (fine_cells - 1);
-					else if (u < 0 || u >= fine_cells)
-						keep = false;
-					code |= split_by3(uint32_t(u) & 1023u) << (2 - a);
-				}
-				if (keep) {
-					b = P.fine_begin[code];
-					e = P.fine_end[code];
-				}
-			} else if (k < total) {
-				const int iv[3] = {k % nax[0], (k / nax[0]) % nax[1], k / (nax[0] * nax[1])};
-				float gap2 = 0.0f;
-				bool keep = true;
-				uint32_t code = 0;
-#pragma unroll
-				for (int a = 0; a < 3; ++a) {
-					int u = lo[a] + iv[a];
-					if (!P.full[a]) {
-						const int h0 = hc[a] * span;
-						const int apart = u < h0 ? h0 - u - 1 : (u >= h0 + span ? u - h0 - span : 0);
-						const float g = fmaxf(0.0f, float(apart) * P.cw[a] - 2.0f * P.margin[a]);
-						gap2 += g * g;
-						if (P.box.periodic[a])
-							u = (u + fine_cells) & (fine_cells - 1);
-						else if (u < 0 || u >= fine_cells)
-							keep = false;
+		uint32_t nk = 0; // queued candidates (wave-uniform), fewer than 64 between blocks
+		const auto block = [&](bool live, const float4& c) {
+			test_block<MODE>(P, c0, nh, live ? __float_as_uint(c.w) : ~0u, live ? c.x : INFINITY, c.y, c.z, X, own_rows,
+					   filter, cnt, nbr);
+		};
+		// the next step's cells and the stencil words of the one after are in flight while a
+		// step's candidates are tested
+		uint32_t off = cells.offset(lane);
+		uint2 rg = cells.range(lane, off);
+		off = cells.offset(64u + lane);
+		for (uint32_t k0 = 0; k0 < cells.total; k0 += 64) {
+			const uint32_t b = rg.x, n = rg.y > rg.x ? rg.y - rg.x : 0u;
+			if (k0 + 64 < cells.total) {
+				rg = cells.range(k0 + 64 + lane, off);
+				off = cells.offset(k0 + 128 + lane);
+			}
+			const uint64_t some = __ballot(n > 0);
+			if (some == 0)
+				continue;
+			// candidate q of this step (q < total, cells in lane order) is slot q + delta of its
+			// cell; a cell's rank is the number of cells starting at or before q
+			const uint32_t incl = wave_inclusive_scan(n), excl = incl - n;
+			const uint32_t total = bcast_u32(incl, 63);
+			wave_lds_sync(); // (reads of the last step's words)
+			if (n > 0)
+				S.delta[bits_below(some)] = b - excl;
+			for (uint32_t w0 = 0; w0 < total; w0 += kWalkWindow) {
+				if (w0 > 0)
+					wave_lds_sync();
+				if (lane < kWalkWindow / 32)
+					S.start[lane] = 0u;
+				wave_lds_sync();
+				if (n > 0 && excl - w0 < kWalkWindow)
+					atomicOr(&S.start[(excl - w0) >> 5], 1u << (excl & 31u));
+				uint32_t before = uint32_t(__popcll(__ballot(n > 0 && excl < w0)));
+				wave_lds_sync();
+				const uint32_t end = min(total, w0 + kWalkWindow);
+				const auto load = [&](uint32_t q0, uint32_t& j, float4& q) {
+					const uint32_t at = (q0 - w0) >> 5;
+					const uint32_t lo = uint32_t(__builtin_amdgcn_readfirstlane(int(S.start[at])));
+					const uint32_t hi = uint32_t(__builtin_amdgcn_readfirstlane(int(S.start[at + 1])));
+					const uint64_t bits = uint64_t(lo) | (uint64_t(hi) << 32);
+					const uint32_t rank = before + bits_below(bits) + uint32_t((bits >> lane) & 1u) - 1u;
+					before += uint32_t(__popcll(bits));
+					// past the end: the last cell's last candidate, dropped by `live`
+					j = min(q0 + lane, total - 1u) + S.delta[rank];
+					q = P.spos[j];
+				};
+				uint32_t j;
+				float4 q;
+				load(w0, j, q);
+				for (uint32_t q0 = w0; q0 < end; q0 += 64) {
+					uint32_t jn = j;
+					float4 qn = q;
+					if (q0 + 64 < end)
+						load(q0 + 64, jn, qn);
+					bool kept = q0 + lane < total;
+					if (MODE != kWalkGeneral || P.pre) {
+						q.x = frame_axis<MODE>(P, 0, q.x, ox);
+						q.y = frame_axis<MODE>(P, 1, q.y, oy);
+						q.z = frame_axis<MODE>(P, 2, q.z, oz);
+						// farther than the cutoff from the home particles' bounding box: its d2' to
+						// every home particle is at least this, by the same monotone operations, so
+						// the prefilter would drop it for each of them
+						const float ax = fmaxf(fmaxf(lox - q.x, q.x - hix), 0.0f);
+						const float ay = fmaxf(fmaxf(loy - q.y, q.y - hiy), 0.0f);
+						const float az = fmaxf(fmaxf(loz - q.z, q.z - hiz), 0.0f);
+						kept = kept && !(fmaf(ax, ax, fmaf(ay, ay, az * az)) > P.pre_hi2);
 					}
-					code |= split_by3(uint32_t(u) & 1023u) << (2 - a);
+					const uint64_t km = __ballot(kept);
+					if (kept)
+						S.keep[nk + bits_below(km)] = make_float4(q.x, q.y, q.z, __uint_as_float(j));
+					nk += uint32_t(__popcll(km));
+					wave_lds_sync();
+					if (nk >= 64) {
+						const float4 c = S.keep[lane], rest = S.keep[64 + lane];
+						wave_lds_sync();
+						nk -= 64;
+						if (lane < nk)
+							S.keep[lane] = rest;
+						wave_lds_sync();
+						block(true, c);
+					}
+					j = jn;
+					q = qn;
 				}
-				if (keep && gap2 <= P.rc2) {
-					b = P.fine_begin[code];
-					e = P.fine_end[code];
-				}
 			}
-			const uint32_t c = e > b ? e - b : 0u;
-			const uint64_t mask = __ballot(c > 0);
-			const uint32_t nnew = uint32_t(__popcll(mask));
-			if (nseg + nnew > uint32_t(kSegMax)) {
-				home_test_segments<FILL>(P, seg_b, seg_pre, nseg, ntot, valid, t, p, cnt, nbr, home_pos, keep);
-				nseg = 0;
-				ntot = 0;
-				flushed = true;
-			}
-			const uint32_t incl = wave_inclusive_scan(c);
-			const uint32_t sum = bcast_u32(incl, 63);
-			if (c > 0) {
-				const uint32_t r = nseg + uint32_t(__popcll(mask & lt_mask));
-				seg_b[r] = b;
-				seg_pre[r] = ntot + incl - c;
-			}
-			nseg += nnew;
-			ntot += sum;
 		}
-		home_test_segments<FILL>(P, seg_b, seg_pre, nseg, ntot, valid, t, p, cnt, nbr, home_pos, keep);
-		cached = !flushed;
+		if (nk > 0) {
+			const float4 c = S.keep[lane];
+			wave_lds_sync();
+			block(lane < nk, c);
+		}
 		if (valid) {
+			const uint32_t t = c0 + lane;
 			counts[t] = cnt;
-			if (FILL && cnt <= P.cap) {
+			if (cnt <= P.cap) {
 				const uint64_t row = (uint64_t(t) >> 6) * 64u * P.cap;
 				for (uint32_t k = cnt; (k & 3u) != 0; ++k)
 					nbr[nbr_slot_index(row, t, k)] = t;
@@ -580,22 +634,37 @@ __device__ void walk_home_cell(const HomeParams& P, uint32_t home, uint32_t* seg
 	}
 }
 
-// Bounded to 80 VGPRs (6 waves per SIMD, a few dwords of spill): the home-particle loop
-// waits on an LDS read per home particle, which more waves hide (re-walk at 1M beads
-// 0.48 -> 0.46 ms against 90 VGPRs and 5 waves).
-template<bool FILL>
+template<int MODE>
 __global__ __launch_bounds__(256, 6) void k_walk_home(HomeParams P, uint32_t* __restrict__ counts,
-												   uint32_t* __restrict__ nbr) {
-	__shared__ uint32_t seg_b[kHomeWaves][kSegMax];
-	__shared__ uint32_t seg_pre[kHomeWaves][kSegMax + 1];
-	__shared__ float4 home_pos[kHomeWaves][kHomeLds];
-	__shared__ uint32_t keep[kHomeWaves][kHomeKeep];
-	const int wv = threadIdx.x >> 6;
+													  uint32_t* __restrict__ nbr) {
+	__shared__ WalkLds lds[kHomeWaves];
+	static_assert(kHomeWaves == 4, "a group's four cells");
+	const uint32_t wv = uint32_t(__builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)));
 	const TileRange R = xcd_tiles((P.num_home + kHomeWaves - 1) / kHomeWaves);
 	for (uint32_t g = R.tile; g < R.end; g += R.stride) {
-		const uint32_t home = g * kHomeWaves + uint32_t(wv);
-		if (home < P.num_home)
-			walk_home_cell<FILL>(P, home, seg_b[wv], seg_pre[wv], home_pos[wv], keep[wv], counts, nbr);
+		if constexpr (MODE == kWalkPlain) {
+			const uint32_t home = g * kHomeWaves + wv;
+			if (home < P.num_home) {
+				const uint2 r = *(const uint2 MMD_CONST_AS*)(uint64_t(P.home) + 8ull * home);
+				if (r.x < r.y)
+					walk_home_cell<MODE>(P, home, r.x, r.y, lds[wv], counts, nbr);
+			}
+		} else {
+			// systems with exclusions are crowded along their chains: the 64-particle chunks of
+			// the group's cells are dealt to its waves in turn (polymers of 100k beads: 209 ->
+			// 158 us; the plain walk's extra scalar registers cost it 6% at 1M beads)
+			uint32_t chunk = 0; // chunks of the cells so far
+			for (uint32_t k = 0; k < uint32_t(kHomeWaves); ++k) {
+				const uint32_t home = g * kHomeWaves + k;
+				if (home >= P.num_home)
+					break;
+				const uint2 r = *(const uint2 MMD_CONST_AS*)(uint64_t(P.home) + 8ull * home);
+				const uint32_t chunks = r.y > r.x ? (r.y - r.x + 63u) / 64u : 0u;
+				for (uint32_t c = (wv - chunk) & 3u; c < chunks; c += 4u)
+					walk_home_cell<MODE>(P, home, r.x + 64u * c, min(r.y, r.x + 64u * c + 64u), lds[wv], counts, nbr);
+				chunk += chunks;
+			}
+		}
 	}
 }
 

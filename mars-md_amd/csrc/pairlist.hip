@@ -177,6 +177,24 @@ __global__ void k_cell_ranges(const uint32_t* __restrict__ codes, uint64_t n, in
 		end[c] = uint32_t(i + 1);
 }
 
+// The same ranges of the walk's fine and home cells at once, as {begin, end}.
+__global__ void k_walk_cells(const uint32_t* __restrict__ codes, uint64_t n, int fine_shift, int home_shift,
+							 uint2* __restrict__ fine, uint2* __restrict__ home) {
+	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (i >= n)
+		return;
+	const uint32_t c = codes[i];
+	const uint32_t cp = i > 0 ? codes[i - 1] : ~c, cn = i + 1 < n ? codes[i + 1] : ~c;
+	if (i == 0 || (cp >> fine_shift) != (c >> fine_shift))
+		fine[c >> fine_shift].x = uint32_t(i);
+	if (i + 1 == n || (cn >> fine_shift) != (c >> fine_shift))
+		fine[c >> fine_shift].y = uint32_t(i + 1);
+	if (i == 0 || (cp >> home_shift) != (c >> home_shift))
+		home[c >> home_shift].x = uint32_t(i);
+	if (i + 1 == n || (cn >> home_shift) != (c >> home_shift))
+		home[c >> home_shift].y = uint32_t(i + 1);
+}
+
 // BuildCellNeighborsKernel (ZOrderNeighbor.h:55-139), for the reference tables.
 __global__ void k_cell_neighbors(uint32_t* __restrict__ out, uint64_t num_cells, int m, int3 r,
 								 int slots, int3 per) {
@@ -704,13 +722,8 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 	const int m = build_grid.m;
 	if (m < 1)
 		return false;
-	// home level: at least home_target particles per home cell on average (by default
-	// about 24..190), below the build grid; the candidate cells are fine_offset levels
-	// finer than the home cells
-	int h = 0;
-	while (h + 1 <= m - 1 && (n >> (3 * (h + 1))) >= uint64_t(std::max(1, home_target)))
-		++h;
-	const int mf = std::min(10, h + std::max(1, fine_offset));
+	const WalkLevel lv = walk_level(n, m, cells_auto ? 0 : home_target, fine_offset, kWalkFill, excl.offsets ? 2 : 4);
+	const int h = lv.h, mf = std::min(10, lv.h + lv.s);
 	const uint64_t tiles = (n + 63) / 64;
 	HomeParams P{};
 	P.spos = spos.data();
@@ -734,35 +747,45 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 		P.cw[a] = float(double(extent) * k / 1023.0);
 		P.margin[a] = float(W * 1.001 + 1e-5 * double(extent) + 1e-3);
 	}
-	const uint64_t num_fine = uint64_t(1) << (3 * mf);
-	cell_begin.resize(num_fine);
-	cell_end.resize(num_fine);
-	fill_u32(cell_begin.data(), 0u, num_fine, s);
-	fill_u32(cell_end.data(), 0u, num_fine, s);
-	k_cell_ranges<<<grid_for(n, 256), 256, 0, s>>>(sorter.codes.data(), n, 3 * (10 - mf), cell_begin.data(),
-													cell_end.data());
+	const uint64_t num_fine = uint64_t(1) << (3 * mf), num_home = uint64_t(1) << (3 * h);
+	walk_cells.resize(num_fine + num_home);
+	uint2* fine = walk_cells.data();
+	uint2* home = fine + num_fine;
+	fill_u32(reinterpret_cast<uint32_t*>(fine), 0u, 2 * (num_fine + num_home), s);
+	k_walk_cells<<<grid_for(n, 256), 256, 0, s>>>(sorter.codes.data(), n, 3 * (10 - mf), 3 * (10 - h), fine, home);
 	MMD_LAUNCH_CHECK();
+	P.fine = fine;
+	P.home = home;
 	P.rc2 = cutoff_squared;
 	P.box = make_devbox(box);
 	P.ex = excl;
+	P.ex_slot = excl_symmetric && excl.offsets && !excl.rigid_body_id ? sorter.inverse.data() : nullptr;
 	P.pre = home_prefilter_band(box, domain_min, domain_max, h, cutoff, &P.pre_lo2, &P.pre_hi2) ? 1 : 0;
 	// the stencil depends on the geometry only: made and uploaded when that changes
+	const bool wraps = P.box.periodic[0] && P.box.periodic[1] && P.box.periodic[2];
 	const std::vector<float> key = {float(h),	   float(P.s),		   float(P.reach[0]), float(P.reach[1]),
 									float(P.reach[2]), float(P.full[0]),   float(P.full[1]),  float(P.full[2]),
 									P.cw[0],		   P.cw[1],			   P.cw[2],			  P.margin[0],
-									P.margin[1],	   P.margin[2],		   P.rc2};
+									P.margin[1],	   P.margin[2],		   P.rc2,			  wraps ? 1.0f : 0.0f};
 	if (key != stencil_key) {
 		stencil_key = key;
-		stencil_host = home_stencil(h, P.s, P.reach, P.full, P.cw, P.margin, P.rc2, 8192);
-		if (!stencil_host.empty()) {
-			stencil_dev.resize(stencil_host.size());
-			MMD_HIP(hipMemcpy(stencil_dev.data(), stencil_host.data(), sizeof(int4) * stencil_host.size(),
-							  hipMemcpyHostToDevice));
+		const std::vector<int4> cells = home_stencil(h, P.s, P.reach, P.full, P.cw, P.margin, P.rc2, 8192);
+		stencil_n = uint32_t(cells.size());
+		if (stencil_n > 0 && wraps) {
+			std::vector<uint32_t> words;
+			for (const int4& o : cells)
+				words.push_back(stencil_offset_code(o, mf));
+			stencil_codes.resize(stencil_n);
+			MMD_HIP(hipMemcpy(stencil_codes.data(), words.data(), sizeof(uint32_t) * stencil_n, hipMemcpyHostToDevice));
+		} else if (stencil_n > 0) {
+			stencil_dev.resize(stencil_n);
+			MMD_HIP(hipMemcpy(stencil_dev.data(), cells.data(), sizeof(int4) * stencil_n, hipMemcpyHostToDevice));
 		}
 	}
-	if (!stencil_host.empty()) {
-		P.stencil = stencil_dev.data();
-		P.stencil_n = uint32_t(stencil_host.size());
+	if (stencil_n > 0) {
+		P.stencil_code = wraps ? stencil_codes.data() : nullptr;
+		P.stencil = wraps ? nullptr : stencil_dev.data();
+		P.stencil_n = stencil_n;
 	}
 	if (!ref_complete) {
 		// keep exactly the pairs the reference grid's stencil reaches
@@ -783,18 +806,6 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 		const double mean = double(n) / volume * 4.0 / 3.0 * 3.141592653589793 * double(cutoff) * cutoff * cutoff;
 		home_cap = uint32_t(std::min(1.6 * mean + 16.0, 4096.0) + 3) & ~3u;
 	}
-	const uint64_t home_cells = uint64_t(P.num_home);
-	home_begin.resize(home_cells);
-	home_end.resize(home_cells);
-	fill_u32(home_begin.data(), 0u, home_cells, s);
-	fill_u32(home_end.data(), 0u, home_cells, s);
-	k_cell_ranges<<<grid_for(n, 256), 256, 0, s>>>(sorter.codes.data(), n, 3 * (10 - h), home_begin.data(),
-													home_end.data());
-	MMD_LAUNCH_CHECK();
-	P.home_begin = home_begin.data();
-	P.home_end = home_end.data();
-	P.fine_begin = cell_begin.data();
-	P.fine_end = cell_end.data();
 	const unsigned groups = unsigned((P.num_home + kHomeWaves - 1) / kHomeWaves);
 	const unsigned grid = std::max(8u, (groups + 7u) / 8u * 8u);
 	for (int attempt = 0; attempt < 2; ++attempt) {
@@ -806,7 +817,11 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 		P.cap = home_cap;
 		k_uniform_tile_base<<<grid_for(tiles + 1, 256), 256, 0, s>>>(tile_base.data(), tiles, 64u * home_cap);
 		MMD_LAUNCH_CHECK();
-		k_walk_home<true><<<grid, 256, 0, s>>>(P, counts.data(), nbr.data());
+		const int mode = walk_mode(P);
+		const auto kern = mode == kWalkPlain	 ? k_walk_home<kWalkPlain>
+						  : mode == kWalkOwnRows ? k_walk_home<kWalkOwnRows>
+												 : k_walk_home<kWalkGeneral>;
+		kern<<<grid, 256, 0, s>>>(P, counts.data(), nbr.data());
 		MMD_LAUNCH_CHECK();
 		count_stats(n, s);
 		uint32_t* host = readback.ptr; // max count, flag word, total entries (2 words)

@@ -85,15 +85,19 @@ struct PairlistImpl {
 	DevArray<uint32_t> cell_begin, cell_end;
 	// full neighbour list over sorted indices in wave tiles (see NbrList)
 	DevArray<uint32_t> counts, tile_rows, tile_base, nbr;
-	// home-cell walk: home-level cell ranges and the per-slot capacity of its rows
-	DevArray<uint32_t> home_begin, home_end;
+	// home-cell walk: its fine, then home cells' {begin, end} and the capacity of its rows
+	DevArray<uint2> walk_cells;
 	uint32_t home_cap = 0;
 	// cell configuration of the home walk: home cells of the finest level holding at
 	// least home_target particles on average, candidate cells fine_offset levels below
 	int home_target = 24, fine_offset = 2;
-	std::vector<int4> stencil_host; // the home walk's fine-cell stencil
+	bool cells_auto = true;         // neither set nor tuned: walk_level chooses
+	bool excl_symmetric = false;    // every exclusion is in both ends' rows (the Patch's own CSR)
+	// the home walk's fine-cell stencil: Morton codes in a wholly periodic box, else offsets
+	DevArray<uint32_t> stencil_codes;
 	DevArray<int4> stencil_dev;
-	std::vector<float> stencil_key; // the parameters stencil_dev was made for
+	uint32_t stencil_n = 0;
+	std::vector<float> stencil_key; // the parameters the stencil was made for
 	PinnedWords readback{8};
 	int home_level = -1; // level of the last home-cell walk (-1: count / scan / fill path)
 	uint64_t list_version = 0; // counts the builds and re-walks that rewrote the rows

@@ -878,6 +878,7 @@ void PatchImpl::build(float pairlist_cutoff, hipStream_t s) {
 		ev.num_particles = n;
 	}
 	pl->excl = ev;
+	pl->excl_symmetric = true; // rebuild_exclusions enters each pair in both rows
 	pl->build(pos[cur].data(), slot_of_canon.data(), true, nullptr, n, pairlist_cutoff, s);
 	// The sorted positions become the slot-order state; gather the rest.
 	slot_tmp.resize(std::max<uint64_t>(n, 1));
@@ -1290,6 +1291,7 @@ void PatchImpl::set_cells(int home_target, int fine_offset) {
 		raise(MARSMD_ERR_VALUE, "Patch: fine_offset must be in [1, 4]");
 	pl->home_target = home_target;
 	pl->fine_offset = fine_offset;
+	pl->cells_auto = false;
 }
 
 void PatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, uint64_t num_steps, hipStream_t s,
@@ -1308,10 +1310,11 @@ void PatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, 
 			return b;
 		};
 		int bt = pl->home_target, bf = pl->fine_offset;
+		bool own = pl->cells_auto; // the library's own choice, until a candidate beats it
 		best = measure();
 		for (int t : {8, 12, 16, 24, 48})
 			for (int f : {1, 2, 3}) {
-				if (t == bt && f == bf)
+				if (!own && t == bt && f == bf)
 					continue;
 				set_cells(t, f);
 				const double ms = measure();
@@ -1319,9 +1322,11 @@ void PatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, 
 					best = ms;
 					bt = t;
 					bf = f;
+					own = false;
 				}
 			}
 		set_cells(bt, bf);
+		pl->cells_auto = own;
 		(void)pl->rewalk_ms(s); // the live list as the choice walks it
 	}
 	*walk_out = best > 0.0 ? best : 0.0;
