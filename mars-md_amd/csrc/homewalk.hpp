@@ -111,6 +111,9 @@ struct HomeParams {
 	const uint32_t* stencil_code;
 	const int4* stencil;
 	uint32_t stencil_n;
+	// rows in the order of a coarser level's cells: one list of codes for each position of a
+	// home cell within its cell of that level, the home code's bits under this mask
+	uint32_t stencil_lists;
 };
 
 // The fine cells of the walk's enumeration that pass its gap test, as offsets (see
@@ -159,21 +162,20 @@ inline std::vector<int4> home_stencil(int h, int s, const int reach[3], const in
 	return out;
 }
 // The walk's home level h and its fine cells' depth s below it. target > 0: the finest
-// level holding `target` particles per home cell on average, and `offset`. Else the
-// library's own choice for n particles (fine cells = home cells, which the candidates'
+// level below m holding `target` particles per home cell on average, and `offset`. Else
+// the library's own choice for n particles (fine cells = home cells, which the candidates'
 // bounding-box test prunes more cheaply than a larger stencil does): a level finer while
-// its cells hold 5 particles on average, or (`fill`: home cells that occupy the chip) 1
-// while there are fewer cells than that. Walk times (us; one beads type, cutoff 35):
-// 10k beads at 6.4e-4 per A^3: level 2 (156 a cell) 642, 3 (20) 54, 4 (2.4) 21; 60k at
-// 1.25e-4: 3 (117) 240, 4 (15) 31, 5 (1.8) 44; 250k: 4 (61) 150, 5 (7.6) 67; 1M: 5 (30)
-// 261, 6 (3.8) 375.
+// its cells hold per_cell particles on average or there are fewer of them than occupy the
+// chip (`fill`). Walk times (us; one bead type, cutoff 35): 10k beads at 6.4e-4 per A^3:
+// level 2 (156 a cell) 642, 3 (20) 54, 4 (2.4) 21; 60k at 1.25e-4: 3 (117) 240, 4 (15) 31,
+// 5 (1.8) 44; 250k: 4 (61) 150, 5 (7.6) 67; 1M: 5 (30) 261, 6 (3.8) 375.
 struct WalkLevel {
 	int h, s;
 };
 inline WalkLevel walk_level(uint64_t n, int m, int target, int offset, double fill, uint64_t per_cell = 4) {
 	int h = 0;
 	if (target > 0) {
-		while (h + 1 <= m && (n >> (3 * (h + 1))) >= uint64_t(target))
+		while (h + 1 <= m - 1 && (n >> (3 * (h + 1))) >= uint64_t(target))
 			++h;
 		return WalkLevel{h, offset};
 	}
@@ -181,6 +183,14 @@ inline WalkLevel walk_level(uint64_t n, int m, int target, int offset, double fi
 		++h;
 	return WalkLevel{h, 0};
 }
+// A Patch's rows list a particle's neighbours by the Morton order of their offsets from
+// the particle's cell at the level that holds kRowTarget particles per cell on average (by
+// slot where that level's stencil wraps onto itself on every axis), whatever level the
+// walk runs at: the FP32 sum over a row is then the same bits.
+constexpr int kRowTarget = 24, kRowOffset = 2;
+// particles up to which rows by slot come from walking the whole box (n / 64 candidate
+// blocks a home cell)
+constexpr uint64_t kWholeBoxMax = 16384;
 
 // An offset of home_stencil as the Morton code of its components modulo 2^level cells.
 inline uint32_t stencil_offset_code(const int4& o, int level) {
@@ -422,11 +432,13 @@ template<int MODE>
 struct WalkCells {
 	const HomeParams& P;
 	uint32_t home, total;
+	const uint32_t* codes; // this home cell's list
 	uint32_t base[3], mask[3]; // home code with every bit outside the axis set, axis bits
 	int hc[3], lo[3], nax[3];
 	__device__ __forceinline__ WalkCells(const HomeParams& P_, uint32_t home_) : P(P_), home(home_) {
 		const uint32_t all = uint32_t((uint64_t(1) << (3 * (P.h + P.s))) - 1u);
-		const uint32_t code = home << (3 * P.s);
+		const uint32_t code = all ? home << (3 * P.s) : 0u; // (fine level 0: one cell, the whole box)
+		codes = P.stencil_code + uint64_t(home & P.stencil_lists) * P.stencil_n;
 #pragma unroll
 		for (int a = 0; a < 3; ++a) {
 			mask[a] = (0x24924924u >> a) & all;
@@ -453,7 +465,7 @@ struct WalkCells {
 		}
 	}
 	__device__ __forceinline__ uint32_t offset(uint32_t k) const { // the stencil word, loaded ahead
-		return (MODE != kWalkGeneral || P.stencil_code) && k < total ? P.stencil_code[k] : 0u;
+		return (MODE != kWalkGeneral || P.stencil_code) && k < total ? codes[k] : 0u;
 	}
 	__device__ __forceinline__ uint2 range(uint32_t k, uint32_t off) const {
 		uint2 none = make_uint2(0u, 0u);

@@ -96,7 +96,7 @@ struct PairlistImpl {
 	// the home walk's fine-cell stencil: Morton codes in a wholly periodic box, else offsets
 	DevArray<uint32_t> stencil_codes;
 	DevArray<int4> stencil_dev;
-	uint32_t stencil_n = 0;
+	uint32_t stencil_n = 0, stencil_lists = 1;
 	std::vector<float> stencil_key; // the parameters the stencil was made for
 	PinnedWords readback{8};
 	int home_level = -1; // level of the last home-cell walk (-1: count / scan / fill path)
