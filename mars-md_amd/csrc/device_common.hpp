@@ -594,6 +594,68 @@ __device__ inline GridSample sample_cubic(const marsmd_grid_view& g, float px, f
 	return s;
 }
 
+// The value of lane K of this lane's quad (all four lanes active).
+template<int K>
+__device__ __forceinline__ float quad_lane(float v) {
+	return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), K * 0x55, 0xf, 0xf, true));
+}
+
+// sample_cubic of one position by the four lanes of a quad (all at the same position, all
+// active): lane k reads the four runs of the stencil's y row k and does its x pass, the
+// quad exchanges those 8 values and every lane does the y and z passes. Each product and
+// sum is sample_cubic's, in its order: the same bits, with 16 taps in a lane's registers
+// instead of 64 and a quarter of the loads in a lane's chain.
+__device__ inline GridSample sample_cubic_quad(const marsmd_grid_view& g, float px, float py, float pz, int bc) {
+	const CubicStencil c = cubic_stencil(g, px, py, pz);
+	const uint64_t nx = g.dims[0], ny = g.dims[1], nz = g.dims[2];
+	const int iy = int(threadIdx.x & 3u);
+	float r[4][4]; // [x][z] taps of row iy
+	if (nx * ny * nz < (1ull << 30) && c.hx >= 1 && int64_t(c.hx) + 2 < int64_t(nx) && c.hy >= 1 &&
+		int64_t(c.hy) + 2 < int64_t(ny) && c.hz >= 1 && int64_t(c.hz) + 2 < int64_t(nz)) {
+		const uint32_t sy = 4u * uint32_t(nz), sx = sy * uint32_t(ny); // as cubic_taps_interior
+		const uint32_t first = uint32_t(c.hx - 1) * sx + uint32_t(c.hy - 1 + iy) * sy + 4u * uint32_t(c.hz - 1);
+		MMD_GLOBAL_AS const char* __restrict__ base = (MMD_GLOBAL_AS const char*)g.data;
+#pragma unroll
+		for (int ix = 0; ix < 4; ++ix) {
+			const GridRun4 v = *(MMD_GLOBAL_AS const GridRun4*)(base + (first + uint32_t(ix) * sx));
+#pragma unroll
+			for (int q = 0; q < 4; ++q)
+				r[ix][q] = v.v[q];
+		}
+	} else {
+		const int64_t sx = int64_t(ny) * int64_t(nz); // as cubic_taps_mapped
+		const int64_t oy = tap_offset(c.hy - 1 + iy, int(ny), bc, int64_t(nz));
+#pragma unroll
+		for (int ix = 0; ix < 4; ++ix) {
+			const int64_t ox = tap_offset(c.hx - 1 + ix, int(nx), bc, sx);
+			if (ox < 0 || oy < 0) {
+#pragma unroll
+				for (int q = 0; q < 4; ++q)
+					r[ix][q] = 0.0f;
+			} else {
+				load_run<4>(grid_data(g) + ox + oy, c.hz - 1, int(nz), bc, r[ix]);
+			}
+		}
+	}
+	const CrWeights Wx = cr_weights(c.wx), Wy = cr_weights(c.wy), Wz = cr_weights(c.wz);
+	float d2x[4], d2y[4], v2[4];
+#pragma unroll
+	for (int iz = 0; iz < 4; ++iz) {
+		const float d1 = dot4(Wx.d, r[0][iz], r[1][iz], r[2][iz], r[3][iz]);
+		const float v1 = dot4(Wx.w, r[0][iz], r[1][iz], r[2][iz], r[3][iz]);
+		const float v[4] = {quad_lane<0>(v1), quad_lane<1>(v1), quad_lane<2>(v1), quad_lane<3>(v1)};
+		d2x[iz] = dot4(Wy.w, quad_lane<0>(d1), quad_lane<1>(d1), quad_lane<2>(d1), quad_lane<3>(d1));
+		d2y[iz] = dot4(Wy.d, v[0], v[1], v[2], v[3]);
+		v2[iz] = dot4(Wy.w, v[0], v[1], v[2], v[3]);
+	}
+	const float gg[3] = {dot4(Wz.w, d2x[0], d2x[1], d2x[2], d2x[3]), dot4(Wz.w, d2y[0], d2y[1], d2y[2], d2y[3]),
+						 dot4(Wz.d, v2[0], v2[1], v2[2], v2[3])};
+	GridSample s;
+	s.value = dot4(Wz.w, v2[0], v2[1], v2[2], v2[3]);
+	mat_transpose_transform(g.basis_inv, gg, s.grad);
+	return s;
+}
+
 // Runs body(grid view) for the active lanes whose grid index is gid, one distinct
 // index at a time: the index is wave-uniform inside, so the view is read with scalar
 // loads instead of occupying vector registers in every lane. Lanes with gid < 0 skip.
@@ -619,8 +681,9 @@ __device__ __forceinline__ void for_each_grid(int gid, const marsmd_grid_view* _
 
 // compute_position_dependent_force (src/Interactions/Nonbonded/Pmf.h:68-124) for one
 // interpolation scheme. The returned .w is the PMF energy (the reference's .t). Each
-// lane adds its type's terms in term order, as the reference does.
-template<bool CUBIC>
+// lane adds its type's terms in term order, as the reference does. QUAD: the four lanes of
+// a quad ask for one position together and share the cubic sampling.
+template<bool CUBIC, bool QUAD = false>
 __device__ inline float4 position_dependent_force_t(float px, float py, float pz, int type,
 													const marsmd_particle_types& types,
 													const marsmd_grid_view* __restrict__ grids, const float ef[3]) {
@@ -642,7 +705,9 @@ __device__ inline float4 position_dependent_force_t(float px, float py, float pz
 			if (g.data == nullptr)
 				return;
 			const int bc = term.boundary_condition >= 0 ? term.boundary_condition : g.boundary_condition;
-			const GridSample s = CUBIC ? sample_cubic(g, px, py, pz, bc) : sample_linear(g, px, py, pz, bc);
+			const GridSample s = !CUBIC ? sample_linear(g, px, py, pz, bc)
+								 : QUAD ? sample_cubic_quad(g, px, py, pz, bc)
+										: sample_cubic(g, px, py, pz, bc);
 			const float ns = -term.scale;
 			f.x += s.grad[0] * ns;
 			f.y += s.grad[1] * ns;
@@ -655,8 +720,9 @@ __device__ inline float4 position_dependent_force_t(float px, float py, float pz
 		for_each_grid(types.force_grid_id[type][a], grids, [&](const marsmd_grid_view& g) {
 			if (g.data == nullptr)
 				return;
-			const float v = CUBIC ? sample_cubic(g, px, py, pz, g.boundary_condition).value
-								  : sample_linear(g, px, py, pz, g.boundary_condition).value;
+			const float v = !CUBIC ? sample_linear(g, px, py, pz, g.boundary_condition).value
+							: QUAD ? sample_cubic_quad(g, px, py, pz, g.boundary_condition).value
+								   : sample_cubic(g, px, py, pz, g.boundary_condition).value;
 			const float add = types.force_grid_scale[type][a] * v;
 			if (a == 0)
 				f.x += add;

@@ -49,11 +49,12 @@ __device__ __forceinline__ uint32_t fb(float f) { return __float_as_uint(f); }
 // tabulated-only path carries none of the analytical code). `knots` points into LDS or
 // global memory, as the caller's instantiation says: a pointer that might be either
 // would be read with flat loads, whose waits also drain the position gathers in flight.
+// Returns what the pair adds to the slot's force and energy (+-0 from a pair that is skipped,
+// which leaves the sums' bits unchanged: they start at +0 and can never become -0).
 template<bool ANALYTIC>
-__device__ __forceinline__ void nb_pair(const float4& p, uint32_t ct, uint32_t tt, const float4& q,
-										const NbTables& T, const float* __restrict__ knots, const NbLds& S,
-										const DevBox& box, float cut_d, bool energy, float& fx, float& fy,
-										float& fz, float& e) {
+__device__ __forceinline__ float4 nb_pair_term(const float4& p, uint32_t ct, uint32_t tt, const float4& q,
+											   const NbTables& T, const float* __restrict__ knots, const NbLds& S,
+											   const DevBox& box, float cut_d, bool energy) {
 	const uint32_t mj = fb(q.w);
 	const uint32_t tj = meta_type(mj);
 	// ct < cj, from the meta words (canonical index in the high bits; a pad entry is the
@@ -103,17 +104,13 @@ __device__ __forceinline__ void nb_pair(const float4& p, uint32_t ct, uint32_t t
 		// (force over distance once, then per axis: the product rounds in another order
 		// than fm * (r / d), a relative change of about 1e-7)
 		const float g = ((in_cut && d > 1e-6f) ? (t_is_x ? -fm : fm) : 0.0f) * inv;
-		fx += g * r.x;
-		fy += g * r.y;
-		fz += g * r.z;
-		if (energy)
-			e += (in_cut && !(d < 1e-6f)) ? en * 0.5f : 0.0f;
-		return;
+		return make_float4(g * r.x, g * r.y, g * r.z, energy && in_cut && !(d < 1e-6f) ? en * 0.5f : 0.0f);
 	}
+	const float4 none = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 	const uint32_t tag = S.tag[(tx << 4) | ty];
 	const uint32_t terms = tag & T.enabled;
 	if (terms == 0u)
-		return;
+		return none;
 	const float3 r = wrap_diff(box, sub3(py, px));
 	const float r2 = len2(r);
 	const float d = sqrtf(r2);
@@ -124,10 +121,8 @@ __device__ __forceinline__ void nb_pair(const float4& p, uint32_t ct, uint32_t t
 		uy = inv * r.y;
 		uz = inv * r.z;
 	}
-	if (d < 1e-6f)
-		return;
-	if (d > cut_d)
-		return;
+	if (d < 1e-6f || d > cut_d)
+		return none;
 	float fm = 0.0f, en = 0.0f;
 	if (ANALYTIC && (terms & kAnalyticTerms)) {
 		const float4 cx = S.coef[tx], cy = S.coef[ty];
@@ -140,17 +135,20 @@ __device__ __forceinline__ void nb_pair(const float4& p, uint32_t ct, uint32_t t
 		en += v.e;
 	}
 	const float gx = fm * ux, gy = fm * uy, gz = fm * uz;
-	if (t_is_x) {
-		fx += -gx;
-		fy += -gy;
-		fz += -gz;
-	} else {
-		fx += gx;
-		fy += gy;
-		fz += gz;
-	}
+	const float en_half = energy ? en * 0.5f : 0.0f;
+	return t_is_x ? make_float4(-gx, -gy, -gz, en_half) : make_float4(gx, gy, gz, en_half);
+}
+template<bool ANALYTIC>
+__device__ __forceinline__ void nb_pair(const float4& p, uint32_t ct, uint32_t tt, const float4& q,
+										const NbTables& T, const float* __restrict__ knots, const NbLds& S,
+										const DevBox& box, float cut_d, bool energy, float& fx, float& fy,
+										float& fz, float& e) {
+	const float4 v = nb_pair_term<ANALYTIC>(p, ct, tt, q, T, knots, S, box, cut_d, energy);
+	fx += v.x;
+	fy += v.y;
+	fz += v.z;
 	if (energy)
-		e += en * 0.5f;
+		e += v.w;
 }
 
 // Position record of slot j, addressed by a 32-bit byte offset from the array base
@@ -215,6 +213,112 @@ __device__ __forceinline__ float4 nb_force_list(uint32_t t, const float4& p, con
 	return make_float4(fx, fy, fz, e);
 }
 
+// LDS written by some lanes of this wave and read by others: order the accesses.
+__device__ __forceinline__ void wave_lds_order() {
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The same sum with each slot's row dealt to m = 2^split adjacent lanes (4 or 8; this one's
+// index `sub`): a round takes m groups of 4 entries, lane k evaluates group k's
+// pairs and leaves their terms in LDS, and then four lanes per slot, one a component, add
+// the round's 4 m terms to their running sums one by one. The additions are
+// nb_force_list's, in its order, so the bits do not depend on the split. A row of g groups
+// takes ceil(g / m) rounds instead of g, which is what bounds a step whose slots do not
+// fill the chip; the serial additions are about a quarter of a round's instructions
+// (handing the sum from lane to lane instead: the step of 10k beads with 115 neighbours
+// 14.6 us instead of 11.2).
+// log2 of the lanes that share a slot's row (0: one), from the slots, the longest row and
+// the entries of all rows: 8 lanes up to 2^15 slots and 4 up to 7 2^14 (7 waves on each of
+// the chip's 1024 SIMDs), of which each has a group of the longest row to take; with long
+// rows (12 groups on average) beyond that while a lane keeps 6 groups of the longest one,
+// whose tail bounds uneven rows. Step kernel, us at 1, 4, 8, 16 lanes: 10k beads of 115
+// neighbours 39, 16, 11.2, 11.4; 60k of 22 (trilinear grid) 18, 14.6, 18, 27; 100k polymer
+// beads 92, 44, 41, 45; 100k of 22 (tricubic) 32, 27, 29, 47; 120k of 22 (trilinear) 23, 24,
+// 32; 200k of 108 74, 64, 67, 77; 1M of 22 (tricubic) 140, 165, 213.
+inline uint32_t row_split(uint64_t n, uint32_t max_neighbors, uint64_t entries) {
+	const uint32_t groups = (max_neighbors + 3u) >> 2;
+	const bool long_rows = entries >= 48 * n;
+	for (uint32_t s : {3u, 2u})
+		if ((groups >> s) >= 1 && (n <= (s == 3 ? 1u << 15 : 7u << 14) || (long_rows && (groups >> s) >= 6)))
+			return s;
+	return 0;
+}
+
+struct RowHead { // what a lane reads before its first pair term
+	float4 p;
+	uint32_t ng;
+	const uint4* row;
+	uint4 j, self; // its first group's entries; the slot itself four times
+};
+// (a slot past the end stands in as the last slot with an empty row)
+__device__ __forceinline__ RowHead row_head(uint32_t slot, uint32_t n, uint32_t sub, const float4* __restrict__ pos,
+											const NbrList& L) {
+	const uint32_t t = min(slot, n - 1u);
+	RowHead h;
+	h.p = pos[t];
+	h.ng = slot < n ? (L.count[t] + 3u) >> 2 : 0u;
+	h.row = reinterpret_cast<const uint4*>(L.nbr + L.tile_base[t >> 6]) + (t & 63u);
+	h.self = make_uint4(t, t, t, t);
+	h.j = h.self;
+	if (sub < h.ng)
+		h.j = h.row[uint64_t(sub) * 64u];
+	return h;
+}
+// Floats of LDS per wave: three components (with energies four) of 64 / m rows of 4 m terms
+// (and 4 spare against bank conflicts).
+constexpr uint32_t split_terms(bool energy) { return (energy ? 4u : 3u) * (256u + 64u); }
+// The wave's slots' sums: lane 4 s + c (s < 64 >> split) returns component c of the wave's
+// slot s (x, y, z, energy). Called by every lane of the wave.
+template<bool ANALYTIC>
+__device__ __forceinline__ float nb_force_split(const RowHead& h, uint32_t sub, uint32_t split,
+												const float4* __restrict__ pos, const NbTables& T,
+												const float* __restrict__ knots, const NbLds& S, const DevBox& box,
+												float cut_d, bool energy, float* terms) {
+	const float4 p = h.p;
+	const uint32_t mt = fb(p.w);
+	const uint32_t ct = meta_canon(mt);
+	const uint32_t tt = meta_type(mt);
+	const uint32_t m = 1u << split, ng = h.ng, lane = threadIdx.x & 63u;
+	const uint32_t row = 4u * m + 4u, comp = (64u >> split) * row;
+	float* const mine = terms + (lane >> split) * row + 4u * sub;
+	const uint32_t slot = lane >> 2, c = lane & 3u;
+	const bool adds = slot < (64u >> split) && (c < 3u || energy);
+	const float* const theirs = terms + c * comp + slot * row;
+	float sum = 0.0f;
+	uint4 j = h.j; // past the row: the slot itself, whose terms are +0
+	for (uint32_t g0 = 0; __ballot(g0 < ng) != 0; g0 += m) {
+		const float4 q0 = pos_at(pos, j.x), q1 = pos_at(pos, j.y), q2 = pos_at(pos, j.z), q3 = pos_at(pos, j.w);
+		j = h.self;
+		if (g0 + m + sub < ng)
+			j = h.row[uint64_t(g0 + m + sub) * 64u];
+		const float4 t0 = nb_pair_term<ANALYTIC>(p, ct, tt, q0, T, knots, S, box, cut_d, energy);
+		const float4 t1 = nb_pair_term<ANALYTIC>(p, ct, tt, q1, T, knots, S, box, cut_d, energy);
+		const float4 t2 = nb_pair_term<ANALYTIC>(p, ct, tt, q2, T, knots, S, box, cut_d, energy);
+		const float4 t3 = nb_pair_term<ANALYTIC>(p, ct, tt, q3, T, knots, S, box, cut_d, energy);
+		wave_lds_order(); // (the last round's reads)
+		*reinterpret_cast<float4*>(mine) = make_float4(t0.x, t1.x, t2.x, t3.x);
+		*reinterpret_cast<float4*>(mine + comp) = make_float4(t0.y, t1.y, t2.y, t3.y);
+		*reinterpret_cast<float4*>(mine + 2u * comp) = make_float4(t0.z, t1.z, t2.z, t3.z);
+		if (energy)
+			*reinterpret_cast<float4*>(mine + 3u * comp) = make_float4(t0.w, t1.w, t2.w, t3.w);
+		wave_lds_order();
+		if (adds) {
+			for (uint32_t k = 0; k < m; k += 4) {
+				float4 v[4];
+#pragma unroll
+				for (uint32_t u = 0; u < 4; ++u)
+					v[u] = *reinterpret_cast<const float4*>(theirs + 4u * (k + u));
+#pragma unroll
+				for (uint32_t u = 0; u < 4; ++u)
+					sum = sum + v[u].x + v[u].y + v[u].z + v[u].w;
+			}
+		}
+	}
+	return sum;
+}
+
 // Stage the tag matrix, the table parameters and the per-type coefficients in LDS (the
 // caller synchronises).
 __device__ __forceinline__ void stage_params(const NbTables& T, NbLds& S) {
@@ -255,7 +359,13 @@ __device__ __forceinline__ void stage_tables(const NbTables& T, const float* __r
 											 NbLds& S) {
 	stage_params(T, S);
 	if (T.lds) {
-		for (int i = threadIdx.x; i < T.total_knots; i += blockDim.x)
+		// 16 bytes a lane (a caller's knots may be only 4-byte aligned: GridRun4), then the rest
+		const int quads = T.total_knots >> 2;
+		for (int i = threadIdx.x; i < quads; i += blockDim.x) {
+			const GridRun4 v = reinterpret_cast<const GridRun4*>(knots_g)[i];
+			reinterpret_cast<float4*>(lds_knots)[i] = make_float4(v.v[0], v.v[1], v.v[2], v.v[3]);
+		}
+		for (int i = 4 * quads + int(threadIdx.x); i < T.total_knots; i += blockDim.x)
 			lds_knots[i] = knots_g[i];
 	}
 	__syncthreads();

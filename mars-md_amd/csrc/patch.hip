@@ -37,19 +37,47 @@ namespace mmd {
 namespace {
 
 constexpr int kBlock = 256;
+// workgroups of the kernels that deal a slot's row to several lanes: eight waves share
+// the staged tables
+constexpr int kSplitBlock = 512;
 
 
 template<bool ANALYTIC>
 __global__ __launch_bounds__(kBlock) void k_nb_forces(const float4* __restrict__ pos, uint64_t n, NbrList L,
-													  NbTables T, const float* __restrict__ knots_g, DevBox box,
+													  const NbTables* __restrict__ T_dev, const float* __restrict__ knots_g, DevBox box,
 													  float cut_d, int energy, float4* __restrict__ force) {
 	extern __shared__ float lds_knots[];
 	__shared__ NbLds lds_nb;
+	const NbTables& T = *T_dev;
 	stage_tables(T, knots_g, lds_knots, lds_nb);
 	const uint64_t t = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
 	if (t >= n)
 		return;
 	force[t] = nb_force<ANALYTIC>(uint32_t(t), pos[t], pos, L, T, lds_knots, knots_g, lds_nb, box, cut_d, energy != 0);
+}
+
+// k_nb_forces with each row dealt to 2^split lanes (nb_force_split).
+template<bool ANALYTIC>
+__global__ __launch_bounds__(kSplitBlock) void k_nb_forces_split(const float4* __restrict__ pos, uint64_t n, NbrList L,
+																 const NbTables* __restrict__ T_dev,
+																 const float* __restrict__ knots_g, DevBox box,
+																 float cut_d, int energy, float4* __restrict__ force,
+																 uint32_t split) {
+	extern __shared__ float lds_knots[];
+	__shared__ NbLds lds_nb;
+	const NbTables& T = *T_dev;
+	__shared__ float terms[kSplitBlock / 64][split_terms(true)];
+	const uint32_t i = blockIdx.x * kSplitBlock + threadIdx.x, lane = threadIdx.x & 63u;
+	// in flight while the tables are staged
+	const RowHead h = row_head(i >> split, uint32_t(n), i & ((1u << split) - 1u), pos, L);
+	stage_tables(T, knots_g, lds_knots, lds_nb);
+	float* const wt = terms[threadIdx.x >> 6];
+	const uint32_t sub = i & ((1u << split) - 1u);
+	const float f = T.lds ? nb_force_split<ANALYTIC>(h, sub, split, pos, T, lds_knots, lds_nb, box, cut_d, energy != 0, wt)
+						  : nb_force_split<ANALYTIC>(h, sub, split, pos, T, knots_g, lds_nb, box, cut_d, energy != 0, wt);
+	const uint32_t t = ((i - lane) >> split) + (lane >> 2); // component lane & 3 of slot t
+	if ((lane >> 2) < (64u >> split) && t < n)
+		reinterpret_cast<float*>(force)[4u * uint64_t(t) + (lane & 3u)] = f;
 }
 
 __global__ void k_zero_force(float4* __restrict__ f, uint64_t n) {
@@ -278,15 +306,93 @@ __global__ __launch_bounds__(256) void k_prune(const float4* __restrict__ pos, u
 		p_nbr[nbr_slot_index(pb, t, m)] = s;
 }
 
+// Where a step's position-dependent force comes from: no grids (the electric field alone,
+// which Brownian steps add), sampled here linearly or cubically, or given (sampled
+// before: by k_pmf_force, or by the workgroup's quads). A template parameter, so that a kernel carries no sampler's
+// registers but its own (the cubic one's hold the fused step at 4 waves per SIMD).
+constexpr int kPmfNone = 0, kPmfLinear = 1, kPmfCubic = 2, kPmfGiven = 3;
+
+// The rest of slot t's step once its nonbonded force f is summed: bonded force (from
+// `force`), position-dependent force, integrator. Returns the new position.
+template<int INTEG, bool ENERGY, int PMF>
+__device__ __forceinline__ float4 step_finish(uint32_t t, const float4 p, float4 f, float4* __restrict__ mom,
+											  float4* __restrict__ force, const marsmd_particle_types& types,
+											  const TypeStep* steps, const marsmd_grid_view* __restrict__ grids,
+											  const StepParams& S, int has_bonded, int store_force,
+											  const float4 given) {
+	if (has_bonded) {
+		const float4 b = force[t];
+		f.x += b.x;
+		f.y += b.y;
+		f.z += b.z;
+		f.w += b.w;
+	}
+	float4 pmf = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	if (PMF == kPmfGiven)
+		pmf = given;
+	else if (PMF == kPmfLinear || PMF == kPmfCubic)
+		pmf = position_dependent_force_t<PMF == kPmfCubic>(p.x, p.y, p.z, int(meta_type(fb(p.w))), types, grids, S.ef);
+	else if (INTEG == MARSMD_INTEGRATOR_BROWNIAN)
+		pmf = position_dependent_force_t<false>(p.x, p.y, p.z, int(meta_type(fb(p.w))), types, nullptr, S.ef);
+	float4 pn;
+	if (INTEG == MARSMD_INTEGRATOR_BROWNIAN) {
+		pn = bd_update(p, f, steps[meta_type(fb(p.w))], pmf, S);
+	} else {
+		if (PMF != kPmfNone) {
+			f.x += pmf.x;
+			f.y += pmf.y;
+			f.z += pmf.z;
+			f.w += pmf.w;
+		}
+		float4 mo = mom[t];
+		pn = baoab_update(p, mo, f, steps[meta_type(fb(p.w))], S);
+		mom[t] = mo;
+	}
+	if (ENERGY || store_force)
+		force[t] = f;
+	return pn;
+}
+
+// The workgroup's largest squared displacement (non-negative floats order as their bits)
+// into this step's record and the life's.
+__device__ __forceinline__ void record_displacement(const PruneView& PR, float disp2, float* lds_red) {
+	for (int o = 32; o > 0; o >>= 1)
+		disp2 = fmaxf(disp2, __shfl_xor(disp2, o));
+	if ((threadIdx.x & 63u) == 0u)
+		lds_red[threadIdx.x >> 6] = disp2;
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		float m = lds_red[0];
+		for (int w = 1; w < int(blockDim.x >> 6); ++w)
+			m = fmaxf(m, lds_red[w]);
+		atomicMax(&PR.disp[PR.since & 3u], __float_as_uint(m));
+		atomicMax(&PR.disp[4], __float_as_uint(m));
+		if (blockIdx.x == 0)
+			PR.disp[(PR.since + 1u) & 3u] = 0u; // the next step's record starts empty
+	}
+}
+
+// The particle types and the integrator's per-type constants in LDS (the caller
+// synchronises).
+template<int INTEG>
+__device__ __forceinline__ void stage_step(const marsmd_particle_types& types, const StepParams& S,
+										   marsmd_particle_types& lds_types, TypeStep* lds_steps) {
+	stage_types(types, lds_types);
+	if (threadIdx.x < uint32_t(types.num_types))
+		lds_steps[threadIdx.x] = INTEG == MARSMD_INTEGRATOR_BROWNIAN ? bd_type_step(types, int(threadIdx.x), S)
+																	 : baoab_type_step(types, int(threadIdx.x), S);
+}
+
 // The fused step: nonbonded + bonded (from `force` when has_bonded) + PMF + integrator,
 // persistent over XCD-local tiles so the table knots are staged once per workgroup.
 // Bounded to 128 VGPRs (4 waves per SIMD; the tricubic sampler alone would take ~140
 // and leave 3): measured faster despite a few dwords of spill.
-template<int INTEG, bool ENERGY, bool ANALYTIC, bool PMF_IN>
-__global__ __launch_bounds__(kBlock, 4) void k_step(const float4* __restrict__ pos, float4* __restrict__ pos_next,
+template<int INTEG, bool ENERGY, bool ANALYTIC, int PMF>
+__global__ __launch_bounds__(kBlock, PMF == kPmfCubic ? 4 : 5) void k_step(const float4* __restrict__ pos, float4* __restrict__ pos_next,
 												 float4* __restrict__ mom, float4* __restrict__ force, uint64_t n,
-												 NbrList L, NbTables T, const float* __restrict__ knots_g,
-												 marsmd_particle_types types_arg,
+												 NbrList L, const NbTables* __restrict__ T_dev,
+												 const float* __restrict__ knots_g,
+												 const marsmd_particle_types* __restrict__ types_dev,
 												 const marsmd_grid_view* __restrict__ grids, StepParams S,
 												 int has_bonded, int store_force, const float4* __restrict__ pmf_in,
 												 PruneView PR) {
@@ -295,10 +401,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_step(const float4* __restrict__ p
 	__shared__ marsmd_particle_types lds_types;
 	__shared__ float lds_red[kBlock / 64];
 	__shared__ TypeStep lds_steps[MARSMD_MAX_TYPES]; // the integrator's per-type constants
-	stage_types(types_arg, lds_types);
-	if (threadIdx.x < uint32_t(types_arg.num_types))
-		lds_steps[threadIdx.x] = INTEG == MARSMD_INTEGRATOR_BROWNIAN ? bd_type_step(types_arg, int(threadIdx.x), S)
-																	 : baoab_type_step(types_arg, int(threadIdx.x), S);
+	const NbTables& T = *T_dev;
+	stage_step<INTEG>(*types_dev, S, lds_types, lds_steps);
 	stage_tables(T, knots_g, lds_knots, lds_nb);
 	const marsmd_particle_types& types = lds_types;
 	// the pruned rows hold while the previous step's displacement record is below the
@@ -309,92 +413,125 @@ __global__ __launch_bounds__(kBlock, 4) void k_step(const float4* __restrict__ p
 		pruned = __uint_as_float(PR.disp[(PR.since - 1u) & 3u]) < PR.limit2;
 	const NbrList LL = pruned ? PR.list : L;
 	float disp2 = 0.0f;
-	// the rest of slot t's step once its nonbonded force f is summed (kernel arguments
-	// captured by value: by reference the register allocation around the grid sampler
-	// spills)
-	const auto finish = [&, pos, pos_next, mom, force, grids, S, has_bonded, store_force, pmf_in, PR](uint32_t t,
-																										 float4 f) {
-		const float4 p = pos[t];
-		if (has_bonded) {
-			const float4 b = force[t];
-			f.x += b.x;
-			f.y += b.y;
-			f.z += b.z;
-			f.w += b.w;
-		}
-		float4 pn;
-		if (INTEG == MARSMD_INTEGRATOR_BROWNIAN) {
-			const float4 pmf = PMF_IN ? pmf_in[t]
-									  : position_dependent_force(p.x, p.y, p.z, int(meta_type(fb(p.w))), types,
-																 S.has_grids ? grids : nullptr, S.ef, S.scheme);
-			pn = bd_update(p, f, lds_steps[meta_type(fb(p.w))], pmf, S);
-		} else {
-			if (S.has_grids) {
-				const float4 g = PMF_IN ? pmf_in[t]
-										: position_dependent_force(p.x, p.y, p.z, int(meta_type(fb(p.w))), types,
-																   grids, S.ef, S.scheme);
-				f.x += g.x;
-				f.y += g.y;
-				f.z += g.z;
-				f.w += g.w;
-			}
-			float4 mo = mom[t];
-			pn = baoab_update(p, mo, f, lds_steps[meta_type(fb(p.w))], S);
-			mom[t] = mo;
-		}
-		pos_next[t] = pn;
-		if (ENERGY || store_force)
-			force[t] = f;
-		if (track)
-			disp2 = fmaxf(disp2, len2(wrap_diff_uniform(S.box, sub3(pn, PR.ref[t]))));
-	};
 	const TileRange R = xcd_tiles(uint32_t((n + kBlock - 1) / kBlock));
 	for (uint32_t tile = R.tile; tile < R.end; tile += R.stride) {
 		const uint32_t lt = tile * uint32_t(kBlock) + threadIdx.x; // lane position
 		if (lt >= n)
 			continue;
 		const uint32_t t = PR.lane_slot ? PR.lane_slot[lt] : lt; // slot
-		finish(t, nb_force<ANALYTIC>(pruned ? lt : t, pos[t], pos, LL, T, lds_knots, knots_g, lds_nb, S.box, S.cut_d,
-									 ENERGY));
+		const float4 f = nb_force<ANALYTIC>(pruned ? lt : t, pos[t], pos, LL, T, lds_knots, knots_g, lds_nb, S.box,
+											S.cut_d, ENERGY);
+		const float4 pn = step_finish<INTEG, ENERGY, PMF>(t, pos[t], f, mom, force, types, lds_steps, grids, S,
+														  has_bonded, store_force,
+														  PMF == kPmfGiven ? pmf_in[t] : float4{});
+		pos_next[t] = pn;
+		if (track)
+			disp2 = fmaxf(disp2, len2(wrap_diff_uniform(S.box, sub3(pn, PR.ref[t]))));
 	}
-	if (track) {
-		// the workgroup's largest squared displacement (non-negative floats order as
-		// their bits) into this step's record and the life's
-		for (int o = 32; o > 0; o >>= 1)
-			disp2 = fmaxf(disp2, __shfl_xor(disp2, o));
-		if ((threadIdx.x & 63u) == 0u)
-			lds_red[threadIdx.x >> 6] = disp2;
-		__syncthreads();
-		if (threadIdx.x == 0) {
-			float m = lds_red[0];
-			for (int w = 1; w < kBlock / 64; ++w)
-				m = fmaxf(m, lds_red[w]);
-			atomicMax(&PR.disp[PR.since & 3u], __float_as_uint(m));
-			atomicMax(&PR.disp[4], __float_as_uint(m));
-			if (blockIdx.x == 0)
-				PR.disp[(PR.since + 1u) & 3u] = 0u; // the next step's record starts empty
-		}
-	}
+	if (track)
+		record_displacement(PR, disp2, lds_red);
 }
 
-using StepFn = decltype(&k_step<MARSMD_INTEGRATOR_BROWNIAN, false, false, false>);
-template<int I, bool E, bool A>
-StepFn pick_step_pmf(bool pmf_in) {
-	return pmf_in ? k_step<I, E, A, true> : k_step<I, E, A, false>;
+// The fused step with each slot's row dealt to 2^split lanes (nb_force_split): a workgroup
+// sums the pair forces of 512 >> split slots with all its lanes, hands them over in LDS
+// and finishes the slots with its first lanes. The next slots' first row entries are in
+// flight meanwhile, the first ones' while the tables are staged.
+template<int INTEG, bool ENERGY, bool ANALYTIC, int PMF>
+__global__ __launch_bounds__(kSplitBlock, 4) void k_step_split(
+	const float4* __restrict__ pos, float4* __restrict__ pos_next, float4* __restrict__ mom, float4* __restrict__ force,
+	uint64_t n, NbrList L, const NbTables* __restrict__ T_dev, const float* __restrict__ knots_g, uint32_t knot_words,
+	const marsmd_particle_types* __restrict__ types_dev, const marsmd_grid_view* __restrict__ grids, StepParams S,
+	int has_bonded, int store_force, PruneView PR, uint32_t split) {
+	extern __shared__ float lds_knots[]; // knot_words words (a multiple of 4), then the handed-over forces
+	__shared__ NbLds lds_nb;
+	__shared__ marsmd_particle_types lds_types;
+	__shared__ float lds_red[kSplitBlock / 64];
+	__shared__ TypeStep lds_steps[MARSMD_MAX_TYPES];
+	const NbTables& T = *T_dev;
+	const uint32_t per = uint32_t(kSplitBlock) >> split; // slots of a tile
+	const uint32_t mine = threadIdx.x >> split, sub = threadIdx.x & ((1u << split) - 1u);
+	__shared__ float terms[kSplitBlock / 64][split_terms(ENERGY)];
+	float4* lds_force = reinterpret_cast<float4*>(lds_knots + knot_words); // two tiles' forces in turn
+	float4* lds_pmf = lds_force + 2u * per;                                // and their grid forces (cubic)
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint32_t first = (threadIdx.x - lane) >> split; // the wave's first slot of a tile
+	const TileRange R = xcd_tiles(uint32_t((n + per - 1) / per));
+	RowHead h{};
+	if (R.tile < R.end)
+		h = row_head(R.tile * per + mine, uint32_t(n), sub, pos, L);
+	stage_step<INTEG>(*types_dev, S, lds_types, lds_steps);
+	stage_tables(T, knots_g, lds_knots, lds_nb);
+	const bool track = PR.lane_slot && PR.limit2 > 0.0f;
+	float disp2 = 0.0f;
+	uint32_t turn = 0;
+	for (uint32_t tile = R.tile; tile < R.end; tile += R.stride, turn ^= 1u) {
+		float* const wt = terms[threadIdx.x >> 6];
+		const float f =
+			T.lds ? nb_force_split<ANALYTIC>(h, sub, split, pos, T, lds_knots, lds_nb, S.box, S.cut_d, ENERGY, wt)
+				  : nb_force_split<ANALYTIC>(h, sub, split, pos, T, knots_g, lds_nb, S.box, S.cut_d, ENERGY, wt);
+		if ((lane >> 2) < (64u >> split))
+			reinterpret_cast<float*>(lds_force)[4u * (turn * per + first + (lane >> 2)) + (lane & 3u)] = f;
+		if (tile + R.stride < R.end)
+			h = row_head((tile + R.stride) * per + mine, uint32_t(n), sub, pos, L);
+		if (PMF == kPmfCubic) // a quad per slot samples the grids
+			for (uint32_t k = threadIdx.x >> 2; k < per && tile * per + k < n; k += kSplitBlock / 4) {
+				const float4 p = pos[tile * per + k];
+				const float4 g = position_dependent_force_t<true, true>(p.x, p.y, p.z, int(meta_type(fb(p.w))), lds_types,
+																		grids, S.ef);
+				if ((threadIdx.x & 3u) == 0u)
+					lds_pmf[turn * per + k] = g;
+			}
+		__syncthreads(); // (the other buffers' readers finished before it)
+		const uint32_t u = tile * per + threadIdx.x;
+		if (threadIdx.x < per && u < n) {
+			const uint32_t at = turn * per + threadIdx.x;
+			const float4 pn = step_finish<INTEG, ENERGY, PMF == kPmfCubic ? kPmfGiven : PMF>(
+				u, pos[u], lds_force[at], mom, force, lds_types, lds_steps, grids, S, has_bonded, store_force,
+				PMF == kPmfCubic ? lds_pmf[at] : float4{});
+			pos_next[u] = pn;
+			if (track)
+				disp2 = fmaxf(disp2, len2(wrap_diff_uniform(S.box, sub3(pn, PR.ref[u]))));
+		}
+	}
+	if (track)
+		record_displacement(PR, disp2, lds_red);
 }
-template<int I, bool E>
-StepFn pick_step_an(bool an, bool pmf_in) {
-	return an ? pick_step_pmf<I, E, true>(pmf_in) : pick_step_pmf<I, E, false>(pmf_in);
+
+using SplitStepFn = decltype(&k_step_split<MARSMD_INTEGRATOR_BROWNIAN, false, false, kPmfNone>);
+template<int I, bool E, bool A>
+SplitStepFn pick_split_pmf(int pmf) {
+	return pmf == kPmfCubic ? k_step_split<I, E, A, kPmfCubic>
+							: pmf == kPmfLinear ? k_step_split<I, E, A, kPmfLinear> : k_step_split<I, E, A, kPmfNone>;
 }
 template<int I>
-StepFn pick_step_e(bool energy, bool an, bool pmf_in) {
-	return energy ? pick_step_an<I, true>(an, pmf_in) : pick_step_an<I, false>(an, pmf_in);
+SplitStepFn pick_split_i(bool energy, bool an, int pmf) {
+	if (energy)
+		return an ? pick_split_pmf<I, true, true>(pmf) : pick_split_pmf<I, true, false>(pmf);
+	return an ? pick_split_pmf<I, false, true>(pmf) : pick_split_pmf<I, false, false>(pmf);
 }
-// The fused step kernel for an integrator, energy step, analytical terms and whether
-// the position-dependent force comes precomputed.
-StepFn pick_step(bool bd, bool energy, bool an, bool pmf_in) {
-	return bd ? pick_step_e<MARSMD_INTEGRATOR_BROWNIAN>(energy, an, pmf_in)
-			  : pick_step_e<MARSMD_INTEGRATOR_LANGEVIN>(energy, an, pmf_in);
+SplitStepFn pick_split(bool bd, bool energy, bool an, int pmf) {
+	return bd ? pick_split_i<MARSMD_INTEGRATOR_BROWNIAN>(energy, an, pmf)
+			  : pick_split_i<MARSMD_INTEGRATOR_LANGEVIN>(energy, an, pmf);
+}
+using StepFn = decltype(&k_step<MARSMD_INTEGRATOR_BROWNIAN, false, false, kPmfNone>);
+template<int I, bool E, bool A>
+StepFn pick_step_pmf(int pmf) {
+	return pmf == kPmfGiven		? k_step<I, E, A, kPmfGiven>
+		   : pmf == kPmfCubic	? k_step<I, E, A, kPmfCubic>
+		   : pmf == kPmfLinear	? k_step<I, E, A, kPmfLinear>
+								: k_step<I, E, A, kPmfNone>;
+}
+template<int I>
+StepFn pick_step_i(bool energy, bool an, int pmf) {
+	if (energy)
+		return an ? pick_step_pmf<I, true, true>(pmf) : pick_step_pmf<I, true, false>(pmf);
+	return an ? pick_step_pmf<I, false, true>(pmf) : pick_step_pmf<I, false, false>(pmf);
+}
+// The fused step kernel for an integrator, energy step, analytical terms and the source
+// of the position-dependent force.
+StepFn pick_step(bool bd, bool energy, bool an, int pmf) {
+	return bd ? pick_step_i<MARSMD_INTEGRATOR_BROWNIAN>(energy, an, pmf)
+			  : pick_step_i<MARSMD_INTEGRATOR_LANGEVIN>(energy, an, pmf);
 }
 
 // Permute slot-indexed state into the new sorted order:
@@ -575,7 +712,17 @@ uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 
 struct PatchImpl::Tables {
 	NbTables nb{};
-	DevArray<float> nb_knots;
+	// the step kernels' constants in device memory (one upload): the parameters, which as
+	// kernel arguments were 3.4 KB copied and read back by every workgroup of every launch,
+	// and the nonbonded knots
+	struct Consts {
+		alignas(16) NbTables nb;
+		alignas(16) marsmd_particle_types types;
+	};
+	DevArray<uint8_t> consts;
+	const NbTables* nb_dev() const { return &reinterpret_cast<const Consts*>(consts.data())->nb; }
+	const marsmd_particle_types* types_dev() const { return &reinterpret_cast<const Consts*>(consts.data())->types; }
+	const float* nb_knots() const { return reinterpret_cast<const float*>(consts.data() + sizeof(Consts)); }
 	std::vector<marsmd_table> bond_h, angle_h, dihedral_h;
 	DevArray<float> bond_knots, angle_knots, dihedral_knots;
 	DevArray<marsmd_table> bond_dev, angle_dev, dihedral_dev;
@@ -620,9 +767,13 @@ PatchImpl::PatchImpl(const marsmd_patch_desc& d) : tables(new Tables) {
 	}
 	T.total_knots = int(knots.size());
 	T.lds = T.total_knots <= kLdsKnots ? 1 : 0;
-	tables->nb_knots.resize(std::max<uint64_t>(knots.size(), 1));
+	std::vector<uint8_t> consts(sizeof(Tables::Consts) + 4 * std::max<size_t>(knots.size(), 1), 0);
+	const Tables::Consts head{T, types};
+	std::memcpy(consts.data(), &head, sizeof(head));
 	if (!knots.empty())
-		MMD_HIP(hipMemcpy(tables->nb_knots.data(), knots.data(), knots.size() * 4, hipMemcpyHostToDevice));
+		std::memcpy(consts.data() + sizeof(head), knots.data(), 4 * knots.size());
+	tables->consts.resize(consts.size());
+	MMD_HIP(hipMemcpy(tables->consts.data(), consts.data(), consts.size(), hipMemcpyHostToDevice));
 	auto upload_tables = [&](int num, const marsmd_table* src, std::vector<marsmd_table>& host, DevArray<float>& kd,
 							 DevArray<marsmd_table>& td) {
 		std::vector<float> kn;
@@ -943,15 +1094,23 @@ unsigned PatchImpl::lds_bytes() const {
 	return tables->nb.lds ? unsigned(std::max(tables->nb.total_knots, 2)) * 4u : 0u;
 }
 
-// Workgroups for a persistent launch over the 256-slot tiles: as many as are resident
-// at once (occupancy x CUs), a multiple of 8 (one share per XCD), at most the tiles.
-unsigned PatchImpl::persistent_grid(const void* kernel, uint64_t nn) {
-	const uint64_t tiles = (nn + kBlock - 1) / kBlock;
-	const unsigned lds = lds_bytes();
+// Tiles, block and dynamic LDS of the step kernel.
+PatchImpl::StepShape PatchImpl::step_shape(uint32_t split, int sampled) const {
+	if (split == 0)
+		return StepShape{(n + kBlock - 1) / kBlock, kBlock, lds_bytes(), 0};
+	const uint64_t per = uint64_t(kSplitBlock) >> split;
+	const uint32_t words = (lds_bytes() / 4u + 3u) & ~3u;
+	// the knots, then the handed-over forces of two tiles (and their grid forces)
+	return StepShape{(n + per - 1) / per, kSplitBlock, 4u * words + (sampled == kPmfCubic ? 64u : 32u) * unsigned(per), words};
+}
+
+// Workgroups for a persistent launch over `tiles` tiles: as many as are resident at once
+// (occupancy x CUs), a multiple of 8 (one share per XCD), at most the tiles.
+unsigned PatchImpl::persistent_grid(const void* kernel, uint64_t tiles, int block, unsigned lds) {
 	auto it = occupancy.find(kernel);
 	if (it == occupancy.end() || it->second.first != lds) {
 		int occ = 0;
-		MMD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, kBlock, lds));
+		MMD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, block, lds));
 		it = occupancy.insert_or_assign(kernel, std::make_pair(lds, std::max(occ, 1))).first;
 	}
 	if (num_cus == 0) {
@@ -977,9 +1136,18 @@ void PatchImpl::calculate_nonbonded(float pairlist_cutoff, float cutoff, uint64_
 	interpolation = interp;
 	rebuild_policy(pairlist_cutoff, cutoff, step, period, s);
 	const float cut_d = cutoff_threshold(cutoff > 0.0f ? cutoff * cutoff : 0.0f);
-	auto kern = (tables->nb.enabled & kAnalyticTerms) ? k_nb_forces<true> : k_nb_forces<false>;
-	kern<<<grid_for(n, kBlock), kBlock, lds_bytes(), s>>>(pos[cur].data(), n, pl->list(), tables->nb,
-														  tables->nb_knots.data(), make_devbox(box), cut_d,
+	const bool an = (tables->nb.enabled & kAnalyticTerms) != 0;
+	if (const uint32_t split = row_split(n, pl->max_neighbors, pl->nbr_entries); split > 0) {
+		auto kern = an ? k_nb_forces_split<true> : k_nb_forces_split<false>;
+		kern<<<grid_for(n << split, kSplitBlock), kSplitBlock, lds_bytes(), s>>>(
+			pos[cur].data(), n, pl->list(), tables->nb_dev(), tables->nb_knots(), make_devbox(box), cut_d,
+			energy ? 1 : 0, force.data(), split);
+		MMD_LAUNCH_CHECK();
+		return;
+	}
+	auto kern = an ? k_nb_forces<true> : k_nb_forces<false>;
+	kern<<<grid_for(n, kBlock), kBlock, lds_bytes(), s>>>(pos[cur].data(), n, pl->list(), tables->nb_dev(),
+														  tables->nb_knots(), make_devbox(box), cut_d,
 														  energy ? 1 : 0, force.data());
 	MMD_LAUNCH_CHECK();
 }
@@ -1235,10 +1403,17 @@ void PatchImpl::run(const marsmd_run_params& P, uint64_t first_step, uint64_t nu
 		float4* pnext = pos[1 - cur].data();
 		const bool bd = P.integrator == MARSMD_INTEGRATOR_BROWNIAN;
 		const bool an = (tables->nb.enabled & kAnalyticTerms) != 0;
-		// with grids, the position-dependent force may come from its own kernel
-		const bool pmf_in = split_pmf && num_grids > 0;
-		const StepFn kern = pick_step(bd, energy, an, pmf_in);
-		const unsigned grid = persistent_grid(reinterpret_cast<const void*>(kern), n);
+		const uint32_t split = row_split(n, pl->max_neighbors, pl->nbr_entries);
+		// with grids, the position-dependent force may come from its own kernel (the split
+		// rows' step samples it itself: the same bits)
+		const bool pmf_in = split_pmf && num_grids > 0 && split == 0;
+		const int sampled = num_grids == 0 ? kPmfNone : P.interpolation == MARSMD_INTERP_LINEAR ? kPmfLinear : kPmfCubic;
+		const StepFn kern = pick_step(bd, energy, an, pmf_in ? kPmfGiven : sampled);
+		const SplitStepFn kern_split = pick_split(bd, energy, an, sampled);
+		const StepShape shape = step_shape(split, sampled);
+		const unsigned grid = persistent_grid(split > 0 ? reinterpret_cast<const void*>(kern_split)
+														: reinterpret_cast<const void*>(kern),
+											  shape.tiles, shape.block, shape.lds);
 		prepare_prune(P.cutoff, P.pairlist_cutoff, s);
 		PruneView PR{};
 		if (prune_valid) {
@@ -1270,9 +1445,16 @@ void PatchImpl::run(const marsmd_run_params& P, uint64_t first_step, uint64_t nu
 															   pmf_buf.data());
 			MMD_LAUNCH_CHECK();
 		}
-		kern<<<grid, kBlock, lds_bytes(), s>>>(pos[cur].data(), pnext, mom.data(), force.data(), n, pl->list(),
-											   tables->nb, tables->nb_knots.data(), types, grids_dev.data(), S,
-											   has_bonded, store, pmf_in ? pmf_buf.data() : nullptr, PR);
+		if (split > 0)
+			kern_split<<<grid, kSplitBlock, shape.lds, s>>>(pos[cur].data(), pnext, mom.data(), force.data(), n, pl->list(),
+													  tables->nb_dev(), tables->nb_knots(), shape.knot_words,
+													  tables->types_dev(), grids_dev.data(), S, has_bonded, store,
+													  PR, split);
+		else
+			kern<<<grid, kBlock, shape.lds, s>>>(pos[cur].data(), pnext, mom.data(), force.data(), n, pl->list(),
+										   tables->nb_dev(), tables->nb_knots(), tables->types_dev(),
+										   grids_dev.data(), S, has_bonded, store,
+										   pmf_in ? pmf_buf.data() : nullptr, PR);
 		if (timing) {
 			MMD_HIP(hipEventRecord(timing_events[timing_used + 1], s));
 			timing_used += 2;
@@ -1354,16 +1536,20 @@ void PatchImpl::autotune(const marsmd_run_params& P, uint64_t first_step, uint64
 		double ms = 1e300;
 	};
 	std::vector<Cand> cands;
+	const int sampled = num_grids == 0 ? kPmfNone : P.interpolation == MARSMD_INTERP_LINEAR ? kPmfLinear : kPmfCubic;
+	const uint32_t split = pl->built ? row_split(n, pl->max_neighbors, pl->nbr_entries) : 0u;
 	for (bool sp : {false, true}) {
-		if (sp && num_grids == 0)
+		if (sp && (num_grids == 0 || split > 0)) // (split rows sample the grids themselves)
 			continue;
 		// each step kernel's own occupancy (the split one holds fewer registers), then less
-		const StepFn probe = pick_step(bd, false, an, sp);
+		const void* probe = split > 0 ? reinterpret_cast<const void*>(pick_split(bd, false, an, sampled))
+									  : reinterpret_cast<const void*>(pick_step(bd, false, an, sp ? kPmfGiven : sampled));
 		const int saved = blocks_per_cu;
 		blocks_per_cu = 0;
-		(void)persistent_grid(reinterpret_cast<const void*>(probe), std::max<uint64_t>(n, 1));
+		const StepShape shape = step_shape(split, sampled);
+		(void)persistent_grid(probe, shape.tiles, shape.block, shape.lds);
 		blocks_per_cu = saved;
-		const int occ = occupancy[reinterpret_cast<const void*>(probe)].second;
+		const int occ = occupancy[probe].second;
 		std::vector<int> per_cu = {occ};
 		for (int v : {occ - 1, occ / 2})
 			if (v >= 1 && std::find(per_cu.begin(), per_cu.end(), v) == per_cu.end())

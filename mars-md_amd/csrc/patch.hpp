@@ -127,7 +127,13 @@ struct PatchImpl {
 	uint64_t num_shares() const;
 	void build_share_index(hipStream_t s);
 	unsigned lds_bytes() const;
-	unsigned persistent_grid(const void* kernel, uint64_t n);
+	struct StepShape {
+		uint64_t tiles;
+		int block;
+		unsigned lds, knot_words;
+	};
+	StepShape step_shape(uint32_t split, int sampled) const;
+	unsigned persistent_grid(const void* kernel, uint64_t tiles, int block, unsigned lds);
 };
 
 } // namespace mmd
