@@ -27,6 +27,7 @@
 
 #include "homewalk.hpp"
 #include "nbforce.hpp"
+#include "segsort.hpp"
 #include "step.hpp"
 
 #include <algorithm>
@@ -103,27 +104,10 @@ __global__ void k_b_rep_keys(const uint32_t* __restrict__ vals_s, uint64_t total
 }
 
 // The same order in one launch when every replica has at most kSegSortMax particles:
-// a stable LSD radix sort of each replica's Morton keys (three 10-bit digits) by one
-// workgroup of kSegWaves waves, the replica resident in LDS. The encode leaves replica
+// each replica's Morton keys sorted by one workgroup (seg_sort). The encode leaves replica
 // r's entries at [slot0, slot0 + n) in canonical order, so sorting each such range
 // stably by key gives the order of the global stable sort by key followed by the stable
-// sort by replica. Wave w takes the run [w C, w C + C) of the range (C = ceil(n /
-// kSegWaves)) in batches of 64 held in registers, counts its digits, and after the
-// block's exclusive scan (digit-major, wave-minor) scatters each batch in order: the
-// entries of one batch with one digit rank by lane (their peer mask from 10 ballots) and
-// the lowest of them moves the wave's offset for that digit on. Equal digits therefore
-// keep wave, batch and lane order. A pass reads the whole range into registers before
-// its first barrier and scatters it back after the scan, so one LDS copy suffices; the
-// entries carry their canonical position (16 bits), and the old slots are read once,
-// in order, at the end. Counts and offsets stay below 2^16, so two waves share a
-// histogram word (wave 2k in the low half, 2k + 1 in the high half).
-constexpr int kSegWaves = 16;
-constexpr int kSegThreads = kSegWaves * 64;
-constexpr int kSegPerLane = 20;
-constexpr uint32_t kSegSortMax = uint32_t(kSegThreads) * kSegPerLane; // 20480: 159.8 KB of LDS
-constexpr int kSegStride = kSegWaves / 2 + 1;                          // words per digit, padded
-constexpr uint32_t kSegSpare = 1024u * kSegStride;                      // the bin of idle lanes
-
+// sort by replica. The old slots are read once, in order, at the end.
 __global__ __launch_bounds__(kSegThreads) void k_b_seg_sort(const RepGeom* __restrict__ geom,
 															const uint32_t* __restrict__ order,
 															const uint32_t* __restrict__ keys,
@@ -131,116 +115,11 @@ __global__ __launch_bounds__(kSegThreads) void k_b_seg_sort(const RepGeom* __res
 															uint32_t* __restrict__ out_vals) {
 	__shared__ uint32_t s_key[kSegSortMax];
 	__shared__ uint16_t s_pos[kSegSortMax];
-	__shared__ uint32_t hist[1024 * kSegStride + 1];
+	__shared__ uint32_t hist[kSegHistWords];
 	__shared__ uint32_t wsum[kSegWaves];
 	const uint32_t r = order[blockIdx.x];
 	const uint32_t base = geom[r].slot0, n = geom[r].n;
-	const int wv = int(threadIdx.x >> 6), lane = int(threadIdx.x & 63);
-	const uint32_t half = 16u * uint32_t(wv & 1), col = uint32_t(wv >> 1);
-	const uint32_t C = (n + kSegWaves - 1) / kSegWaves; // <= 64 * kSegPerLane
-	const uint32_t w0_ = min(n, uint32_t(wv) * C), w1_ = min(n, w0_ + C);
-	const uint64_t lt = (uint64_t(1) << lane) - 1;
-	uint32_t key[kSegPerLane], at[kSegPerLane];
-	if (w1_ > w0_) { // the first pass's entries, from global memory (reads clamped into the run)
-		const uint32_t nb = (w1_ - w0_ + 63u) / 64u;
-#pragma unroll
-		for (int j = 0; j < kSegPerLane; ++j) {
-			if (uint32_t(j) < nb) { // wave-uniform
-				const uint32_t e = min(w0_ + uint32_t(j) * 64u + uint32_t(lane), w1_ - 1u);
-				key[j] = keys[base + e];
-				at[j] = e;
-			}
-		}
-	}
-#pragma unroll 1
-	for (int pass = 0; pass < 3; ++pass) {
-		const int shift = 10 * pass;
-		// the run's bounds, opaque to the compiler each pass: otherwise it hoists every
-		// batch's address and mask out of the pass loop (64 SGPRs and 32 VGPRs)
-		uint32_t w0 = w0_, w1 = w1_;
-		asm volatile("" : "+v"(w0), "+v"(w1));
-		const uint32_t nb = (w1 - w0 + 63u) / 64u; // batches of this wave
-		for (uint32_t i = threadIdx.x; i <= kSegSpare; i += kSegThreads)
-			hist[i] = 0u;
-		__syncthreads();
-		if (w1 > w0) { // reads clamped into the run, a lane past its end counted in the spare bin
-			if (pass > 0) {
-#pragma unroll
-				for (int j = 0; j < kSegPerLane; ++j) {
-					if (uint32_t(j) < nb) { // wave-uniform
-						const uint32_t e = min(w0 + uint32_t(j) * 64u + uint32_t(lane), w1 - 1u);
-						key[j] = s_key[e];
-						at[j] = s_pos[e];
-					}
-				}
-			}
-#pragma unroll
-			for (int j = 0; j < kSegPerLane; ++j) {
-				if (uint32_t(j) < nb) {
-					const bool live = w0 + uint32_t(j) * 64u + uint32_t(lane) < w1;
-					atomicAdd(&hist[live ? ((key[j] >> shift) & 1023u) * kSegStride + col : kSegSpare],
-							  live ? 1u << half : 1u);
-				}
-			}
-		}
-		__syncthreads();
-		{ // thread t owns digit t: its waves' counts become their first destinations
-			const uint32_t row = threadIdx.x * kSegStride;
-			uint32_t c[kSegWaves / 2], s = 0;
-#pragma unroll
-			for (int k = 0; k < kSegWaves / 2; ++k) {
-				c[k] = hist[row + uint32_t(k)];
-				s += (c[k] & 0xFFFFu) + (c[k] >> 16);
-			}
-			const uint32_t incl = wave_inclusive_scan(s);
-			if (lane == 63)
-				wsum[wv] = incl;
-			__syncthreads();
-			uint32_t run = incl - s;
-			for (int w = 0; w < wv; ++w)
-				run += wsum[w];
-#pragma unroll
-			for (int k = 0; k < kSegWaves / 2; ++k) {
-				const uint32_t lo = run;
-				run += c[k] & 0xFFFFu;
-				hist[row + uint32_t(k)] = lo | (run << 16);
-				run += c[k] >> 16;
-			}
-		}
-		__syncthreads();
-#pragma unroll
-		for (int j = 0; j < kSegPerLane; ++j) {
-			if (uint32_t(j) >= nb) // wave-uniform
-				continue;
-			const bool live = w0 + uint32_t(j) * 64u + uint32_t(lane) < w1;
-			const uint32_t d = (key[j] >> shift) & 1023u;
-			// the peer mask on 32-bit halves, sx all ones where the lane's bit is set: the
-			// lanes that agree on every bit stay (4 VALU a bit instead of 10 on 64-bit masks)
-			const uint64_t lv = __ballot(live);
-			uint32_t plo = uint32_t(lv), phi = uint32_t(lv >> 32);
-#pragma unroll
-			for (int b = 0; b < 10; ++b) {
-				const int32_t sx = int32_t(d << (31 - b)) >> 31;
-				const uint64_t ones = __ballot(sx != 0);
-				plo &= ~(uint32_t(ones) ^ uint32_t(sx));
-				phi &= ~(uint32_t(ones >> 32) ^ uint32_t(sx));
-			}
-			const uint64_t peers = uint64_t(plo) | (uint64_t(phi) << 32);
-			if (live) {
-				// the other half of the word is the sibling wave's: it moves by atomic adds
-				uint32_t* h = &hist[d * kSegStride + col];
-				const uint32_t first = (*h >> half) & 0xFFFFu;
-				const uint32_t rank = uint32_t(__popcll(peers & lt));
-				if (rank == 0u)
-					atomicAdd(h, uint32_t(__popcll(peers)) << half);
-				const uint32_t dst = first + rank;
-				if (pass < 2)
-					s_key[dst] = key[j];
-				s_pos[dst] = uint16_t(at[j]);
-			}
-		}
-		__syncthreads();
-	}
+	seg_sort<false, kSegPerLane>(keys + base, n, 30, s_key, s_pos, hist, wsum);
 #pragma unroll
 	for (int k = 0; k < kSegPerLane; ++k) { // every load in flight at once
 		const uint32_t i = threadIdx.x + uint32_t(k) * kSegThreads;

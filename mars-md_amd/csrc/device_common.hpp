@@ -748,4 +748,19 @@ __device__ __forceinline__ float atomic_add_f32(float* p, float v) {
 	return unsafeAtomicAdd(p, v);
 }
 
+// Wave-wide scans and reductions on the DPP crossbar: row shifts within 16 lanes, then
+// the row broadcasts (lane 15 of rows 0 and 2 into the next row, lane 31 into rows 2 and 3).
+template<int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_add(uint32_t v) {
+	return v + uint32_t(__builtin_amdgcn_update_dpp(0, int(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
+	v = dpp_add<0x111, 0xf>(v); // row_shr:1
+	v = dpp_add<0x112, 0xf>(v);
+	v = dpp_add<0x114, 0xf>(v);
+	v = dpp_add<0x118, 0xf>(v);
+	v = dpp_add<0x142, 0xa>(v); // row_bcast:15 into rows 1 and 3
+	return dpp_add<0x143, 0xc>(v); // row_bcast:31 into rows 2 and 3
+}
+
 } // namespace mmd

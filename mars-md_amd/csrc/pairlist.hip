@@ -36,8 +36,11 @@ __device__ __forceinline__ uint32_t fbits(float f) { return __float_as_uint(f); 
 
 __global__ void k_encode(const float4* __restrict__ pos, uint64_t n, float3 bmin, float3 bmax,
 						 bool canon_from_meta, uint32_t* __restrict__ keys,
-						 uint32_t* __restrict__ vals, uint32_t* __restrict__ outside) {
+						 uint32_t* __restrict__ vals, uint32_t* __restrict__ outside,
+						 uint32_t* __restrict__ next_outside) {
 	const uint64_t s = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (s == 0)
+		*next_outside = 0u;
 	if (s >= n)
 		return;
 	const float4 p = pos[s];
@@ -417,18 +420,37 @@ __global__ __launch_bounds__(256) void k_tile_rows(const uint32_t* __restrict__ 
 		rows[w] = 64u * ((m + 3u) & ~3u);
 }
 
-// Largest count and total entries: grid-stride partials reduced in the workgroup, then
-// one atomic pair per workgroup (launched with a few hundred workgroups).
-// The sorter's flag word is copied to max_count[1], so that one read-back of four words
-// returns the three.
-__global__ __launch_bounds__(256) void k_count_stats(const uint32_t* __restrict__ counts, uint64_t n,
-													 unsigned long long* __restrict__ total,
-													 uint32_t* __restrict__ max_count,
-													 const uint32_t* __restrict__ flag) {
-	if (blockIdx.x == 0 && threadIdx.x == 0)
-		max_count[1] = flag[0];
-	__shared__ uint32_t wmax[4];
-	__shared__ unsigned long long wsum[4];
+// Largest count and total entries of the rows: grid-stride partials reduced in the
+// workgroup, then three atomics per workgroup; the last of them (`acc.ticket`) writes
+// {max, the sorter's flag word, total (8 bytes)} to `out`, the host's pinned words, and
+// leaves the accumulators at zero for the next call. The atomics on one line, about 10 ns
+// each, bound this: 64 workgroups of 16 waves keep them few.
+struct StatWords { // persistent, zero between calls
+	unsigned long long total;
+	uint32_t max_count, ticket;
+	uint32_t disp, disp_ticket;
+};
+constexpr unsigned kStatBlock = 1024;
+
+template<class T, class OP>
+__device__ __forceinline__ T block_reduce(T v, T* lds, OP op) {
+	for (int o = 32; o > 0; o >>= 1)
+		v = op(v, T(__shfl_xor(v, o, 64)));
+	if ((threadIdx.x & 63) == 0)
+		lds[threadIdx.x >> 6] = v;
+	__syncthreads();
+	v = lds[0];
+	for (unsigned k = 1; k < (blockDim.x >> 6); ++k)
+		v = op(v, lds[k]);
+	return v;
+}
+
+__global__ __launch_bounds__(kStatBlock) void k_count_stats(const uint32_t* __restrict__ counts, uint64_t n,
+															StatWords* __restrict__ acc,
+															const uint32_t* __restrict__ flag,
+															uint32_t* __restrict__ out) {
+	__shared__ uint32_t wmax[kStatBlock / 64];
+	__shared__ unsigned long long wsum[kStatBlock / 64];
 	uint32_t m = 0;
 	unsigned long long sum = 0;
 	const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
@@ -441,33 +463,30 @@ __global__ __launch_bounds__(256) void k_count_stats(const uint32_t* __restrict_
 		m = max(max(m, c0), max(c1, max(c2, c3)));
 		sum += (unsigned long long)c0 + c1 + c2 + c3;
 	}
-	for (int o = 32; o > 0; o >>= 1) {
-		m = max(m, uint32_t(__shfl_xor(int(m), o, 64)));
-		sum += __shfl_xor(sum, o, 64);
-	}
-	const int w = threadIdx.x >> 6;
-	if ((threadIdx.x & 63) == 0) {
-		wmax[w] = m;
-		wsum[w] = sum;
-	}
-	__syncthreads();
+	m = block_reduce(m, wmax, [](uint32_t a, uint32_t b) { return max(a, b); });
+	sum = block_reduce(sum, wsum, [](unsigned long long a, unsigned long long b) { return a + b; });
 	if (threadIdx.x == 0) {
-		uint32_t bm = 0;
-		unsigned long long bs = 0;
-		for (int k = 0; k < int(blockDim.x >> 6); ++k) {
-			bm = max(bm, wmax[k]);
-			bs += wsum[k];
+		atomicAdd(&acc->total, sum);
+		atomicMax(&acc->max_count, m);
+		__threadfence(); // both before the ticket
+		if (atomicAdd(&acc->ticket, 1u) == gridDim.x - 1u) {
+			out[0] = atomicExch(&acc->max_count, 0u);
+			out[1] = flag[0];
+			*reinterpret_cast<unsigned long long*>(out + 2) = atomicExch(&acc->total, 0ull);
+			acc->ticket = 0u;
 		}
-		atomicAdd(total, bs);
-		atomicMax(max_count, bm);
 	}
 }
 
-// tile_base[w] = w * row for w in [0, tiles] (rows of `row` entries per tile).
-__global__ void k_uniform_tile_base(uint32_t* __restrict__ tile_base, uint64_t tiles, uint32_t row) {
-	const uint64_t w = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (w <= tiles)
-		tile_base[w] = uint32_t(w * row);
+// Ready for a walk: the cell tables cleared and the uniform rows' bases
+// (tile_base[w] = w * row for w in [0, tiles], rows of `row` entries per tile).
+__global__ void k_walk_setup(uint2* __restrict__ cells, uint64_t num_cells, uint32_t* __restrict__ tile_base,
+							 uint64_t tiles, uint32_t row) {
+	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (i < num_cells)
+		cells[i] = make_uint2(0u, 0u);
+	if (i <= tiles)
+		tile_base[i] = uint32_t(i * row);
 }
 
 __global__ void k_half_counts(NbrList L, uint64_t n, uint32_t* __restrict__ half) {
@@ -500,9 +519,16 @@ __global__ void k_write_pairs(NbrList L, const uint32_t* __restrict__ half_off, 
 	}
 }
 
-__global__ __launch_bounds__(256) void k_max_disp(const float4* __restrict__ cur, const float4* __restrict__ snap,
-												  const uint32_t* __restrict__ sorted_of_slot, uint64_t n,
-												  float3 plen, uint32_t* __restrict__ out_bits) {
+// The largest squared minimum-image displacement between cur and snap (as float bits) to
+// `out` (device or pinned host memory). Bound by the 32 bytes read a particle and the
+// atomics, one pair per workgroup as in k_count_stats: 12.5 us at 10^6 particles, 4.3 at
+// 10^4 (52 and 13 us with one atomic per wave of 1024 workgroups).
+__global__ __launch_bounds__(kStatBlock) void k_max_disp(const float4* __restrict__ cur,
+														 const float4* __restrict__ snap,
+														 const uint32_t* __restrict__ sorted_of_slot, uint64_t n,
+														 float3 plen, StatWords* __restrict__ acc,
+														 uint32_t* __restrict__ out) {
+	__shared__ float wmax[kStatBlock / 64];
 	float m = 0.0f;
 	for (uint64_t s = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; s < n; s += uint64_t(gridDim.x) * blockDim.x) {
 		const float4 a = cur[s];
@@ -523,11 +549,17 @@ __global__ __launch_bounds__(256) void k_max_disp(const float4* __restrict__ cur
 		const float d2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
 		m = fmaxf(m, d2);
 	}
-	for (int o = 32; o > 0; o >>= 1)
-		m = fmaxf(m, __shfl_xor(m, o, 64));
-	if ((threadIdx.x & 63) == 0)
-		atomicMax(out_bits, __float_as_uint(m)); // non-negative floats order as uints
+	m = block_reduce(m, wmax, [](float a, float b) { return fmaxf(a, b); });
+	if (threadIdx.x == 0) {
+		atomicMax(&acc->disp, __float_as_uint(m)); // non-negative floats order as uints
+		__threadfence(); // before the ticket
+		if (atomicAdd(&acc->disp_ticket, 1u) == gridDim.x - 1u) {
+			*out = atomicExch(&acc->disp, 0u);
+			acc->disp_ticket = 0u;
+		}
+	}
 }
+unsigned disp_grid(uint64_t n) { return std::min<unsigned>(grid_for(n, kStatBlock), 256); }
 
 } // namespace
 
@@ -572,7 +604,7 @@ CellGrid select_cell_grid(float cutoff, uint64_t n, const float extent_f[3], uin
 	return g;
 }
 
-ZSort::ZSort(uint64_t max_n) : max_particles(max_n) { outside_flag.resize(1); }
+ZSort::ZSort(uint64_t max_n) : max_particles(max_n) {}
 
 void ZSort::ensure(uint64_t nn) {
 	if (nn > max_particles)
@@ -587,25 +619,32 @@ void ZSort::ensure(uint64_t nn) {
 }
 
 void ZSort::sort(const float4* pos, uint64_t nn, const float bmin[3], const float bmax[3],
-				 const float* domain_dev, bool canon_from_meta, hipStream_t s, bool presorted) {
+				 const float* domain_dev, bool canon_from_meta, hipStream_t s, bool presorted,
+				 bool with_inverse) {
 	(void)domain_dev;
 	ensure(nn);
 	n = nn;
 	if (nn == 0)
 		return;
-	fill_u32(outside_flag.data(), 0u, 1, s);
+	if (!outside_flag.data()) {
+		outside_flag.resize(2);
+		fill_u32(outside_flag.data(), 0u, 2, s);
+	}
+	flag_now ^= 1u;
 	k_encode<<<grid_for(nn, 256), 256, 0, s>>>(pos, nn, make_float3(bmin[0], bmin[1], bmin[2]),
 											   make_float3(bmax[0], bmax[1], bmax[2]), canon_from_meta,
-											   keys_unsorted.data(), vals_unsorted.data(), outside_flag.data());
+											   keys_unsorted.data(), vals_unsorted.data(), flag(), outside_flag.data() + (flag_now ^ 1u));
 	MMD_LAUNCH_CHECK();
 	if (presorted) {
 		k_presorted<<<grid_for(nn, 256), 256, 0, s>>>(keys_unsorted.data(), nn, codes.data(), sorted_idx.data(),
-													  inverse.data(), outside_flag.data());
+													  inverse.data(), flag());
 		MMD_LAUNCH_CHECK();
 		return;
 	}
 	radix_sort_pairs(keys_unsorted.data(), vals_unsorted.data(), codes.data(), sorted_idx.data(), nn, 30,
 					 scratch.data(), scratch.count, s);
+	if (!with_inverse)
+		return;
 	k_inverse<<<grid_for(nn, 256), 256, 0, s>>>(sorted_idx.data(), nn, inverse.data());
 	MMD_LAUNCH_CHECK();
 }
@@ -637,7 +676,6 @@ void ZSort::remap_indices(int32_t* idx, uint64_t count, hipStream_t s) const {
 PairlistImpl::PairlistImpl(uint64_t max_particles_, uint64_t max_pairs_ceiling_)
 	: max_particles(max_particles_), max_pairs_ceiling(max_pairs_ceiling_), sorter(max_particles_) {
 	ref_max_pairs = std::min<uint64_t>(max_pairs_ceiling, std::max<uint64_t>(max_particles, 1));
-	dev_scalars.resize(8);
 }
 
 void PairlistImpl::ensure(uint64_t nn) {
@@ -732,13 +770,20 @@ void PairlistImpl::walk(bool fill, bool use_ref, hipStream_t s) {
 	MMD_LAUNCH_CHECK();
 }
 
-// Largest count, the sorter's flag word and total entries of `counts` into dev_scalars
-// [2], [3] and [4..5].
-void PairlistImpl::count_stats(uint64_t nn, hipStream_t s) {
-	fill_u32(dev_scalars.data() + 2, 0u, 4, s);
-	k_count_stats<<<std::min<unsigned>(grid_for(nn, 256), 240), 256, 0, s>>>(
-		counts.data(), nn, reinterpret_cast<unsigned long long*>(dev_scalars.data() + 4), dev_scalars.data() + 2,
-		sorter.outside_flag.data());
+static StatWords* stat_words(DevArray<uint32_t>& dev_scalars, hipStream_t s) {
+	constexpr uint64_t kWords = sizeof(StatWords) / 4;
+	if (!dev_scalars.data()) {
+		dev_scalars.resize(8 + kWords);
+		fill_u32(dev_scalars.data() + 8, 0u, kWords, s);
+	}
+	return reinterpret_cast<StatWords*>(dev_scalars.data() + 8);
+}
+
+// Largest count, the sorter's flag word and total entries of `counts` (8 bytes) into
+// out[0], [1] and [2..3] of the pinned words.
+void PairlistImpl::count_stats(uint64_t nn, uint32_t* out, hipStream_t s) {
+	k_count_stats<<<std::min<unsigned>(grid_for(nn, kStatBlock), 64), kStatBlock, 0, s>>>(
+		counts.data(), nn, stat_words(dev_scalars, s), sorter.flag(), out);
 	MMD_LAUNCH_CHECK();
 }
 
@@ -801,7 +846,14 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 	walk_cells.resize(num_fine + num_home);
 	uint2* fine = walk_cells.data();
 	uint2* home = fine + num_fine;
-	fill_u32(reinterpret_cast<uint32_t*>(fine), 0u, 2 * (num_fine + num_home), s);
+	if (home_cap == 0) {
+		// first build: the mean count of a uniform system, with room for its fluctuations
+		const double mean = double(n) / volume * 4.0 / 3.0 * 3.141592653589793 * double(cutoff) * cutoff * cutoff;
+		home_cap = uint32_t(std::min(1.6 * mean + 16.0, 4096.0) + 3) & ~3u;
+	}
+	k_walk_setup<<<grid_for(std::max(num_fine + num_home, tiles + 1), 256), 256, 0, s>>>(
+		fine, num_fine + num_home, tile_base.data(), tiles, 64u * home_cap);
+	MMD_LAUNCH_CHECK();
 	k_walk_cells<<<grid_for(n, 256), 256, 0, s>>>(sorter.codes.data(), n, 3 * (10 - mf), 3 * (10 - h), fine, home);
 	MMD_LAUNCH_CHECK();
 	P.fine = fine;
@@ -861,11 +913,6 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 			P.dom_hi[a] = domain_max[a];
 		}
 	}
-	if (home_cap == 0) {
-		// first build: the mean count of a uniform system, with room for its fluctuations
-		const double mean = double(n) / volume * 4.0 / 3.0 * 3.141592653589793 * double(cutoff) * cutoff * cutoff;
-		home_cap = uint32_t(std::min(1.6 * mean + 16.0, 4096.0) + 3) & ~3u;
-	}
 	const unsigned groups = unsigned((P.num_home + kHomeWaves - 1) / kHomeWaves);
 	const unsigned grid = std::max(8u, (groups + 7u) / 8u * 8u);
 	for (int attempt = 0; attempt < 2; ++attempt) {
@@ -875,17 +922,18 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 		if (storage > nbr.count)
 			nbr.resize(storage + storage / 8 + 1024);
 		P.cap = home_cap;
-		k_uniform_tile_base<<<grid_for(tiles + 1, 256), 256, 0, s>>>(tile_base.data(), tiles, 64u * home_cap);
-		MMD_LAUNCH_CHECK();
+		if (attempt > 0) { // larger rows
+			k_walk_setup<<<grid_for(tiles + 1, 256), 256, 0, s>>>(nullptr, 0, tile_base.data(), tiles, 64u * home_cap);
+			MMD_LAUNCH_CHECK();
+		}
 		const int mode = walk_mode(P);
 		const auto kern = mode == kWalkPlain	 ? k_walk_home<kWalkPlain>
 						  : mode == kWalkOwnRows ? k_walk_home<kWalkOwnRows>
 												 : k_walk_home<kWalkGeneral>;
 		kern<<<grid, 256, 0, s>>>(P, counts.data(), nbr.data());
 		MMD_LAUNCH_CHECK();
-		count_stats(n, s);
 		uint32_t* host = readback.ptr; // max count, flag word, total entries (2 words)
-		MMD_HIP(hipMemcpyAsync(host, dev_scalars.data() + 2, 16, hipMemcpyDeviceToHost, s));
+		count_stats(n, host, s);
 		MMD_HIP(hipStreamSynchronize(s));
 		if (host[1] & 2u)
 			raise(MARSMD_ERR_RUNTIME, "pairlist: keys after a reorder were not in order");
@@ -928,6 +976,7 @@ void PairlistImpl::build(const float4* pos, const uint32_t* slot_of_canon, bool 
 	float lo[3], hi[3];
 	if (!all_periodic) {
 		dev_domain.resize(1);
+		(void)stat_words(dev_scalars, s);
 		k_init_bbox<<<1, 64, 0, s>>>(dev_scalars.data());
 		MMD_LAUNCH_CHECK();
 		k_bbox<<<std::min<unsigned>(grid_for(nn, 256), 1024), 256, 0, s>>>(pos, nn, dev_scalars.data());
@@ -961,7 +1010,7 @@ void PairlistImpl::build(const float4* pos, const uint32_t* slot_of_canon, bool 
 	// very keys, so the sort is the identity
 	const bool presorted = presorted_next && all_periodic && canon_from_meta;
 	presorted_next = false;
-	sorter.sort(pos, nn, lo, hi, nullptr, canon_from_meta, s, presorted);
+	sorter.sort(pos, nn, lo, hi, nullptr, canon_from_meta, s, presorted, false); // k_finalize writes the inverse
 	k_finalize<<<grid_for(nn, 256), 256, 0, s>>>(sorter.sorted_idx.data(), nn, pos, slot_of_canon, canon_from_meta,
 												 types, sorter.inverse.data(), spos.data());
 	MMD_LAUNCH_CHECK();
@@ -995,11 +1044,10 @@ void PairlistImpl::build(const float4* pos, const uint32_t* slot_of_canon, bool 
 		const uint64_t tiles = (nn + 63) / 64;
 		k_tile_rows<<<grid_for(nn, 256), 256, 0, s>>>(counts.data(), nn, tile_rows.data());
 		MMD_LAUNCH_CHECK();
-		count_stats(nn, s);
-		exclusive_scan_u32(tile_rows.data(), tile_base.data(), tiles, scan_scratch.data(), s);
 		uint32_t* host = readback.ptr; // storage, then max count, flag word, total entries
+		count_stats(nn, host + 2, s);
+		exclusive_scan_u32(tile_rows.data(), tile_base.data(), tiles, scan_scratch.data(), s);
 		MMD_HIP(hipMemcpyAsync(&host[0], tile_base.data() + tiles, 4, hipMemcpyDeviceToHost, s));
-		MMD_HIP(hipMemcpyAsync(&host[2], dev_scalars.data() + 2, 16, hipMemcpyDeviceToHost, s));
 		MMD_HIP(hipStreamSynchronize(s));
 		host[1] = host[3]; // the flag word, where the checks below read it
 		if (host[1] & 2u)
@@ -1043,15 +1091,13 @@ float PairlistImpl::max_displacement(const float4* pos, const uint32_t* sorted_o
 									 hipStream_t s) {
 	if (nn == 0)
 		return 0.0f;
-	fill_u32(dev_scalars.data() + 1, 0u, 1, s);
 	const float3 plen = make_float3(box.periodic[0] ? box.size[0] : 0.0f, box.periodic[1] ? box.size[1] : 0.0f,
 									box.periodic[2] ? box.size[2] : 0.0f);
-	k_max_disp<<<std::min<unsigned>(grid_for(nn, 256), 1024), 256, 0, s>>>(pos, spos.data(), sorted_of_slot, nn, plen,
-																			 dev_scalars.data() + 1);
+	k_max_disp<<<disp_grid(nn), kStatBlock, 0, s>>>(pos, spos.data(), sorted_of_slot, nn, plen,
+													stat_words(dev_scalars, s), readback.ptr);
 	MMD_LAUNCH_CHECK();
-	uint32_t bits = 0;
-	MMD_HIP(hipMemcpyAsync(&bits, dev_scalars.data() + 1, 4, hipMemcpyDeviceToHost, s));
 	MMD_HIP(hipStreamSynchronize(s));
+	const uint32_t bits = readback.ptr[0];
 	float d2;
 	std::memcpy(&d2, &bits, 4);
 	return std::sqrt(d2);
@@ -1076,16 +1122,18 @@ float ZSort::compute_max_displacement(const float4* pos, uint64_t nn, const floa
 									std::to_string(disp_n));
 	if (nn == 0)
 		return 0.0f;
-	disp_bits.resize(1);
-	fill_u32(disp_bits.data(), 0u, 1, s);
+	constexpr uint64_t kWords = sizeof(StatWords) / 4; // then the result
+	disp_bits.resize(kWords + 1);
+	fill_u32(disp_bits.data(), 0u, kWords, s);
 	const float3 plen = make_float3(box_len && box_len[0] > 0.0f ? box_len[0] : 0.0f,
 									box_len && box_len[1] > 0.0f ? box_len[1] : 0.0f,
 									box_len && box_len[2] > 0.0f ? box_len[2] : 0.0f);
-	k_max_disp<<<std::min<unsigned>(grid_for(nn, 256), 1024), 256, 0, s>>>(pos, disp_ref.data(), nullptr, nn, plen,
-																			 disp_bits.data());
+	k_max_disp<<<disp_grid(nn), kStatBlock, 0, s>>>(pos, disp_ref.data(), nullptr, nn, plen,
+													reinterpret_cast<StatWords*>(disp_bits.data()),
+													disp_bits.data() + kWords);
 	MMD_LAUNCH_CHECK();
 	uint32_t bits = 0;
-	MMD_HIP(hipMemcpyAsync(&bits, disp_bits.data(), 4, hipMemcpyDeviceToHost, s));
+	MMD_HIP(hipMemcpyAsync(&bits, disp_bits.data() + kWords, 4, hipMemcpyDeviceToHost, s));
 	MMD_HIP(hipStreamSynchronize(s));
 	float d2;
 	std::memcpy(&d2, &bits, 4);

@@ -22,7 +22,11 @@ struct ZSort {
 	DevArray<uint32_t> keys_unsorted, vals_unsorted; // canonical-order keys and iota
 	DevArray<uint32_t> codes, sorted_idx, inverse;    // results
 	DevArray<uint8_t> scratch;
-	DevArray<uint32_t> outside_flag; // bit 0: a coordinate was clamped by the encode
+	// bit 0 of flag(): a coordinate was clamped by the encode. Two words in turn: each
+	// encode clears the next one's.
+	DevArray<uint32_t> outside_flag;
+	uint32_t flag_now = 0;
+	uint32_t* flag() const { return outside_flag.data() + flag_now; }
 	explicit ZSort(uint64_t max_n);
 	void ensure(uint64_t n);
 	// Encode positions (slot order) into canonical-order keys and sort them.
@@ -31,10 +35,11 @@ struct ZSort {
 	// when non-null.
 	// presorted: the canonical-order keys are known to be nondecreasing (the particles
 	// were just relabelled by a sort of the same keys), so the stable sort is the
-	// identity and is replaced by a copy that checks the order (bit 1 of outside_flag
-	// when violated).
+	// identity and is replaced by a copy that checks the order (bit 1 of flag()
+	// when violated). with_inverse: false leaves `inverse` to the caller (unless presorted).
 	void sort(const float4* pos, uint64_t n, const float bmin[3], const float bmax[3],
-			  const float* domain_dev, bool canon_from_meta, hipStream_t s, bool presorted = false);
+			  const float* domain_dev, bool canon_from_meta, hipStream_t s, bool presorted = false,
+			  bool with_inverse = true);
 	// ReorderDataKernel<T> (ZOrderKernels.h:48-63).
 	void reorder_data(const void* in, void* out, uint64_t n, uint32_t elem, hipStream_t s) const;
 	// RemapIndicesKernel (ZOrderKernels.h:87-101).
@@ -115,7 +120,7 @@ struct PairlistImpl {
 	float domain_min[3]{}, domain_max[3]{};
 	double last_build_ms = 0.0;
 	uint32_t max_neighbors = 0;
-	// misc device scalars: [1] max displacement^2 bits, [2] max count, [4..5] entries (u64)
+	// device scalars: [0..5] the bounding box, [8..] the reductions' accumulators
 	DevArray<uint32_t> dev_scalars;
 	DevArray<float> dev_domain;
 	DevArray<uint32_t> ref_begin, ref_end, ref_neighbors;
@@ -148,7 +153,7 @@ struct PairlistImpl {
 	void choose_grids(uint64_t n);
 	void walk(bool fill, bool use_ref_grid, hipStream_t s);
 	bool walk_home(hipStream_t s, bool& outside);
-	void count_stats(uint64_t n, hipStream_t s);
+	void count_stats(uint64_t n, uint32_t* out, hipStream_t s);
 	void ensure(uint64_t n);
 };
 

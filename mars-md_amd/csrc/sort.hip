@@ -19,7 +19,10 @@
 // sort is stable. Both kernels issue all 16 row loads of a wave before ranking, so a
 // wave waits on memory once per tile rather than once per row; the scatter stages the
 // ranked tile in LDS and writes it out in digit order.
+// Up to 12288 keys one workgroup sorts in one launch instead (k_rs_one_group).
+#include "device_common.hpp"
 #include "internal.hpp"
+#include "segsort.hpp"
 
 #include <mutex>
 
@@ -272,6 +275,34 @@ __global__ __launch_bounds__(kRsBlock) void k_rs_scatter(const uint32_t* __restr
 	}
 }
 
+// The whole sort of at most kOneGroupMax keys by one workgroup, keys resident in LDS
+// (seg_sort). Bound there by the latency of its LDS passes, the passes above by that of
+// their launches on a nearly idle chip. Both, microseconds a sort: 30-bit keys 48.1 and
+// 12.8 at 500 keys, 58.3 and 21.4 at 5000, 58.7 and 37.1 at 12000, 59.9 and 47.1 at 16000;
+// 32-bit 64.8 and 49.6 at 12000, 64.8 and 63.0 at 16000; 10-bit 20.4 and 17.3 at 12000,
+// 21.2 and 22.0 at 16000. The line lies where one workgroup is still ahead at every width.
+constexpr uint64_t kOneGroupMax = 12288;
+static_assert(kOneGroupMax <= kSegSortMax, "one workgroup's keys");
+__global__ __launch_bounds__(kSegThreads) void k_rs_one_group(const uint32_t* __restrict__ keys,
+															  const uint32_t* __restrict__ vals,
+															  uint32_t* __restrict__ keys_out,
+															  uint32_t* __restrict__ vals_out, uint32_t n,
+															  int key_bits) {
+	__shared__ uint32_t s_key[kOneGroupMax];
+	__shared__ uint16_t s_pos[kOneGroupMax];
+	__shared__ uint32_t hist[kSegHistWords];
+	__shared__ uint32_t wsum[kSegWaves];
+	seg_sort<true, int(kOneGroupMax / kSegThreads)>(keys, n, key_bits, s_key, s_pos, hist, wsum);
+#pragma unroll
+	for (int k = 0; k < int(kOneGroupMax / kSegThreads); ++k) { // every load in flight at once
+		const uint32_t i = threadIdx.x + uint32_t(k) * kSegThreads;
+		if (i < n) {
+			keys_out[i] = s_key[i];
+			vals_out[i] = vals[s_pos[i]];
+		}
+	}
+}
+
 constexpr int kScanBlock = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanBlock * kScanItems;
@@ -349,6 +380,11 @@ void radix_sort_pairs(const uint32_t* keys_in, const uint32_t* vals_in, uint32_t
 	if (overlap(keys_in, keys_out) || overlap(keys_in, vals_out) || overlap(vals_in, keys_out) ||
 		overlap(vals_in, vals_out) || overlap(keys_out, vals_out))
 		raise(MARSMD_ERR_VALUE, "radix sort: output buffers must not overlap the inputs or each other");
+	if (n <= kOneGroupMax) {
+		k_rs_one_group<<<1, kSegThreads, 0, s>>>(keys_in, vals_in, keys_out, vals_out, uint32_t(n), key_bits);
+		MMD_LAUNCH_CHECK();
+		return;
+	}
 	const uint32_t tiles = uint32_t((n + kRsTile - 1) / kRsTile);
 	char* sp = static_cast<char*>(scratch);
 	uint32_t* tmp_k = reinterpret_cast<uint32_t*>(sp);
