@@ -353,23 +353,6 @@ __global__ void k_b_import(const float4* __restrict__ pos_h, const float4* __res
 	force[g] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
-__global__ void k_b_export(const float4* __restrict__ pos, const float4* __restrict__ mom,
-						   const float4* __restrict__ force, const int32_t* __restrict__ ids,
-						   const uint32_t* __restrict__ slot_of_canon, uint64_t total, float4* __restrict__ pos_o,
-						   float4* __restrict__ mom_o, float4* __restrict__ force_o, int32_t* __restrict__ type_o,
-						   int32_t* __restrict__ ids_o) {
-	const uint64_t g = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (g >= total)
-		return;
-	const uint32_t s = slot_of_canon[g];
-	const float4 p = pos[s];
-	pos_o[g] = make_float4(p.x, p.y, p.z, 0.0f);
-	mom_o[g] = mom[s];
-	force_o[g] = force[s];
-	type_o[g] = int32_t(meta_type(__float_as_uint(p.w)));
-	ids_o[g] = ids[s];
-}
-
 __global__ void k_b_half_counts(NbrList L, uint64_t slot0, uint64_t n, uint32_t* __restrict__ half) {
 	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
 	if (i >= n)
@@ -672,24 +655,14 @@ void BatchImpl::copy_to_host(float* pos4, float* mom4, float* force4, int32_t* t
 							 uint64_t n) {
 	if (n != total)
 		raise(MARSMD_ERR_VALUE, "batch: copy_particles_to_host returns every replica's particles");
-	DevArray<float4> op(total), om(total), of(total);
-	DevArray<int32_t> ot(total), oi(total);
 	MMD_HIP(hipDeviceSynchronize());
-	k_b_export<<<grid_for(total, 256), 256>>>(pos[cur].data(), mom.data(), force.data(), ids.data(),
-											  slot_of_canon.data(), total, op.data(), om.data(), of.data(), ot.data(),
-											  oi.data());
-	MMD_LAUNCH_CHECK();
-	MMD_HIP(hipDeviceSynchronize());
-	if (pos4)
-		MMD_HIP(hipMemcpy(pos4, op.data(), 16 * total, hipMemcpyDeviceToHost));
-	if (mom4)
-		MMD_HIP(hipMemcpy(mom4, om.data(), 16 * total, hipMemcpyDeviceToHost));
-	if (force4)
-		MMD_HIP(hipMemcpy(force4, of.data(), 16 * total, hipMemcpyDeviceToHost));
-	if (type_ids)
-		MMD_HIP(hipMemcpy(type_ids, ot.data(), 4 * total, hipMemcpyDeviceToHost));
-	if (id_out)
-		MMD_HIP(hipMemcpy(id_out, oi.data(), 4 * total, hipMemcpyDeviceToHost));
+	const ParticleRecords out{reinterpret_cast<float4*>(pos4), reinterpret_cast<float4*>(mom4),
+							  reinterpret_cast<float4*>(force4), type_ids, id_out};
+	host_export.copy(total, out, [this](uint64_t first, uint64_t count, const ParticleRecords& to) {
+		k_export<<<grid_for(count, 256), 256>>>(pos[cur].data(), mom.data(), force.data(), ids.data(),
+												slot_of_canon.data(), first, count, to);
+		MMD_LAUNCH_CHECK();
+	});
 }
 
 // Sort every replica (stable by Morton key of its box, ties by canonical index), move

@@ -4,6 +4,7 @@
 #include <map>
 #include <vector>
 
+#include "hostexport.hpp"
 #include "pairlist.hpp"
 
 namespace mmd {
@@ -101,6 +102,7 @@ struct BatchImpl {
 	BatchImpl& operator=(const BatchImpl&) = delete;
 
 	void copy_from_host(const float* pos4, const float* mom4, const int32_t* type_ids, uint64_t n);
+	HostExport host_export;
 	void copy_to_host(float* pos4, float* mom4, float* force4, int32_t* type_ids, int32_t* ids, uint64_t n);
 	void run(const marsmd_run_params& p, uint64_t first_step, uint64_t num_steps, hipStream_t s);
 	void finish_deferred_kick(float dt, hipStream_t s);

@@ -687,23 +687,6 @@ __global__ void k_import(const float4* __restrict__ pos_h, const float4* __restr
 	slot_of_canon[c] = uint32_t(c);
 }
 
-__global__ void k_export(const float4* __restrict__ pos, const float4* __restrict__ mom,
-						 const float4* __restrict__ force, const int32_t* __restrict__ ids,
-						 const uint32_t* __restrict__ slot_of_canon, uint64_t n, float4* __restrict__ pos_o,
-						 float4* __restrict__ mom_o, float4* __restrict__ force_o, int32_t* __restrict__ type_o,
-						 int32_t* __restrict__ ids_o) {
-	const uint64_t c = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (c >= n)
-		return;
-	const uint32_t s = slot_of_canon[c];
-	const float4 p = pos[s];
-	pos_o[c] = make_float4(p.x, p.y, p.z, 0.0f);
-	mom_o[c] = mom[s];
-	force_o[c] = force[s];
-	type_o[c] = int32_t(meta_type(fb(p.w)));
-	ids_o[c] = ids[s];
-}
-
 uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 
 } // namespace
@@ -1001,23 +984,14 @@ void PatchImpl::copy_to_host(float* pos4, float* mom4, float* force4, int32_t* t
 									  std::to_string(n));
 	if (nn == 0)
 		return;
-	DevArray<float4> op(n), om(n), of(n);
-	DevArray<int32_t> ot(n), oi(n);
 	MMD_HIP(hipDeviceSynchronize());
-	k_export<<<grid_for(n, 256), 256>>>(pos[cur].data(), mom.data(), force.data(), ids.data(), slot_of_canon.data(), n,
-										op.data(), om.data(), of.data(), ot.data(), oi.data());
-	MMD_LAUNCH_CHECK();
-	MMD_HIP(hipDeviceSynchronize());
-	if (pos4)
-		MMD_HIP(hipMemcpy(pos4, op.data(), 16 * nn, hipMemcpyDeviceToHost));
-	if (mom4)
-		MMD_HIP(hipMemcpy(mom4, om.data(), 16 * nn, hipMemcpyDeviceToHost));
-	if (force4)
-		MMD_HIP(hipMemcpy(force4, of.data(), 16 * nn, hipMemcpyDeviceToHost));
-	if (type_ids)
-		MMD_HIP(hipMemcpy(type_ids, ot.data(), 4 * nn, hipMemcpyDeviceToHost));
-	if (id_out)
-		MMD_HIP(hipMemcpy(id_out, oi.data(), 4 * nn, hipMemcpyDeviceToHost));
+	const ParticleRecords out{reinterpret_cast<float4*>(pos4), reinterpret_cast<float4*>(mom4),
+							  reinterpret_cast<float4*>(force4), type_ids, id_out};
+	host_export.copy(nn, out, [this](uint64_t first, uint64_t count, const ParticleRecords& to) {
+		k_export<<<grid_for(count, 256), 256>>>(pos[cur].data(), mom.data(), force.data(), ids.data(),
+												slot_of_canon.data(), first, count, to);
+		MMD_LAUNCH_CHECK();
+	});
 }
 
 void PatchImpl::build(float pairlist_cutoff, hipStream_t s) {

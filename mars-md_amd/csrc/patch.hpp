@@ -6,6 +6,7 @@
 #include <utility>
 #include <vector>
 
+#include "hostexport.hpp"
 #include "pairlist.hpp"
 
 namespace mmd {
@@ -90,6 +91,7 @@ struct PatchImpl {
 	PatchImpl& operator=(const PatchImpl&) = delete;
 
 	void copy_from_host(const float* pos4, const float* mom4, const int32_t* type_ids, uint64_t n);
+	HostExport host_export;
 	void copy_to_host(float* pos4, float* mom4, float* force4, int32_t* type_ids, int32_t* ids, uint64_t n);
 	void calculate_nonbonded(float pairlist_cutoff, float cutoff, uint64_t step, uint64_t period, const float ef[3],
 							 int interp, bool energy, hipStream_t s);
