@@ -51,53 +51,148 @@ __device__ __forceinline__ void bonded_zero(float4* contrib, uint64_t first, int
 			contrib[first + uint64_t(r)] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
+// Per-particle sums of one workgroup's pairs, in LDS: a hash table of particles (linear
+// probing, at most kProbes cells) and their force and energy components.
+constexpr int kPairBlock = 512, kPairsPerLane = 4;
+constexpr uint32_t kPairCells = 2048, kProbes = 8, kNoParticle = 0xFFFFFFFFu;
+struct PairSums {
+	uint32_t particle[kPairCells];
+	float v[4][kPairCells];
+};
+// The cell of `particle`, or kPairCells when its probes are taken by others.
+__device__ __forceinline__ uint32_t pair_cell(PairSums& t, uint32_t particle) {
+	uint32_t c = (particle * 2654435761u) >> 21;
+	static_assert(kPairCells == 1u << (32 - 21), "hash width");
+	for (uint32_t k = 0; k < kProbes; ++k, c = (c + 1u) & (kPairCells - 1u)) {
+		uint32_t have = *reinterpret_cast<volatile uint32_t*>(&t.particle[c]);
+		if (have == kNoParticle)
+			have = atomicCAS(&t.particle[c], kNoParticle, particle);
+		if (have == kNoParticle || have == particle)
+			return c;
+	}
+	return kPairCells;
+}
+__device__ __forceinline__ void lds_add(float* p, float v) {
+	__hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ void pair_add(PairSums& t, float4* __restrict__ fe, int32_t i, float x, float y, float z,
+										 float e, bool energy) {
+	const uint32_t c = pair_cell(t, uint32_t(i));
+	if (c < kPairCells) {
+		lds_add(&t.v[0][c], x);
+		lds_add(&t.v[1][c], y);
+		lds_add(&t.v[2][c], z);
+		if (energy)
+			lds_add(&t.v[3][c], e);
+	} else {
+		atomic_add4(&fe[i], x, y, z);
+		if (energy)
+			atomic_add_f32(reinterpret_cast<float*>(&fe[i]) + 3, e);
+	}
+}
+
 // PairNonbondedComputer::operator() (Pairwise.h:214-304) with ANALYTIC / TABULATED
 // selecting its branches; AnalyticalPairKernel::operator() (AnalyticalPairKernels.h:
 // 44-104) is the ANALYTIC-only instance. The pair's own (x, y) orientation is kept.
-template<bool ANALYTIC, bool TABULATED>
-__global__ void k_pairwise(const int2* __restrict__ pairs, const float4* __restrict__ pos, float4* fe,
-						   const int32_t* __restrict__ type_ids, const uint32_t* __restrict__ tags,
-						   const marsmd_table* __restrict__ tables, PairCoeffs C, DevBox box, int get_energy,
-						   uint64_t np, float cutoff2, uint32_t enabled) {
-	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (i >= np)
-		return;
-	const uint32_t tag = tags ? tags[i] : enabled;
-	const uint32_t terms = tag & enabled & (TABULATED ? MARSMD_PAIR_TERM_MASK : kAnalyticTerms);
-	if (terms == 0u)
-		return;
-	const int2 ij = pairs[i];
-	const float3 r = wrap_diff(box, sub3(pos[ij.y], pos[ij.x]));
-	const float r2 = len2(r);
-	const float d = sqrtf(r2);
-	float3 u = make_float3(0.0f, 0.0f, 0.0f);
-	if (d > 1e-6f) {
-		const float inv = 1.0f / d;
-		u = make_float3(inv * r.x, inv * r.y, inv * r.z);
+// Bound by its global atomics, six or eight a pair (26 G/s). With SUMS a workgroup takes
+// kPairBlock * kPairsPerLane consecutive pairs and adds them up per particle in LDS first:
+// a list that runs along its particles, as a pairlist's, names each one several times in
+// that many pairs, and each then costs one set of atomics per workgroup: 1.43 10^6 pairs of
+// 80021 particles in pairlist order 424 -> 72 us, sorted by (x, y) 383 -> 233 us. A wave whose
+// pairs do not run along a particle skips the sums: in random order 362 -> 367 us.
+template<bool ANALYTIC, bool TABULATED, bool SUMS>
+__global__ __launch_bounds__(kPairBlock) void k_pairwise(const int2* __restrict__ pairs,
+														 const float4* __restrict__ pos, float4* fe,
+														 const int32_t* __restrict__ type_ids,
+														 const uint32_t* __restrict__ tags,
+														 const marsmd_table* __restrict__ tables, PairCoeffs C,
+														 DevBox box, int get_energy, uint64_t np, float cutoff2,
+														 uint32_t enabled) {
+	__shared__ uint32_t lds[SUMS ? sizeof(PairSums) / 4 : 1];
+	[[maybe_unused]] PairSums* const sums = reinterpret_cast<PairSums*>(lds);
+	constexpr int per = SUMS ? kPairsPerLane : 1;
+	if constexpr (SUMS) {
+		for (uint32_t c = threadIdx.x; c < kPairCells; c += blockDim.x) {
+			sums->particle[c] = kNoParticle;
+			for (int k = 0; k < 4; ++k)
+				sums->v[k][c] = 0.0f;
+		}
+		__syncthreads();
 	}
-	if (d < 1e-6f)
-		return;
-	if (cutoff2 > 0.0f && d * d > cutoff2)
-		return;
-	float fm = 0.0f, en = 0.0f;
-	if (ANALYTIC && (terms & kAnalyticTerms)) {
-		const int ti = type_ids[ij.x], tj = type_ids[ij.y];
-		analytic_terms(terms, d, r2, C.charge[ti], C.charge[tj], C.radius[ti], C.radius[tj], C.eps[ti], C.eps[tj],
-					   C.prm, fm, en);
+	// every load of the lane's pairs in flight before the first is used (pairs past the end
+	// and those without a term read as the last pair)
+	const uint64_t first = uint64_t(blockIdx.x) * blockDim.x * per + threadIdx.x;
+	uint32_t tag[per], terms[per];
+	int2 ij[per];
+	float4 px[per], py[per];
+#pragma unroll
+	for (int q = 0; q < per; ++q) {
+		const uint64_t i = first + uint64_t(q) * blockDim.x, at = i < np ? i : np - 1;
+		ij[q] = pairs[at];
+		tag[q] = tags ? tags[at] : enabled;
+		terms[q] = i < np ? tag[q] & enabled & (TABULATED ? MARSMD_PAIR_TERM_MASK : kAnalyticTerms) : 0u;
 	}
-	if (TABULATED && (terms & MARSMD_PAIR_TERM_TABULATED)) {
-		const marsmd_table t = tables[tag >> MARSMD_PAIR_TABLE_SHIFT];
-		const FE v = table_compute(d, t.pot, int(t.size), t.start, t.step_inv, t.is_periodic != 0);
-		fm += v.f;
-		en += v.e;
+#pragma unroll
+	for (int q = 0; q < per; ++q) {
+		px[q] = terms[q] ? pos[ij[q].x] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+		py[q] = terms[q] ? pos[ij[q].y] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 	}
-	const float fx = fm * u.x, fy = fm * u.y, fz = fm * u.z;
-	atomic_add4(&fe[ij.x], -fx, -fy, -fz);
-	atomic_add4(&fe[ij.y], fx, fy, fz);
-	if (get_energy) {
-		const float h = en * 0.5f;
-		atomic_add_f32(reinterpret_cast<float*>(&fe[ij.x]) + 3, h);
-		atomic_add_f32(reinterpret_cast<float*>(&fe[ij.y]) + 3, h);
+#pragma unroll
+	for (int q = 0; q < per; ++q) {
+		bool runs = false; // whether the wave's pairs run along their particles
+		if constexpr (SUMS) {
+			const int2 b = make_int2(__shfl_up(ij[q].x, 1, 64), __shfl_up(ij[q].y, 1, 64));
+			runs = __popcll(__ballot(ij[q].x == b.x || ij[q].y == b.y || ij[q].x == b.y || ij[q].y == b.x)) >= 32;
+		}
+		if (terms[q] == 0u)
+			continue;
+		const float3 r = wrap_diff(box, sub3(py[q], px[q]));
+		const float r2 = len2(r);
+		const float d = sqrtf(r2);
+		float3 u = make_float3(0.0f, 0.0f, 0.0f);
+		if (d > 1e-6f) {
+			const float inv = 1.0f / d;
+			u = make_float3(inv * r.x, inv * r.y, inv * r.z);
+		}
+		if (d < 1e-6f)
+			continue;
+		if (cutoff2 > 0.0f && d * d > cutoff2)
+			continue;
+		float fm = 0.0f, en = 0.0f;
+		if (ANALYTIC && (terms[q] & kAnalyticTerms)) {
+			const int ti = type_ids[ij[q].x], tj = type_ids[ij[q].y];
+			analytic_terms(terms[q], d, r2, C.charge[ti], C.charge[tj], C.radius[ti], C.radius[tj], C.eps[ti],
+						   C.eps[tj], C.prm, fm, en);
+		}
+		if (TABULATED && (terms[q] & MARSMD_PAIR_TERM_TABULATED)) {
+			const marsmd_table t = tables[tag[q] >> MARSMD_PAIR_TABLE_SHIFT];
+			const FE v = table_compute(d, t.pot, int(t.size), t.start, t.step_inv, t.is_periodic != 0);
+			fm += v.f;
+			en += v.e;
+		}
+		const float fx = fm * u.x, fy = fm * u.y, fz = fm * u.z, h = en * 0.5f;
+		if (SUMS && runs) {
+			pair_add(*sums, fe, ij[q].x, -fx, -fy, -fz, h, get_energy != 0);
+			pair_add(*sums, fe, ij[q].y, fx, fy, fz, h, get_energy != 0);
+		} else {
+			atomic_add4(&fe[ij[q].x], -fx, -fy, -fz);
+			atomic_add4(&fe[ij[q].y], fx, fy, fz);
+			if (get_energy) {
+				atomic_add_f32(reinterpret_cast<float*>(&fe[ij[q].x]) + 3, h);
+				atomic_add_f32(reinterpret_cast<float*>(&fe[ij[q].y]) + 3, h);
+			}
+		}
+	}
+	if constexpr (SUMS) {
+		__syncthreads();
+		for (uint32_t c = threadIdx.x; c < kPairCells; c += blockDim.x) {
+			const uint32_t i = sums->particle[c];
+			if (i == kNoParticle)
+				continue;
+			atomic_add4(&fe[i], sums->v[0][c], sums->v[1][c], sums->v[2][c]);
+			if (get_energy)
+				atomic_add_f32(reinterpret_cast<float*>(&fe[i]) + 3, sums->v[3][c]);
+		}
 	}
 }
 
@@ -421,6 +516,16 @@ void launch_resolve_pair_tables(const int32_t* pairs, const int32_t* types, cons
 	MMD_LAUNCH_CHECK();
 }
 
+// From 2^18 pairs on the sums in LDS pay whatever the list's order; below, a workgroup's
+// 2048 pairs leave too few workgroups. Microseconds without and with, in pairlist, sorted
+// and random order: 2^17 pairs 46, 39, 38 and 25, 43, 42; 2^18 pairs 86, 74, 74 and
+// 29, 60, 75.
+static bool pair_sums(uint64_t np) { return np >= (uint64_t(1) << 18); }
+static unsigned pair_block(uint64_t np) { return pair_sums(np) ? kPairBlock : 256; }
+static unsigned pair_grid(uint64_t np) {
+	return pair_sums(np) ? grid_for(np, kPairBlock * kPairsPerLane) : grid_for(np, 256);
+}
+
 void launch_pairwise_nonbonded(const int32_t* pairs, const marsmd_particle_view& v, const uint32_t* tags,
 							   const marsmd_table* tables, const marsmd_particle_types* types, const marsmd_box& box,
 							   bool energy, uint64_t np, float cutoff2, uint32_t enabled,
@@ -433,10 +538,13 @@ void launch_pairwise_nonbonded(const int32_t* pairs, const marsmd_particle_view&
 	if ((enabled & MARSMD_PAIR_TERM_TABULATED) && !tables)
 		raise(MARSMD_ERR_VALUE, "launch_pairwise_nonbonded: the tabulated term needs the tables");
 	const PairCoeffs C = types ? make_pair_coeffs(*types, params) : PairCoeffs{};
-	auto kern = an ? k_pairwise<true, true> : k_pairwise<false, true>;
-	kern<<<grid_for(np, 256), 256, 0, s>>>(reinterpret_cast<const int2*>(pairs), reinterpret_cast<const float4*>(v.pos),
-										   reinterpret_cast<float4*>(v.force_energy), v.type_id, tags, tables, C,
-										   make_devbox(box), energy ? 1 : 0, np, cutoff2, enabled);
+	const bool sums = pair_sums(np);
+	auto kern = an ? (sums ? k_pairwise<true, true, true> : k_pairwise<true, true, false>)
+				   : (sums ? k_pairwise<false, true, true> : k_pairwise<false, true, false>);
+	kern<<<pair_grid(np), pair_block(np), 0, s>>>(
+		reinterpret_cast<const int2*>(pairs), reinterpret_cast<const float4*>(v.pos),
+		reinterpret_cast<float4*>(v.force_energy), v.type_id, tags, tables, C, make_devbox(box), energy ? 1 : 0, np,
+		cutoff2, enabled);
 	MMD_LAUNCH_CHECK();
 }
 
@@ -446,7 +554,8 @@ void launch_analytical_pair_nonbonded(const int32_t* pairs, const float* pos, fl
 									  float cutoff2, hipStream_t s) {
 	if (np == 0 || (enabled & kAnalyticTerms) == 0u)
 		return;
-	k_pairwise<true, false><<<grid_for(np, 256), 256, 0, s>>>(
+	auto kern = pair_sums(np) ? k_pairwise<true, false, true> : k_pairwise<true, false, false>;
+	kern<<<pair_grid(np), pair_block(np), 0, s>>>(
 		reinterpret_cast<const int2*>(pairs), reinterpret_cast<const float4*>(pos), reinterpret_cast<float4*>(fe),
 		type_ids, tags, nullptr, make_pair_coeffs(types, params), make_devbox(box), energy ? 1 : 0, np, cutoff2,
 		enabled);
