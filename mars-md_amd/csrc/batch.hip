@@ -255,10 +255,18 @@ __global__ __launch_bounds__(256, 6) void k_b_walk(const RepGeom* __restrict__ g
 
 // max over particles of |min_image(pos - snapshot)|^2, per batch (the largest replica
 // displacement decides): DisplacementKernel (AdaptiveKernels.h:48-101).
-__global__ __launch_bounds__(256) void k_b_max_disp(const float4* __restrict__ cur, const float4* __restrict__ snap,
-													uint64_t total, const uint32_t* __restrict__ rep_of_slot,
-													const RepGeom* __restrict__ geom,
-													uint32_t* __restrict__ out_bits) {
+// The largest squared displacement since the build (as float bits) to the host's pinned
+// word. Bound by the 36 bytes read a particle and the atomics, one pair per workgroup; the
+// last workgroup writes the word and clears acc (two words): 29 us at 2.6 10^6 beads (64 with
+// one atomic per wave and the word copied).
+constexpr int kDispBlock = 1024;
+__global__ __launch_bounds__(kDispBlock) void k_b_max_disp(const float4* __restrict__ cur,
+														   const float4* __restrict__ snap, uint64_t total,
+														   const uint32_t* __restrict__ rep_of_slot,
+														   const RepGeom* __restrict__ geom,
+														   uint32_t* __restrict__ acc,
+														   unsigned long long* __restrict__ out) {
+	__shared__ float wmax[kDispBlock / 64];
 	float m = 0.0f;
 	for (uint64_t s = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; s < total;
 		 s += uint64_t(gridDim.x) * blockDim.x) {
@@ -280,7 +288,61 @@ __global__ __launch_bounds__(256) void k_b_max_disp(const float4* __restrict__ c
 	for (int o = 32; o > 0; o >>= 1)
 		m = fmaxf(m, __shfl_xor(m, o, 64));
 	if ((threadIdx.x & 63) == 0)
-		atomicMax(out_bits, __float_as_uint(m));
+		wmax[threadIdx.x >> 6] = m;
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		for (int w = 1; w < kDispBlock / 64; ++w)
+			m = fmaxf(m, wmax[w]);
+		atomicMax(&acc[0], __float_as_uint(m)); // non-negative floats order as uints
+		__threadfence(); // before the ticket
+		if (atomicAdd(&acc[1], 1u) == gridDim.x - 1u) {
+			*out = atomicExch(&acc[0], 0u);
+			acc[1] = 0u;
+		}
+	}
+}
+
+// The step kernels' constants in device memory (as kernel arguments they were 3.4 KB read
+// back by every workgroup of every launch).
+struct BatchConsts {
+	alignas(16) NbTables nb;
+	alignas(16) marsmd_particle_types types;
+};
+constexpr int kBatchSplitBlock = 512;
+
+// The rest of slot t's step once its nonbonded force f is summed.
+template<int INTEG, bool ENERGY>
+__device__ __forceinline__ void b_step_finish(uint64_t t, const float4 p, float4 f, const RepGeom& G, uint32_t step,
+											  float4* __restrict__ pos_next, float4* __restrict__ mom,
+											  float4* __restrict__ force, const marsmd_particle_types& types,
+											  const TypeStep* steps, const StepParams& S, uint64_t base_seed,
+											  int store_force) {
+	StepParams P = S;
+	P.box = G.box;
+	P.step = step;
+	P.seed = mix_seed(base_seed, G.pid, uint64_t(step));
+	float4 pn;
+	if (INTEG == MARSMD_INTEGRATOR_BROWNIAN) {
+		const float4 pmf =
+			position_dependent_force(p.x, p.y, p.z, int(meta_type(fb(p.w))), types, nullptr, P.ef, P.scheme);
+		pn = bd_update(p, f, steps[meta_type(fb(p.w))], pmf, P);
+	} else {
+		float4 mo = mom[t];
+		pn = baoab_update(p, mo, f, steps[meta_type(fb(p.w))], P);
+		mom[t] = mo;
+	}
+	pos_next[t] = pn;
+	if (ENERGY || store_force)
+		force[t] = f;
+}
+
+template<int INTEG>
+__device__ __forceinline__ void b_stage_step(const BatchConsts& C, const StepParams& S, marsmd_particle_types& types,
+											 TypeStep* steps) {
+	stage_types(C.types, types);
+	if (threadIdx.x < uint32_t(C.types.num_types))
+		steps[threadIdx.x] = INTEG == MARSMD_INTEGRATOR_BROWNIAN ? bd_type_step(C.types, int(threadIdx.x), S)
+																 : baoab_type_step(C.types, int(threadIdx.x), S);
 }
 
 // The fused step over every replica's particles, persistent over XCD-local tiles: the
@@ -291,21 +353,18 @@ template<int INTEG, bool ENERGY, bool ANALYTIC>
 __global__ __launch_bounds__(kBatchBlock, 5) void k_b_step(const float4* __restrict__ pos, float4* __restrict__ pos_next,
 														  float4* __restrict__ mom, float4* __restrict__ force,
 														  uint64_t total, const uint32_t* __restrict__ rep_of_slot,
-														  const RepGeom* __restrict__ geom, NbrList L, NbTables T,
-														  const float* __restrict__ knots_g,
-														  marsmd_particle_types types_arg, StepParams S,
+														  const RepGeom* __restrict__ geom, NbrList L,
+														  const BatchConsts* __restrict__ C,
+														  const float* __restrict__ knots_g, StepParams S,
 														  uint64_t base_seed, int store_force,
-														  const uint32_t* __restrict__ step_base) {
+														  const uint32_t* __restrict__ step_base, uint32_t, uint32_t) {
 	extern __shared__ float lds_knots[];
 	__shared__ NbLds lds_nb;
 	__shared__ marsmd_particle_types lds_types;
 	__shared__ TypeStep lds_steps[MARSMD_MAX_TYPES]; // the integrator's per-type constants
-	stage_types(types_arg, lds_types);
-	if (threadIdx.x < uint32_t(types_arg.num_types))
-		lds_steps[threadIdx.x] = INTEG == MARSMD_INTEGRATOR_BROWNIAN ? bd_type_step(types_arg, int(threadIdx.x), S)
-																	 : baoab_type_step(types_arg, int(threadIdx.x), S);
+	const NbTables& T = C->nb;
+	b_stage_step<INTEG>(*C, S, lds_types, lds_steps);
 	stage_tables(T, knots_g, lds_knots, lds_nb);
-	const marsmd_particle_types& types = lds_types;
 	// a replayed segment carries the step's offset in S.step and its first step in memory
 	const uint32_t step = S.step + (step_base ? step_base[0] : 0u);
 	const TileRange R = xcd_tiles(uint32_t((total + kBatchBlock - 1) / kBatchBlock));
@@ -314,25 +373,58 @@ __global__ __launch_bounds__(kBatchBlock, 5) void k_b_step(const float4* __restr
 		if (t >= total)
 			continue;
 		const RepGeom& G = geom[rep_of_slot[t]];
-		StepParams P = S;
-		P.box = G.box;
-		P.step = step;
-		P.seed = mix_seed(base_seed, G.pid, uint64_t(step));
 		const float4 p = pos[t];
-		float4 f = nb_force<ANALYTIC>(uint32_t(t), p, pos, L, T, lds_knots, knots_g, lds_nb, P.box, P.cut_d, ENERGY);
-		float4 pn;
-		if (INTEG == MARSMD_INTEGRATOR_BROWNIAN) {
-			const float4 pmf = position_dependent_force(p.x, p.y, p.z, int(meta_type(fb(p.w))), types, nullptr, P.ef,
-														P.scheme);
-			pn = bd_update(p, f, lds_steps[meta_type(fb(p.w))], pmf, P);
-		} else {
-			float4 mo = mom[t];
-			pn = baoab_update(p, mo, f, lds_steps[meta_type(fb(p.w))], P);
-			mom[t] = mo;
-		}
-		pos_next[t] = pn;
-		if (ENERGY || store_force)
-			force[t] = f;
+		const DevBox box = G.box;
+		const float4 f =
+			nb_force<ANALYTIC>(uint32_t(t), p, pos, L, T, lds_knots, knots_g, lds_nb, box, S.cut_d, ENERGY);
+		b_step_finish<INTEG, ENERGY>(t, p, f, G, step, pos_next, mom, force, lds_types, lds_steps, S, base_seed,
+									 store_force);
+	}
+}
+
+// The same step with 1 << split lanes to a slot's row (row_split, nb_force_split), for
+// batches whose slots do not fill the chip: the serial walk along a row bounds them. A
+// tile is 512 >> split slots; the sums change hands in LDS (two tiles' buffers in turn)
+// and one lane per slot finishes the step. 24 replicas, 45k beads (4 lanes a row): 13.4 -> 9.8 us.
+template<int INTEG, bool ENERGY, bool ANALYTIC>
+__global__ __launch_bounds__(kBatchSplitBlock, 4) void k_b_step_split(
+	const float4* __restrict__ pos, float4* __restrict__ pos_next, float4* __restrict__ mom, float4* __restrict__ force,
+	uint64_t total, const uint32_t* __restrict__ rep_of_slot, const RepGeom* __restrict__ geom, NbrList L,
+	const BatchConsts* __restrict__ C, const float* __restrict__ knots_g, StepParams S, uint64_t base_seed,
+	int store_force, const uint32_t* __restrict__ step_base, uint32_t split, uint32_t knot_words) {
+	extern __shared__ float lds_knots[]; // knot_words words (a multiple of 4), then the handed-over forces
+	__shared__ NbLds lds_nb;
+	__shared__ marsmd_particle_types lds_types;
+	__shared__ TypeStep lds_steps[MARSMD_MAX_TYPES];
+	__shared__ float terms[kBatchSplitBlock / 64][split_terms(ENERGY)];
+	const NbTables& T = C->nb;
+	const uint32_t per = uint32_t(kBatchSplitBlock) >> split; // slots of a tile
+	const uint32_t mine = threadIdx.x >> split, sub = threadIdx.x & ((1u << split) - 1u);
+	float4* lds_force = reinterpret_cast<float4*>(lds_knots + knot_words);
+	const uint32_t lane = threadIdx.x & 63u;
+	const uint32_t first = (threadIdx.x - lane) >> split; // the wave's first slot of a tile
+	const TileRange R = xcd_tiles(uint32_t((total + per - 1) / per));
+	RowHead h{};
+	if (R.tile < R.end)
+		h = row_head(R.tile * per + mine, uint32_t(total), sub, pos, L);
+	b_stage_step<INTEG>(*C, S, lds_types, lds_steps);
+	stage_tables(T, knots_g, lds_knots, lds_nb);
+	const uint32_t step = S.step + (step_base ? step_base[0] : 0u);
+	float* const wt = terms[threadIdx.x >> 6];
+	uint32_t turn = 0;
+	for (uint32_t tile = R.tile; tile < R.end; tile += R.stride, turn ^= 1u) {
+		const DevBox box = geom[rep_of_slot[min(tile * per + mine, uint32_t(total) - 1u)]].box;
+		const float f = T.lds ? nb_force_split<ANALYTIC>(h, sub, split, pos, T, lds_knots, lds_nb, box, S.cut_d, ENERGY, wt)
+							  : nb_force_split<ANALYTIC>(h, sub, split, pos, T, knots_g, lds_nb, box, S.cut_d, ENERGY, wt);
+		if ((lane >> 2) < (64u >> split))
+			reinterpret_cast<float*>(lds_force)[4u * (turn * per + first + (lane >> 2)) + (lane & 3u)] = f;
+		if (tile + R.stride < R.end)
+			h = row_head((tile + R.stride) * per + mine, uint32_t(total), sub, pos, L);
+		__syncthreads(); // (the other buffer's readers finished before it)
+		const uint32_t u = tile * per + threadIdx.x;
+		if (threadIdx.x < per && u < total)
+			b_step_finish<INTEG, ENERGY>(u, pos[u], lds_force[turn * per + threadIdx.x], geom[rep_of_slot[u]], step,
+										 pos_next, mom, force, lds_types, lds_steps, S, base_seed, store_force);
 	}
 }
 
@@ -387,27 +479,42 @@ __global__ void k_b_write_pairs(NbrList L, const float4* __restrict__ pos, uint6
 
 // Full-list entries of each replica (twice its pair count): one workgroup per replica
 // sums the counts of its slots, which are one contiguous range.
-__global__ __launch_bounds__(256) void k_b_rep_pairs(const uint32_t* __restrict__ counts,
-													 const RepGeom* __restrict__ geom,
+// Each replica's entries and longest row to the host's pinned words out[1 + r] and
+// out[1 + R + r], and the build's flags to out[0] (cleared for the next build).
+__global__ __launch_bounds__(256) void k_b_rep_stats(const uint32_t* __restrict__ counts,
+													 const RepGeom* __restrict__ geom, uint32_t* __restrict__ flags,
 													 unsigned long long* __restrict__ out) {
 	__shared__ unsigned long long wsum[4];
+	__shared__ uint32_t wmax[4];
 	const uint32_t b = geom[blockIdx.x].slot0;
 	const uint32_t e = b + geom[blockIdx.x].n;
 	unsigned long long sum = 0;
+	uint32_t m = 0;
 	for (uint32_t i = b + threadIdx.x; i < e; i += 1024u) { // four loads in flight
 		const uint32_t c0 = counts[i];
 		const uint32_t c1 = i + 256u < e ? counts[i + 256u] : 0u;
 		const uint32_t c2 = i + 512u < e ? counts[i + 512u] : 0u;
 		const uint32_t c3 = i + 768u < e ? counts[i + 768u] : 0u;
 		sum += (unsigned long long)c0 + c1 + c2 + c3;
+		m = max(max(m, c0), max(c1, max(c2, c3)));
 	}
-	for (int o = 32; o > 0; o >>= 1)
+	for (int o = 32; o > 0; o >>= 1) {
 		sum += __shfl_xor(sum, o, 64);
-	if ((threadIdx.x & 63) == 0)
+		m = max(m, uint32_t(__shfl_xor(int(m), o, 64)));
+	}
+	if ((threadIdx.x & 63) == 0) {
 		wsum[threadIdx.x >> 6] = sum;
+		wmax[threadIdx.x >> 6] = m;
+	}
 	__syncthreads();
-	if (threadIdx.x == 0)
-		out[blockIdx.x] = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+	if (threadIdx.x == 0) {
+		out[1 + blockIdx.x] = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+		out[1 + gridDim.x + blockIdx.x] = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
+		if (blockIdx.x == 0) {
+			out[0] = flags[0];
+			flags[0] = 0u;
+		}
+	}
 }
 
 // BAOAB_LastUpdate (BAOAB.h:151-172) on every replica's particles.
@@ -432,63 +539,40 @@ __global__ void k_b_set_word(uint32_t* __restrict__ word, uint32_t value) {
 }
 
 using StepKernel = void (*)(const float4*, float4*, float4*, float4*, uint64_t, const uint32_t*, const RepGeom*,
-							NbrList, NbTables, const float*, marsmd_particle_types, StepParams, uint64_t, int,
-							const uint32_t*);
+							NbrList, const BatchConsts*, const float*, StepParams, uint64_t, int, const uint32_t*,
+							uint32_t, uint32_t);
+
+template<int INTEG, bool ENERGY, bool ANALYTIC>
+StepKernel b_step_kernel(bool split) {
+	return split ? k_b_step_split<INTEG, ENERGY, ANALYTIC> : k_b_step<INTEG, ENERGY, ANALYTIC>;
+}
+StepKernel pick_b_step(bool split, bool bd, bool energy, bool analytic) {
+	constexpr int B = MARSMD_INTEGRATOR_BROWNIAN, L = MARSMD_INTEGRATOR_LANGEVIN;
+	if (bd)
+		return energy ? (analytic ? b_step_kernel<B, true, true>(split) : b_step_kernel<B, true, false>(split))
+					  : (analytic ? b_step_kernel<B, false, true>(split) : b_step_kernel<B, false, false>(split));
+	return energy ? (analytic ? b_step_kernel<L, true, true>(split) : b_step_kernel<L, true, false>(split))
+				  : (analytic ? b_step_kernel<L, false, true>(split) : b_step_kernel<L, false, false>(split));
+}
 
 // What a captured segment bakes in besides the step offsets: the graph cache's key.
 struct SegmentKey {
 	const void* kernel;
 	unsigned grid, lds;
+	uint32_t split, knot_words;
 	uint64_t count, total, base_seed;
 	const void* ptr[9];
 	StepParams S;
-	NbTables T;
-	marsmd_particle_types types;
 };
 
-__global__ void k_b_uniform_tile_base(uint32_t* __restrict__ tile_base, uint64_t tiles, uint32_t row) {
-	const uint64_t w = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (w <= tiles)
-		tile_base[w] = uint32_t(w * row);
-}
-
-__global__ __launch_bounds__(256) void k_b_count_stats(const uint32_t* __restrict__ counts, uint64_t n,
-													   unsigned long long* __restrict__ total,
-													   uint32_t* __restrict__ max_count) {
-	__shared__ uint32_t wmax[4];
-	__shared__ unsigned long long wsum[4];
-	uint32_t m = 0;
-	unsigned long long sum = 0;
-	const uint64_t stride = uint64_t(gridDim.x) * blockDim.x;
-	for (uint64_t t = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x; t < n; t += 4 * stride) {
-		// four loads in flight per thread (0 is neutral for both the sum and the maximum)
-		const uint32_t c0 = counts[t];
-		const uint32_t c1 = t + stride < n ? counts[t + stride] : 0u;
-		const uint32_t c2 = t + 2 * stride < n ? counts[t + 2 * stride] : 0u;
-		const uint32_t c3 = t + 3 * stride < n ? counts[t + 3 * stride] : 0u;
-		m = max(max(m, c0), max(c1, max(c2, c3)));
-		sum += (unsigned long long)c0 + c1 + c2 + c3;
-	}
-	for (int o = 32; o > 0; o >>= 1) {
-		m = max(m, uint32_t(__shfl_xor(int(m), o, 64)));
-		sum += __shfl_xor(sum, o, 64);
-	}
-	const int w = threadIdx.x >> 6;
-	if ((threadIdx.x & 63) == 0) {
-		wmax[w] = m;
-		wsum[w] = sum;
-	}
-	__syncthreads();
-	if (threadIdx.x == 0) {
-		uint32_t bm = 0;
-		unsigned long long bs = 0;
-		for (int k = 0; k < int(blockDim.x >> 6); ++k) {
-			bm = max(bm, wmax[k]);
-			bs += wsum[k];
-		}
-		atomicAdd(total, bs);
-		atomicMax(max_count, bm);
-	}
+// Ready for a walk: the cell tables cleared and the uniform rows' bases.
+__global__ void k_b_walk_setup(uint2* __restrict__ cells, uint64_t num_cells, uint32_t* __restrict__ tile_base,
+							   uint64_t tiles, uint32_t row) {
+	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (i < num_cells)
+		cells[i] = make_uint2(0u, 0u);
+	if (i <= tiles)
+		tile_base[i] = uint32_t(i * row);
 }
 
 } // namespace
@@ -549,6 +633,14 @@ BatchImpl::BatchImpl(const marsmd_batch_desc& d) : tables(new NbTables{}) {
 			raise(MARSMD_ERR_VALUE, "batch: a pair tag names a missing table");
 	T.total_knots = int(kn.size());
 	T.lds = T.total_knots <= kLdsKnots ? 1 : 0;
+	{
+		BatchConsts c;
+		std::memset(&c, 0, sizeof(c));
+		c.nb = T;
+		c.types = types;
+		consts.resize(sizeof(c));
+		MMD_HIP(hipMemcpy(consts.data(), &c, sizeof(c), hipMemcpyHostToDevice));
+	}
 	knots.resize(std::max<uint64_t>(kn.size(), 1));
 	if (!kn.empty())
 		MMD_HIP(hipMemcpy(knots.data(), kn.data(), kn.size() * 4, hipMemcpyHostToDevice));
@@ -576,11 +668,9 @@ BatchImpl::BatchImpl(const marsmd_batch_desc& d) : tables(new NbTables{}) {
 	ids_tmp.resize(total);
 	slot_of_canon.resize(total);
 	slot_of_canon_tmp.resize(total);
-	scalars.resize(8);
 	ref_max_pairs.resize(R);
 	for (uint64_t r = 0; r < R; ++r)
 		ref_max_pairs[r] = std::max<uint64_t>(count[r], 1);
-	rep_pairs.resize(R);
 	rep_pairs_host.resize(R);
 }
 
@@ -776,7 +866,7 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 	// keeps it off the GPU's idle time when a run starts with a rebuild
 	if (!(plan.valid && plan.rc == rc && plan.target == cell_target && plan.fine == cell_fine && plan.own == cells_auto &&
 		  plan.ref == ref_max_pairs)) {
-		plan.valid = false; // until planned whole
+		plan.valid = geom_uploaded = false; // until planned whole and uploaded
 		plan_geometry(rc, geom_host, items, plan.fine_total, plan.home_total);
 		plan.valid = true;
 		plan.rc = rc;
@@ -789,17 +879,20 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 	num_fine = fine_total;
 	num_home = home_total;
 	num_items = items[R];
-	// both uploads from pinned memory, so that they queue behind the running steps
-	// without the host waiting for them (the last build's copies ended before its wait)
-	const size_t gbytes = R * sizeof(RepGeom);
-	if (!staging)
-		MMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&staging), gbytes + 4 * (R + 1), hipHostMallocDefault));
-	std::memcpy(staging, geom_host.data(), gbytes);
-	std::memcpy(staging + gbytes, items.data(), 4 * (R + 1));
-	geom.resize(gbytes);
-	MMD_HIP(hipMemcpyAsync(geom.data(), staging, gbytes, hipMemcpyHostToDevice, s));
-	item_off.resize(R + 1);
-	MMD_HIP(hipMemcpyAsync(item_off.data(), staging + gbytes, 4 * (R + 1), hipMemcpyHostToDevice, s));
+	if (!geom_uploaded) {
+		// both uploads from pinned memory, so that they queue behind the running steps
+		// without the host waiting for them (the last build's copies ended before its wait)
+		const size_t gbytes = R * sizeof(RepGeom);
+		if (!staging)
+			MMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&staging), gbytes + 4 * (R + 1), hipHostMallocDefault));
+		std::memcpy(staging, geom_host.data(), gbytes);
+		std::memcpy(staging + gbytes, items.data(), 4 * (R + 1));
+		geom.resize(gbytes);
+		MMD_HIP(hipMemcpyAsync(geom.data(), staging, gbytes, hipMemcpyHostToDevice, s));
+		item_off.resize(R + 1);
+		MMD_HIP(hipMemcpyAsync(item_off.data(), staging + gbytes, 4 * (R + 1), hipMemcpyHostToDevice, s));
+		geom_uploaded = true;
+	}
 	const RepGeom* gd = reinterpret_cast<const RepGeom*>(geom.data());
 	// sort: Morton key (stable; ties by canonical index), then replica (stable)
 	keys.resize(total);
@@ -811,7 +904,10 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 	rkeys_s.resize(total);
 	rvals_s.resize(total);
 	codes.resize(total);
-	fill_u32(scalars.data(), 0u, 8, s);
+	if (!scalars.data()) { // zero between builds and checks: their kernels leave them so
+		scalars.resize(4);
+		fill_u32(scalars.data(), 0u, 4, s);
+	}
 	k_b_encode<<<grid_for(total, 256), 256, 0, s>>>(pos[cur].data(), total, rep_of_slot.data(), gd, keys.data(),
 													vals.data(), scalars.data());
 	MMD_LAUNCH_CHECK();
@@ -843,10 +939,6 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 	cells.resize(num_fine + num_home);
 	uint2* const fine = cells.data();
 	uint2* const home = fine + num_fine;
-	fill_u32(reinterpret_cast<uint32_t*>(fine), 0u, 2 * (num_fine + num_home), s);
-	k_b_cell_ranges<<<grid_for(total, 256), 256, 0, s>>>(codes.data(), total, rep_of_slot.data(), gd, fine, home,
-														 scalars.data());
-	MMD_LAUNCH_CHECK();
 	// walk with uniform rows of `cap` entries; once more with larger rows if needed
 	const uint64_t tiles = (total + 63) / 64;
 	counts.resize(total);
@@ -858,6 +950,12 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 		const double mean = double(total) / vol * 4.0 / 3.0 * 3.141592653589793 * double(rc) * rc * rc;
 		cap = uint32_t(std::min(1.6 * mean + 16.0, 4096.0) + 3) & ~3u;
 	}
+	k_b_walk_setup<<<grid_for(std::max(num_fine + num_home, tiles + 1), 256), 256, 0, s>>>(
+		fine, num_fine + num_home, tile_base.data(), tiles, 64u * cap);
+	MMD_LAUNCH_CHECK();
+	k_b_cell_ranges<<<grid_for(total, 256), 256, 0, s>>>(codes.data(), total, rep_of_slot.data(), gd, fine, home,
+														 scalars.data());
+	MMD_LAUNCH_CHECK();
 	const unsigned groups = unsigned((num_items + kHomeWaves - 1) / kHomeWaves);
 	const unsigned grid = std::max(8u, (groups + 7u) / 8u * 8u);
 	for (int attempt = 0; attempt < 2; ++attempt) {
@@ -866,38 +964,37 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 			raise(MARSMD_ERR_CAPACITY, "batch: neighbour storage exceeds 2^32 entries");
 		if (storage > nbr.count)
 			nbr.resize(storage + storage / 8 + 1024);
-		k_b_uniform_tile_base<<<grid_for(tiles + 1, 256), 256, 0, s>>>(tile_base.data(), tiles, 64u * cap);
-		MMD_LAUNCH_CHECK();
+		if (attempt > 0) { // larger rows
+			k_b_walk_setup<<<grid_for(tiles + 1, 256), 256, 0, s>>>(nullptr, 0, tile_base.data(), tiles, 64u * cap);
+			MMD_LAUNCH_CHECK();
+		}
 		k_b_walk<<<grid, 256, 0, s>>>(gd, item_off.data(), uint32_t(R), uint32_t(num_items), pos[cur].data(),
 									  home, fine, rc2, cap, stencils.data(), counts.data(), nbr.data());
 		MMD_LAUNCH_CHECK();
-		fill_u32(scalars.data() + 2, 0u, 4, s);
-		k_b_count_stats<<<std::min<unsigned>(grid_for(total, 256), 240), 256, 0, s>>>(
-			counts.data(), total, reinterpret_cast<unsigned long long*>(scalars.data() + 4), scalars.data() + 2);
-		MMD_LAUNCH_CHECK();
-		// Pairlist::grow_pair_capacity (Pairlist.h:244-251) bookkeeping per replica, read
-		// back with the walk's statistics: one wait for both (into pinned memory)
-		k_b_rep_pairs<<<unsigned(R), 256, 0, s>>>(counts.data(), gd, rep_pairs.data());
-		MMD_LAUNCH_CHECK();
+		// Pairlist::grow_pair_capacity (Pairlist.h:244-251) bookkeeping per replica with the
+		// walk's statistics: one wait for both (in pinned memory)
 		if (!readback)
-			MMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&readback), 32 + 8 * R, hipHostMallocDefault));
-		MMD_HIP(hipMemcpyAsync(readback, scalars.data(), 24, hipMemcpyDeviceToHost, s));
-		MMD_HIP(hipMemcpyAsync(readback + 4, rep_pairs.data(), 8 * R, hipMemcpyDeviceToHost, s));
+			MMD_HIP(hipHostMalloc(reinterpret_cast<void**>(&readback), 8 * (1 + 2 * R), hipHostMallocDefault));
+		k_b_rep_stats<<<unsigned(R), 256, 0, s>>>(counts.data(), gd, scalars.data(),
+												  reinterpret_cast<unsigned long long*>(readback));
+		MMD_LAUNCH_CHECK();
 		MMD_HIP(hipStreamSynchronize(s));
-		uint32_t host[6];
-		std::memcpy(host, readback, 24);
-		if (host[0] & 1u)
+		if (readback[0] & 1u)
 			raise(MARSMD_ERR_VALUE, "batch: a particle left its replica's box (positions must stay wrapped)");
-		if (host[0] & 2u)
+		if (readback[0] & 2u)
 			raise(MARSMD_ERR_RUNTIME, "batch: Morton codes after the sort were not in order");
-		max_neighbors = host[2];
-		std::memcpy(&nbr_entries, &host[4], 8);
+		nbr_entries = 0;
+		max_neighbors = 0;
+		for (uint64_t r = 0; r < R; ++r) {
+			nbr_entries += readback[1 + r];
+			max_neighbors = std::max(max_neighbors, uint32_t(readback[1 + R + r]));
+		}
 		if (max_neighbors <= cap)
 			break;
 		cap = (max_neighbors + max_neighbors / 8 + 4 + 3) & ~3u;
 	}
 	// the pair counts set the reference grid of the next build
-	std::memcpy(rep_pairs_host.data(), readback + 4, 8 * R);
+	std::memcpy(rep_pairs_host.data(), readback + 1, 8 * R);
 	for (uint64_t r = 0; r < R; ++r) {
 		const uint64_t np = rep_pairs_host[r] / 2;
 		if (np > ref_max_pairs[r])
@@ -908,32 +1005,49 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 }
 
 bool BatchImpl::needs_rebuild(float skin, hipStream_t s) {
-	fill_u32(scalars.data() + 1, 0u, 1, s);
-	k_b_max_disp<<<std::min<unsigned>(grid_for(total, 256), 1024), 256, 0, s>>>(
+	// (a build has allocated both)
+	k_b_max_disp<<<std::min<unsigned>(grid_for(total, kDispBlock), 256), kDispBlock, 0, s>>>(
 		pos[cur].data(), snap.data(), total, rep_of_slot.data(), reinterpret_cast<const RepGeom*>(geom.data()),
-		scalars.data() + 1);
+		scalars.data() + 1, reinterpret_cast<unsigned long long*>(readback));
 	MMD_LAUNCH_CHECK();
-	// into the pinned word after the walk's statistics (a build has allocated it)
-	MMD_HIP(hipMemcpyAsync(readback + 3, scalars.data() + 1, 4, hipMemcpyDeviceToHost, s));
 	MMD_HIP(hipStreamSynchronize(s));
+	const uint32_t bits = uint32_t(readback[0]);
 	float d2;
-	std::memcpy(&d2, readback + 3, 4);
+	std::memcpy(&d2, &bits, 4);
 	return std::sqrt(d2) > skin * 0.5f;
 }
 
-unsigned BatchImpl::step_grid(const void* kernel) {
-	const unsigned lds = tables->lds ? unsigned(std::max(tables->total_knots, 2)) * 4u : 0u;
-	if (occupancy == 0) {
-		MMD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occupancy, kernel, kBatchBlock, lds));
+BatchImpl::StepShape BatchImpl::step_shape() const {
+	const unsigned words = tables->lds ? unsigned(std::max(tables->total_knots, 2)) : 0u;
+	StepShape sh;
+	sh.split = row_split(total, max_neighbors, nbr_entries);
+	if (sh.split == 0) {
+		sh.tiles = (total + kBatchBlock - 1) / kBatchBlock;
+		sh.block = kBatchBlock;
+		sh.lds = 4u * words;
+	} else {
+		const unsigned per = unsigned(kBatchSplitBlock) >> sh.split;
+		sh.tiles = (total + per - 1) / per;
+		sh.block = kBatchSplitBlock;
+		sh.knot_words = (words + 3u) & ~3u;
+		sh.lds = 4u * sh.knot_words + 32u * per; // the knots, then the handed-over forces of two tiles
+	}
+	return sh;
+}
+
+unsigned BatchImpl::step_grid(const void* kernel, const StepShape& sh) {
+	if (occupancy == 0 || occupancy_lds != sh.lds || occupancy_block != sh.block) {
+		MMD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occupancy, kernel, int(sh.block), sh.lds));
 		occupancy = std::max(occupancy, 1);
+		occupancy_lds = sh.lds;
+		occupancy_block = sh.block;
 		int dev = 0;
 		MMD_HIP(hipGetDevice(&dev));
 		MMD_HIP(hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, dev));
 		num_cus = std::max(num_cus, 1);
 	}
 	const int per_cu = blocks_per_cu > 0 ? std::min(blocks_per_cu, occupancy) : occupancy;
-	const uint64_t tiles = (total + kBatchBlock - 1) / kBatchBlock;
-	uint64_t g = std::min<uint64_t>(uint64_t(per_cu) * uint64_t(num_cus), (tiles + 7) / 8 * 8);
+	uint64_t g = std::min<uint64_t>(uint64_t(per_cu) * uint64_t(num_cus), (sh.tiles + 7) / 8 * 8);
 	return unsigned(std::max<uint64_t>((g + 7) / 8 * 8, 8));
 }
 
@@ -944,13 +1058,15 @@ void BatchImpl::set_launch(int bpc, bool graph) {
 	use_graph = graph;
 }
 
-hipGraphExec_t BatchImpl::segment_graph(const void* kernel, unsigned grid, unsigned lds, const StepParams& S,
+hipGraphExec_t BatchImpl::segment_graph(const void* kernel, unsigned grid, const StepShape& sh, const StepParams& S,
 										uint64_t count) {
 	SegmentKey k;
 	std::memset(&k, 0, sizeof(k));
 	k.kernel = kernel;
 	k.grid = grid;
-	k.lds = lds;
+	k.lds = sh.lds;
+	k.split = sh.split;
+	k.knot_words = sh.knot_words;
 	k.count = count;
 	k.total = total;
 	k.base_seed = base_seed;
@@ -959,8 +1075,6 @@ hipGraphExec_t BatchImpl::segment_graph(const void* kernel, unsigned grid, unsig
 	std::memcpy(k.ptr, ptrs, sizeof(ptrs));
 	k.S = S;
 	k.S.step = 0;
-	k.T = *tables;
-	k.types = types;
 	const uint8_t* kb = reinterpret_cast<const uint8_t*>(&k);
 	std::vector<uint8_t> key(kb, kb + sizeof(k));
 	for (const SegmentGraph& g : graphs)
@@ -977,10 +1091,10 @@ hipGraphExec_t BatchImpl::segment_graph(const void* kernel, unsigned grid, unsig
 		StepParams Sj = S;
 		Sj.step = uint32_t(j);
 		const int c = (cur + int(j & 1)) & 1;
-		kern<<<grid, kBatchBlock, lds, capture_stream>>>(pos[c].data(), pos[1 - c].data(), mom.data(), force.data(),
-														  total, rep_of_slot.data(),
-														  reinterpret_cast<const RepGeom*>(geom.data()), L, *tables,
-														  knots.data(), types, Sj, base_seed, 0, step_word.data());
+		kern<<<grid, sh.block, sh.lds, capture_stream>>>(
+			pos[c].data(), pos[1 - c].data(), mom.data(), force.data(), total, rep_of_slot.data(),
+			reinterpret_cast<const RepGeom*>(geom.data()), L, reinterpret_cast<const BatchConsts*>(consts.data()),
+			knots.data(), Sj, base_seed, 0, step_word.data(), sh.split, sh.knot_words);
 		err = hipGetLastError();
 	}
 	hipGraph_t graph = nullptr;
@@ -1009,15 +1123,9 @@ void BatchImpl::launch_steps(const marsmd_run_params& P, uint64_t first, uint64_
 	const bool bd = P.integrator == MARSMD_INTEGRATOR_BROWNIAN;
 	const bool energy = count == 1 && P.energy_period > 0 && first % P.energy_period == 0;
 	const bool an = (tables->enabled & kAnalyticTerms) != 0;
-	const StepKernel kern =
-		bd ? (energy ? (an ? k_b_step<MARSMD_INTEGRATOR_BROWNIAN, true, true> : k_b_step<MARSMD_INTEGRATOR_BROWNIAN, true, false>)
-					 : (an ? k_b_step<MARSMD_INTEGRATOR_BROWNIAN, false, true>
-						   : k_b_step<MARSMD_INTEGRATOR_BROWNIAN, false, false>))
-		   : (energy ? (an ? k_b_step<MARSMD_INTEGRATOR_LANGEVIN, true, true> : k_b_step<MARSMD_INTEGRATOR_LANGEVIN, true, false>)
-					 : (an ? k_b_step<MARSMD_INTEGRATOR_LANGEVIN, false, true>
-						   : k_b_step<MARSMD_INTEGRATOR_LANGEVIN, false, false>));
-	const unsigned grid = step_grid(reinterpret_cast<const void*>(kern));
-	const unsigned lds = tables->lds ? unsigned(std::max(tables->total_knots, 2)) * 4u : 0u;
+	const StepShape sh = step_shape();
+	const StepKernel kern = pick_b_step(sh.split > 0, bd, energy, an);
+	const unsigned grid = step_grid(reinterpret_cast<const void*>(kern), sh);
 	StepParams S{};
 	S.cut_d = cutoff_threshold(P.cutoff > 0.0f ? P.cutoff * P.cutoff : 0.0f);
 	S.dt = P.timestep;
@@ -1029,7 +1137,7 @@ void BatchImpl::launch_steps(const marsmd_run_params& P, uint64_t first, uint64_
 	// a segment replays when the launches differ only in their step: no forces kept,
 	// and the deferred-kick state settled (Langevin defers from its first step on)
 	const bool replay = use_graph && count >= 2 && !store && (bd || deferred_kick);
-	hipGraphExec_t exec = replay ? segment_graph(reinterpret_cast<const void*>(kern), grid, lds, S, count) : nullptr;
+	hipGraphExec_t exec = replay ? segment_graph(reinterpret_cast<const void*>(kern), grid, sh, S, count) : nullptr;
 	if (timing) {
 		while (timing_events.size() < timing_used + 2) {
 			hipEvent_t e;
@@ -1050,9 +1158,10 @@ void BatchImpl::launch_steps(const marsmd_run_params& P, uint64_t first, uint64_
 			S.step = uint32_t(first + j);
 			S.deferred = deferred_kick ? 1 : 0;
 			const int keep = store && j + 1 == count ? 1 : 0;
-			kern<<<grid, kBatchBlock, lds, s>>>(pos[cur].data(), pos[1 - cur].data(), mom.data(), force.data(), total,
-												 rep_of_slot.data(), reinterpret_cast<const RepGeom*>(geom.data()), L,
-												 *tables, knots.data(), types, S, base_seed, keep, nullptr);
+			kern<<<grid, sh.block, sh.lds, s>>>(pos[cur].data(), pos[1 - cur].data(), mom.data(), force.data(), total,
+												rep_of_slot.data(), reinterpret_cast<const RepGeom*>(geom.data()), L,
+												reinterpret_cast<const BatchConsts*>(consts.data()), knots.data(), S,
+												base_seed, keep, nullptr, sh.split, sh.knot_words);
 			MMD_LAUNCH_CHECK();
 			if (!bd)
 				deferred_kick = true;
@@ -1108,7 +1217,8 @@ void BatchImpl::autotune(const marsmd_run_params& P, uint64_t first_step, uint64
 	// candidates: workgroups per CU from the occupancy down, each with and without
 	// segment replay; results do not depend on them (each particle's step is one lane's
 	// work, and a replay launches the same kernels with the same arguments)
-	(void)step_grid(reinterpret_cast<const void*>(k_b_step<MARSMD_INTEGRATOR_BROWNIAN, false, false>));
+	const StepShape sh = step_shape();
+	(void)step_grid(reinterpret_cast<const void*>(pick_b_step(sh.split > 0, true, false, false)), sh);
 	std::vector<int> per_cu = {occupancy};
 	for (int v : {occupancy - 1, occupancy / 2, 1})
 		if (v >= 1 && std::find(per_cu.begin(), per_cu.end(), v) == per_cu.end())

@@ -24,6 +24,7 @@ struct BatchImpl {
 	marsmd_particle_types types{};
 	NbTables* tables = nullptr;
 	DevArray<float> knots;
+	DevArray<uint8_t> consts; // the step kernels' tables and types in device memory
 	// state in slot order: replica r owns slots [off_r, off_r + n_r), Morton order within
 	DevArray<float4> pos[2], mom, force, snap;
 	int cur = 0;
@@ -61,8 +62,10 @@ struct BatchImpl {
 	std::vector<uint64_t> ref_max_pairs; // per replica: Pairlist::max_pairs_ bookkeeping
 	std::vector<uint64_t> rep_pairs_host;
 	uint8_t* staging = nullptr;   // pinned: the geometry and item offsets of a build's uploads
-	uint64_t* readback = nullptr; // pinned: the walk's statistics (3 words), then the replicas' pair counts
-	DevArray<unsigned long long> rep_pairs;
+	bool geom_uploaded = false;   // the device holds the plan's geometry
+	// pinned words that kernels write: a build's flags (or a displacement), then each
+	// replica's entries and longest row
+	uint64_t* readback = nullptr;
 	int rep_bits = 1;
 	float built_cutoff = 0.0f;
 	bool built = false, prepared = false, deferred_kick = false;
@@ -72,7 +75,8 @@ struct BatchImpl {
 	std::vector<hipEvent_t> timing_events;
 	std::vector<uint64_t> timing_steps;
 	size_t timing_used = 0;
-	int occupancy = 0, num_cus = 0;
+	int occupancy = 0, num_cus = 0; // of the step kernel launched with
+	unsigned occupancy_lds = 0, occupancy_block = 0;
 	// launch configuration: persistent step-kernel workgroups per CU (0: as many as
 	// fit) and whether runs of steps that need no host decision replay as hipGraphs
 	int blocks_per_cu = 0;
@@ -129,11 +133,18 @@ struct BatchImpl {
 	double walk_ms(hipStream_t s);
 	void build(float pairlist_cutoff, bool relabel, hipStream_t s);
 	bool needs_rebuild(float skin, hipStream_t s);
-	unsigned step_grid(const void* kernel);
+	// The step kernel's launch shape with the current list.
+	struct StepShape {
+		uint64_t tiles = 0;
+		unsigned block = 0, lds = 0;
+		uint32_t split = 0, knot_words = 0;
+	};
+	StepShape step_shape() const;
+	unsigned step_grid(const void* kernel, const StepShape& shape);
 	// count consecutive steps from `first` with the current list; `store` keeps the
 	// forces of the last one
 	void launch_steps(const marsmd_run_params& p, uint64_t first, uint64_t count, bool store, hipStream_t s);
-	hipGraphExec_t segment_graph(const void* kernel, unsigned grid, unsigned lds, const StepParams& S,
+	hipGraphExec_t segment_graph(const void* kernel, unsigned grid, const StepShape& shape, const StepParams& S,
 								 uint64_t count);
 	void clear_graphs();
 };
