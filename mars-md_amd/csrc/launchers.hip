@@ -197,13 +197,10 @@ __global__ __launch_bounds__(kPairBlock) void k_pairwise(const int2* __restrict_
 }
 
 // TabulatedBondComputer (BondComputer.h:163-191).
-__global__ void k_bonds(const int2* __restrict__ bonds, const float4* __restrict__ pos, float4* fe,
-						const marsmd_table* __restrict__ tables, const int32_t* __restrict__ tidx,
-						const int32_t* __restrict__ forms, DevBox box, int get_energy, uint64_t nb,
-						float4* __restrict__ contrib) {
-	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (i >= nb)
-		return;
+__device__ __forceinline__ void bond_term(uint64_t i, const int2* __restrict__ bonds, const float4* __restrict__ pos,
+										   float4* fe, const marsmd_table* __restrict__ tables,
+										   const int32_t* __restrict__ tidx, const int32_t* __restrict__ forms,
+										   DevBox box, int get_energy, float4* __restrict__ contrib) {
 	if (forms && forms[i] != MARSMD_FORM_TABULATED) {
 		bonded_zero(contrib, 2 * i, 2);
 		return;
@@ -226,6 +223,13 @@ __global__ void k_bonds(const int2* __restrict__ bonds, const float4* __restrict
 	const float h = v.e * 0.5f;
 	bonded_emit(fe, contrib, 2 * i, ij.x, -fx, -fy, -fz, get_energy != 0, h);
 	bonded_emit(fe, contrib, 2 * i + 1, ij.y, fx, fy, fz, get_energy != 0, h);
+}
+__global__ void k_bonds(const int2* __restrict__ bonds, const float4* __restrict__ pos, float4* fe,
+							const marsmd_table* __restrict__ tables, const int32_t* __restrict__ tidx,
+							const int32_t* __restrict__ forms, DevBox box, int get_energy, uint64_t nb) {
+	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (i < nb)
+		bond_term(i, bonds, pos, fe, tables, tidx, forms, box, get_energy, nullptr);
 }
 
 // AngleGeometry + TabulatedAngleComputer (BondGeometry.h:13-45; BondComputer.h:231-268).
@@ -259,13 +263,11 @@ __device__ __forceinline__ void angle_forces(const DevBox& box, const float4& pa
 	third = v.e * float(1.0 / 3.0);
 }
 
-__global__ void k_angles(const int4* __restrict__ angles, const float4* __restrict__ pos, float4* fe,
-						 const marsmd_table* __restrict__ tables, const int32_t* __restrict__ tidx,
-						 const int32_t* __restrict__ forms, DevBox box, int get_energy, uint64_t na,
-						 float4* __restrict__ contrib) {
-	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (i >= na)
-		return;
+__device__ __forceinline__ void angle_term(uint64_t i, const int4* __restrict__ angles,
+										   const float4* __restrict__ pos, float4* fe,
+										   const marsmd_table* __restrict__ tables, const int32_t* __restrict__ tidx,
+										   const int32_t* __restrict__ forms, DevBox box, int get_energy,
+										   float4* __restrict__ contrib) {
 	if (forms && forms[i] != MARSMD_FORM_TABULATED) {
 		bonded_zero(contrib, 3 * i, 3);
 		return;
@@ -278,6 +280,13 @@ __global__ void k_angles(const int4* __restrict__ angles, const float4* __restri
 	bonded_emit(fe, contrib, 3 * i, a.x, f1.x, f1.y, f1.z, e, third);
 	bonded_emit(fe, contrib, 3 * i + 1, a.y, -(f1.x + f3.x), -(f1.y + f3.y), -(f1.z + f3.z), e, third);
 	bonded_emit(fe, contrib, 3 * i + 2, a.z, f3.x, f3.y, f3.z, e, third);
+}
+__global__ void k_angles(const int4* __restrict__ angles, const float4* __restrict__ pos, float4* fe,
+							const marsmd_table* __restrict__ tables, const int32_t* __restrict__ tidx,
+							const int32_t* __restrict__ forms, DevBox box, int get_energy, uint64_t na) {
+	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (i < na)
+		angle_term(i, angles, pos, fe, tables, tidx, forms, box, get_energy, nullptr);
 }
 
 __device__ __forceinline__ float3 cross3(const float3& v, const float3& w) {
@@ -331,13 +340,11 @@ __device__ __forceinline__ void dihedral_forces(const DevBox& box, const float4&
 	quarter = v.e * 0.25f;
 }
 
-__global__ void k_dihedrals(const int4* __restrict__ dih, const float4* __restrict__ pos, float4* fe,
-							const marsmd_table* __restrict__ tables, const int32_t* __restrict__ tidx,
-							const int32_t* __restrict__ forms, DevBox box, int get_energy, uint64_t nd,
-							float4* __restrict__ contrib) {
-	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (i >= nd)
-		return;
+__device__ __forceinline__ void dihedral_term(uint64_t i, const int4* __restrict__ dih,
+										   const float4* __restrict__ pos, float4* fe,
+										   const marsmd_table* __restrict__ tables, const int32_t* __restrict__ tidx,
+										   const int32_t* __restrict__ forms, DevBox box, int get_energy,
+										   float4* __restrict__ contrib) {
 	if (forms && forms[i] != MARSMD_FORM_TABULATED) {
 		bonded_zero(contrib, 4 * i, 4);
 		return;
@@ -351,16 +358,21 @@ __global__ void k_dihedrals(const int4* __restrict__ dih, const float4* __restri
 	for (int k = 0; k < 4; ++k)
 		bonded_emit(fe, contrib, 4 * i + uint64_t(k), idx[k], f[k].x, f[k].y, f[k].z, get_energy != 0, quarter);
 }
+__global__ void k_dihedrals(const int4* __restrict__ dih, const float4* __restrict__ pos, float4* fe,
+							const marsmd_table* __restrict__ tables, const int32_t* __restrict__ tidx,
+							const int32_t* __restrict__ forms, DevBox box, int get_energy, uint64_t nd) {
+	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (i < nd)
+		dihedral_term(i, dih, pos, fe, tables, tidx, forms, box, get_energy, nullptr);
+}
 
 // HarmonicRestraintComputer (BondComputer.h:109-129) with CalcDistance
 // (Interactions.h:42-53) and the harmonic form AnalyticalForceComputer<0>
 // (Bonded/Analytical.h:18-30) at r0 = 0: F = unit(wrap_diff(x - x0)) * (-k d), full U.
-__global__ void k_restraints(const int32_t* __restrict__ ids, const float4* __restrict__ pos, float4* fe,
-							 const float4* __restrict__ anchors, const float* __restrict__ kspring, DevBox box,
-							 int get_energy, uint64_t nr, float4* __restrict__ contrib) {
-	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (i >= nr)
-		return;
+__device__ __forceinline__ void restraint_term(uint64_t i, const int32_t* __restrict__ ids,
+										   const float4* __restrict__ pos, float4* fe,
+										   const float4* __restrict__ anchors, const float* __restrict__ kspring,
+										   DevBox box, int get_energy, float4* __restrict__ contrib) {
 	const int id = ids[i];
 	if (id < 0) {
 		bonded_zero(contrib, i, 1);
@@ -377,6 +389,49 @@ __global__ void k_restraints(const int32_t* __restrict__ ids, const float4* __re
 	const float dr = d - 0.0f;
 	const float force = -k * dr;
 	bonded_emit(fe, contrib, i, id, u.x * force, u.y * force, u.z * force, get_energy != 0, 0.5f * k * dr * dr);
+}
+__global__ void k_restraints(const int32_t* __restrict__ ids, const float4* __restrict__ pos, float4* fe,
+							const float4* __restrict__ anchors, const float* __restrict__ kspring, DevBox box,
+							int get_energy, uint64_t nr) {
+	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (i < nr)
+		restraint_term(i, ids, pos, fe, anchors, kspring, box, get_energy, nullptr);
+}
+
+// Every bonded term of a Patch in one launch, its shares stored (see launch_bonded_shares):
+// workgroups in the kinds' order, each kind's last one partly idle. Bound by the latency of
+// one term's loads (a launch per kind pays it once each): 99800 bonds and 99600 angles
+// 5.1 + 5.4 us as two launches, 6.7 us as one.
+__global__ __launch_bounds__(256) void k_bonded_shares(BondedTerms B, const float4* __restrict__ pos, DevBox box,
+													   int get_energy, float4* __restrict__ shares) {
+	uint64_t i = uint64_t(blockIdx.x) * 256u + threadIdx.x;
+	const uint64_t gb = (B.nb + 255) / 256 * 256, ga = (B.na + 255) / 256 * 256, gd = (B.nd + 255) / 256 * 256;
+	if (i < gb) {
+		if (i < B.nb)
+			bond_term(i, reinterpret_cast<const int2*>(B.bonds), pos, nullptr, B.bond_tables, B.bond_table, nullptr,
+					  box, get_energy, shares);
+		return;
+	}
+	i -= gb;
+	shares += 2 * B.nb;
+	if (i < ga) {
+		if (i < B.na)
+			angle_term(i, reinterpret_cast<const int4*>(B.angles), pos, nullptr, B.angle_tables, B.angle_table, nullptr,
+					   box, get_energy, shares);
+		return;
+	}
+	i -= ga;
+	shares += 3 * B.na;
+	if (i < gd) {
+		if (i < B.nd)
+			dihedral_term(i, reinterpret_cast<const int4*>(B.dihedrals), pos, nullptr, B.dihedral_tables,
+						  B.dihedral_table, nullptr, box, get_energy, shares);
+		return;
+	}
+	i -= gd;
+	shares += 4 * B.nd;
+	if (i < B.nr)
+		restraint_term(i, B.restraints, pos, nullptr, B.anchors, B.springs, box, get_energy, shares);
 }
 
 // BDIntegrate::operator() (BD.h:44-92).
@@ -564,47 +619,59 @@ void launch_analytical_pair_nonbonded(const int32_t* pairs, const float* pos, fl
 
 void launch_tabulated_bonds(const int32_t* bonds, const float* pos, float* fe, const marsmd_table* tables,
 							const int32_t* tidx, const int32_t* forms, const marsmd_box& box, bool energy,
-							uint64_t nb, hipStream_t s, float4* contrib) {
+							uint64_t nb, hipStream_t s) {
 	if (nb == 0)
 		return;
 	k_bonds<<<grid_for(nb, 256), 256, 0, s>>>(reinterpret_cast<const int2*>(bonds),
 											   reinterpret_cast<const float4*>(pos), reinterpret_cast<float4*>(fe),
-											   tables, tidx, forms, make_devbox(box), energy ? 1 : 0, nb, contrib);
+											   tables, tidx, forms, make_devbox(box), energy ? 1 : 0, nb);
 	MMD_LAUNCH_CHECK();
 }
 
 void launch_tabulated_angles(const int32_t* angles, const float* pos, float* fe, const marsmd_table* tables,
 							 const int32_t* tidx, const int32_t* forms, const marsmd_box& box, bool energy,
-							 uint64_t na, hipStream_t s, float4* contrib) {
+							 uint64_t na, hipStream_t s) {
 	if (na == 0)
 		return;
 	k_angles<<<grid_for(na, 256), 256, 0, s>>>(reinterpret_cast<const int4*>(angles),
 												reinterpret_cast<const float4*>(pos), reinterpret_cast<float4*>(fe),
-												tables, tidx, forms, make_devbox(box), energy ? 1 : 0, na, contrib);
+												tables, tidx, forms, make_devbox(box), energy ? 1 : 0, na);
 	MMD_LAUNCH_CHECK();
 }
 
 void launch_tabulated_dihedrals(const int32_t* dihedrals, const float* pos, float* fe, const marsmd_table* tables,
 								const int32_t* tidx, const int32_t* forms, const marsmd_box& box, bool energy,
-								uint64_t nd, hipStream_t s, float4* contrib) {
+								uint64_t nd, hipStream_t s) {
 	if (nd == 0)
 		return;
 	k_dihedrals<<<grid_for(nd, 256), 256, 0, s>>>(reinterpret_cast<const int4*>(dihedrals),
 												   reinterpret_cast<const float4*>(pos),
 												   reinterpret_cast<float4*>(fe), tables, tidx, forms,
-												   make_devbox(box), energy ? 1 : 0, nd, contrib);
+												   make_devbox(box), energy ? 1 : 0, nd);
 	MMD_LAUNCH_CHECK();
 }
 
 void launch_harmonic_restraints(const int32_t* ids, const float* pos, float* fe, const float* anchors,
 								const float* kspring, const marsmd_box& box, bool energy, uint64_t nr,
-								hipStream_t s, float4* contrib) {
+								hipStream_t s) {
 	if (nr == 0)
 		return;
 	k_restraints<<<grid_for(nr, 256), 256, 0, s>>>(ids, reinterpret_cast<const float4*>(pos),
 													reinterpret_cast<float4*>(fe),
 													reinterpret_cast<const float4*>(anchors), kspring,
-													make_devbox(box), energy ? 1 : 0, nr, contrib);
+													make_devbox(box), energy ? 1 : 0, nr);
+	MMD_LAUNCH_CHECK();
+}
+
+void launch_bonded_shares(const BondedTerms& B, const float* pos, const marsmd_box& box, bool energy, float4* shares,
+						  hipStream_t s) {
+	uint64_t blocks = 0;
+	for (uint64_t k : {B.nb, B.na, B.nd, B.nr})
+		blocks += (k + 255) / 256;
+	if (blocks == 0)
+		return;
+	k_bonded_shares<<<grid_for(blocks * 256, 256), 256, 0, s>>>(B, reinterpret_cast<const float4*>(pos),
+																make_devbox(box), energy ? 1 : 0, shares);
 	MMD_LAUNCH_CHECK();
 }
 

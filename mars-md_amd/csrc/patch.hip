@@ -557,7 +557,7 @@ __global__ void k_gather_state(const uint32_t* __restrict__ sidx, const uint32_t
 
 // canonical -> slot remap of bonded index tuples (stride ints per term, first k used).
 // ------------------------------------------------------------------ bonded gather
-// The bonded terms' shares (the launchers' contribution slots: bonds 2 per term, then
+// The bonded terms' shares (launch_bonded_shares' order: bonds 2 per term, then
 // angles 3, dihedrals 4, restraints 1) as (slot of the particle, share index) pairs,
 // for a stable sort by slot: each particle's shares then sit in share-index order.
 __global__ void k_share_keys(const int32_t* __restrict__ bonds, uint64_t nb, const int32_t* __restrict__ angles,
@@ -1168,24 +1168,24 @@ void PatchImpl::calculate_bonded(bool energy, hipStream_t s, bool add) {
 		raise(MARSMD_ERR_RUNTIME, "Patch: calculate_bonded_forces before the first nonbonded pass");
 	const uint64_t q = num_shares();
 	shares.resize(q);
-	float4* c = shares.data();
-	const float* p = reinterpret_cast<const float*>(pos[cur].data());
-	if (num_bonds)
-		launch_tabulated_bonds(bonds_slot.data(), p, nullptr, tables->bond_dev.data(), bond_table.data(), nullptr, box,
-							   energy, num_bonds, s, c);
-	c += 2 * num_bonds;
-	if (num_angles)
-		launch_tabulated_angles(angles_slot.data(), p, nullptr, tables->angle_dev.data(), angle_table.data(), nullptr,
-								box, energy, num_angles, s, c);
-	c += 3 * num_angles;
-	if (num_dihedrals)
-		launch_tabulated_dihedrals(dihedrals_slot.data(), p, nullptr, tables->dihedral_dev.data(),
-								   dihedral_table.data(), nullptr, box, energy, num_dihedrals, s, c);
-	c += 4 * num_dihedrals;
-	if (num_restraints)
-		launch_harmonic_restraints(restraint_slot.data(), p, nullptr,
-								   reinterpret_cast<const float*>(restraint_anchor.data()), restraint_k.data(), box,
-								   energy, num_restraints, s, c);
+	BondedTerms B{};
+	B.nb = num_bonds;
+	B.na = num_angles;
+	B.nd = num_dihedrals;
+	B.nr = num_restraints;
+	B.bonds = bonds_slot.data();
+	B.angles = angles_slot.data();
+	B.dihedrals = dihedrals_slot.data();
+	B.restraints = restraint_slot.data();
+	B.bond_tables = tables->bond_dev.data();
+	B.angle_tables = tables->angle_dev.data();
+	B.dihedral_tables = tables->dihedral_dev.data();
+	B.bond_table = bond_table.data();
+	B.angle_table = angle_table.data();
+	B.dihedral_table = dihedral_table.data();
+	B.anchors = restraint_anchor.data();
+	B.springs = restraint_k.data();
+	launch_bonded_shares(B, reinterpret_cast<const float*>(pos[cur].data()), box, energy, shares.data(), s);
 	k_bonded_gather<<<grid_for(n, 256), 256, 0, s>>>(n, share_begin.data(), share_end.data(), share_vals.data() + q,
 													  shares.data(), add ? 1 : 0, force.data());
 	MMD_LAUNCH_CHECK();
