@@ -267,7 +267,8 @@ __global__ __launch_bounds__(kFmAdjBlock) void k_fm_adjoint_rec(const FmSnapView
 }
 
 // seg[y][k] = sum of partial[b][k] over the rows b of segment y (rows in order), then
-// out[k] = sum of seg[y][k] over the segments in order.
+// out[k] = sum of seg[y][k] over the segments in order. Bound by the latency of their loads,
+// which all go out before the additions: 12.6 + 11 -> 6.9 + 4.7 us at 512 rows of 5120 sums.
 constexpr uint32_t kFmSegs = 32;
 __global__ void k_fm_reduce_rows(const double* __restrict__ partial, uint32_t blocks, uint32_t total,
 								 double* __restrict__ seg) {
@@ -278,8 +279,16 @@ __global__ void k_fm_reduce_rows(const double* __restrict__ partial, uint32_t bl
 	const uint32_t per = (blocks + kFmSegs - 1) / kFmSegs;
 	const uint32_t b0 = y * per, b1 = min(blocks, b0 + per);
 	double s = 0.0;
-	for (uint32_t b = b0; b < b1; ++b)
-		s += partial[uint64_t(b) * total + k];
+	for (uint32_t b = b0; b < b1; b += 8) { // eight loads in flight, added in order
+		double v[8];
+#pragma unroll
+		for (uint32_t u = 0; u < 8; ++u)
+			v[u] = partial[uint64_t(min(b + u, b1 - 1u)) * total + k];
+#pragma unroll
+		for (uint32_t u = 0; u < 8; ++u)
+			if (b + u < b1)
+				s += v[u];
+	}
 	seg[uint64_t(y) * total + k] = s;
 }
 // out[k] = S[k] - S[k - 1], S[k] the sum of seg[y][k] over the segments in order.
@@ -287,12 +296,22 @@ __global__ void k_fm_reduce_segs(const double* __restrict__ seg, uint32_t total,
 	const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
 	if (k >= total)
 		return;
-	double s = 0.0, sp = 0.0;
+	// every load in flight before the first addition
+	const uint32_t kp = k > 0 ? k - 1u : 0u;
+	double a[kFmSegs], b[kFmSegs];
+#pragma unroll
 	for (uint32_t y = 0; y < kFmSegs; ++y) {
-		s += seg[uint64_t(y) * total + k];
-		if (k > 0)
-			sp += seg[uint64_t(y) * total + k - 1];
+		a[y] = seg[uint64_t(y) * total + k];
+		b[y] = seg[uint64_t(y) * total + kp];
 	}
+	double s = 0.0, sp = 0.0;
+#pragma unroll
+	for (uint32_t y = 0; y < kFmSegs; ++y) {
+		s += a[y];
+		sp += b[y];
+	}
+	if (k == 0)
+		sp = 0.0;
 	out[k] = s - sp;
 }
 
