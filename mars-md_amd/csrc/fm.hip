@@ -268,7 +268,8 @@ __global__ __launch_bounds__(kFmAdjBlock) void k_fm_adjoint_rec(const FmSnapView
 
 // seg[y][k] = sum of partial[b][k] over the rows b of segment y (rows in order), then
 // out[k] = sum of seg[y][k] over the segments in order. Bound by the latency of their loads,
-// which all go out before the additions: 12.6 + 11 -> 6.9 + 4.7 us at 512 rows of 5120 sums.
+// which all go out before the additions: 12.6 + 11 -> 6.9 + 4.7 us for the
+// 5120 sums of 64 x 100k beads.
 constexpr uint32_t kFmSegs = 32;
 __global__ void k_fm_reduce_rows(const double* __restrict__ partial, uint32_t blocks, uint32_t total,
 								 double* __restrict__ seg) {
