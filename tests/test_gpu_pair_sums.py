@@ -5,6 +5,9 @@ import pytest
 
 import marsmd
 from marsmd import PeriodicBox
+from oracle import pyoracle as orc
+from tests.conftest import rel_force_error
+from tests.test_gpu_analytical_terms import ANALYTIC, FORCE_TOL, _launch_inputs, analytic_spec
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +58,24 @@ def test_long_lists_sum_to_their_parts(cuda, order, count):
     bound = 2.0 * 2.0**-24 * total[:, 2:] * total[:, [0, 0, 0, 1]]
     assert bool(((whole - parts).abs() <= bound).all())
     assert float(whole[:, 3].sum()) > 0.0
+
+
+@pytest.mark.parametrize("terms", [ANALYTIC, ANALYTIC | marsmd._capi.PAIR_TERM_TABULATED])
+def test_long_lists_with_analytical_terms_match_the_oracle(cuda, terms):
+    spec = analytic_spec(n=3000, L=110.0, seed=9)
+    pos, pairs, tags, pd, td, tag_d = _launch_inputs(cuda, spec)
+    assert len(pairs) >= 1 << 18
+    fe = cuda.zeros((len(pos), 4), dtype=cuda.float32, device="cuda")
+    pos_d, cut2 = cuda.from_numpy(pos).cuda(), spec.params.cutoff ** 2
+    if terms == ANALYTIC:
+        marsmd.launch_analytical_pair_nonbonded(pd, pos_d, fe, td, tag_d, spec.types, spec.box, terms, True,
+                                                len(pairs), cut2, params=spec.pair_params)
+    else:
+        view = marsmd.particle_view(pos=pos_d, force_energy=fe, type_id=td)
+        marsmd.launch_pairwise_nonbonded(pd, view, tag_d, marsmd.DeviceTables(spec.nb_tables), spec.box, True,
+                                         len(pairs), cut2, terms, types=spec.types, params=spec.pair_params)
+    ref = orc.pair_forces(pairs, pos, spec.type_ids, tags, spec.nb_tables, spec.box, cut2, mode=1,
+                          enabled_terms=terms, particle_types=spec.types, pair_params=spec.pair_params)
+    g = fe.cpu().numpy()
+    assert rel_force_error(g, ref) <= FORCE_TOL
+    assert abs(g[:, 3].sum() - ref[:, 3].sum()) <= 1e-5 * np.abs(ref[:, 3]).sum()
