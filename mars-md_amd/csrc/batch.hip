@@ -719,7 +719,8 @@ void BatchImpl::copy_from_host(const float* pos4, const float* mom4, const int32
 	if (mom4)
 		MMD_HIP(hipMemcpy(hm.data(), mom4, 16 * total, hipMemcpyHostToDevice));
 	MMD_HIP(hipMemcpy(ht.data(), type_ids, 4 * total, hipMemcpyHostToDevice));
-	// geometry needs only the boxes here; the build fills the rest
+	// the import needs only the boxes: the next build uploads the planned geometry again
+	geom_uploaded = false;
 	std::vector<RepGeom> G(R);
 	for (uint64_t r = 0; r < R; ++r) {
 		G[r].box = make_devbox(boxes[r]);
@@ -891,7 +892,6 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 		MMD_HIP(hipMemcpyAsync(geom.data(), staging, gbytes, hipMemcpyHostToDevice, s));
 		item_off.resize(R + 1);
 		MMD_HIP(hipMemcpyAsync(item_off.data(), staging + gbytes, 4 * (R + 1), hipMemcpyHostToDevice, s));
-		geom_uploaded = true;
 	}
 	const RepGeom* gd = reinterpret_cast<const RepGeom*>(geom.data());
 	// sort: Morton key (stable; ties by canonical index), then replica (stable)
@@ -979,6 +979,7 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 												  reinterpret_cast<unsigned long long*>(readback));
 		MMD_LAUNCH_CHECK();
 		MMD_HIP(hipStreamSynchronize(s));
+		geom_uploaded = true;
 		if (readback[0] & 1u)
 			raise(MARSMD_ERR_VALUE, "batch: a particle left its replica's box (positions must stay wrapped)");
 		if (readback[0] & 2u)

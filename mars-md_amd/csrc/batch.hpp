@@ -62,7 +62,7 @@ struct BatchImpl {
 	std::vector<uint64_t> ref_max_pairs; // per replica: Pairlist::max_pairs_ bookkeeping
 	std::vector<uint64_t> rep_pairs_host;
 	uint8_t* staging = nullptr;   // pinned: the geometry and item offsets of a build's uploads
-	bool geom_uploaded = false;   // the device holds the plan's geometry
+	bool geom_uploaded = false;   // the device holds the plan's geometry (a build's wait was reached)
 	// pinned words that kernels write: a build's flags (or a displacement), then each
 	// replica's entries and longest row
 	uint64_t* readback = nullptr;
