@@ -174,6 +174,7 @@ marsmd_status marsmd_pairlist_set_exclusions(marsmd_pairlist* pl, const marsmd_e
 	return guard([&] {
 		need(pl, "pairlist");
 		pl->impl->excl = view ? *view : marsmd_exclusion_view{};
+		pl->impl->excl_symmetric = false; // a caller's rows, also on a Patch's pairlist
 	});
 }
 marsmd_status marsmd_pairlist_set_max_pairs_ceiling(marsmd_pairlist* pl, uint64_t ceiling) {
@@ -189,6 +190,7 @@ marsmd_status marsmd_pairlist_build(marsmd_pairlist* pl, const float* pos4, cons
 		need(pl, "pairlist");
 		if (n)
 			need(pos4, "positions");
+		pl->impl->excl_symmetric = false; // rows may name particles that are not in this call
 		pl->impl->build(reinterpret_cast<const float4*>(pos4), nullptr, false, type_ids, n, pairlist_cutoff,
 						st(stream));
 	});

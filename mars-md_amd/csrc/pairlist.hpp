@@ -97,7 +97,9 @@ struct PairlistImpl {
 	// least home_target particles on average, candidate cells fine_offset levels below
 	int home_target = 24, fine_offset = 2;
 	bool cells_auto = true;         // neither set nor tuned: walk_level chooses
-	bool excl_symmetric = false;    // every exclusion is in both ends' rows (the Patch's own CSR)
+	// every exclusion is in both ends' rows and names a particle of the build: set by the
+	// Patch for its own CSR and builds only
+	bool excl_symmetric = false;
 	// the home walk's fine-cell stencil: Morton codes in a wholly periodic box, else offsets
 	DevArray<uint32_t> stencil_codes;
 	DevArray<int4> stencil_dev;
