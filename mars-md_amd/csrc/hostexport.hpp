@@ -41,9 +41,10 @@ static __global__ void k_export(const float4* __restrict__ pos, const float4* __
 // the link, while worker threads copy earlier pieces into the caller's arrays. The copies
 // are the larger part (fresh arrays are faulted in and cleared page by page by the thread
 // that first writes them), so they are shared by several threads. The staging memory, at
-// most kSlots pieces (14.7 MB), stays with the object. A call into fresh arrays, against a
-// kernel into five device arrays allocated for it and their copies into pageable memory:
-// 500 particles 97 -> 18 us, 10^5 428 -> 335 us, 10^6 4.4 -> 2.5 ms, 2.6 10^6 16.0 -> 5.6 ms
+// most kSlots pieces (14.7 MB), stays with the object and serves one call at a time (host
+// threads that read one object take turns). A call into fresh arrays, against a kernel into
+// five device arrays allocated for it and their copies into pageable memory: 500 particles
+// 97 -> 18 us, 10^5 428 -> 335 us, 10^6 4.4 -> 2.5 ms, 2.6 10^6 16.0 -> 5.6 ms
 // (147 MB: 26 GB/s). With 1, 2, 4, 6, 8 threads the last took 12.8, 8.1, 5.6, 5.0, 5.3 ms
 // and 10^6 particles 4.0, 3.5, 2.7, 3.1, 3.5 ms.
 class HostExport {
@@ -67,6 +68,7 @@ public:
 	// staging records on the null stream.
 	template<class Launch>
 	void copy(uint64_t n, const ParticleRecords& out, Launch&& launch) {
+		const std::lock_guard<std::mutex> one_call(calls);
 		const uint64_t pieces = (n + kPiece - 1) / kPiece, slots = std::min(pieces, kSlots);
 		reserve(std::min(n, kPiece), slots);
 		const auto count = [&](uint64_t i) { return std::min(kPiece, n - i * kPiece); };
@@ -166,6 +168,7 @@ private:
 		}
 	};
 
+	std::mutex calls;
 	char* staging = nullptr;
 	uint64_t piece = 0, have = 0; // particles of a slot, slots
 	std::vector<hipEvent_t> events;
