@@ -501,8 +501,8 @@ marsmd_status marsmd_patch_set_kernel_timing(marsmd_patch* p, int32_t enable);
 marsmd_status marsmd_patch_get_kernel_timing(marsmd_patch* p, double* total_ms, uint64_t* launches);
 
 /* Launch configuration of marsmd_patch_run's step (no counterpart in the reference).
- * Results do not depend on it: each particle's step is one lane's work whatever the
- * grid, and a precomputed position-dependent force is the same function of the same
+ * Results do not depend on it: each particle's sums are taken in the same order whatever
+ * lanes and workgroups take them, and a precomputed position-dependent force is the same function of the same
  * inputs. With split_pmf, the timing events above bracket both kernels of a step. */
 typedef struct marsmd_patch_launch {
     int32_t blocks_per_cu; /* persistent step-kernel workgroups per CU; 0: as many as fit */

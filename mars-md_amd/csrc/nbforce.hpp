@@ -252,14 +252,18 @@ struct RowHead { // what a lane reads before its first pair term
 	const uint4* row;
 	uint4 j, self; // its first group's entries; the slot itself four times
 };
-// (a slot past the end stands in as the last slot with an empty row)
-__device__ __forceinline__ RowHead row_head(uint32_t slot, uint32_t n, uint32_t sub, const float4* __restrict__ pos,
-											const NbrList& L) {
-	const uint32_t t = min(slot, n - 1u);
+// The head of lane position `at`: its slot is lane_slot[at] (NULL: the position itself) and
+// its row is L's at the position (`placed`: rows in lane order) or at the slot. A position
+// past the end stands in as the last one with an empty row.
+__device__ __forceinline__ RowHead row_head(uint32_t at, uint32_t n, uint32_t sub, const float4* __restrict__ pos,
+											const NbrList& L, const uint32_t* __restrict__ lane_slot = nullptr,
+											bool placed = true) {
+	const uint32_t l = min(at, n - 1u);
+	const uint32_t t = lane_slot ? lane_slot[l] : l, r = placed ? l : t;
 	RowHead h;
 	h.p = pos[t];
-	h.ng = slot < n ? (L.count[t] + 3u) >> 2 : 0u;
-	h.row = reinterpret_cast<const uint4*>(L.nbr + L.tile_base[t >> 6]) + (t & 63u);
+	h.ng = at < n ? (L.count[r] + 3u) >> 2 : 0u;
+	h.row = reinterpret_cast<const uint4*>(L.nbr + L.tile_base[r >> 6]) + (r & 63u);
 	h.self = make_uint4(t, t, t, t);
 	h.j = h.self;
 	if (sub < h.ng)

@@ -435,13 +435,14 @@ __global__ __launch_bounds__(kBlock, PMF == kPmfCubic ? 4 : 5) void k_step(const
 // The fused step with each slot's row dealt to 2^split lanes (nb_force_split): a workgroup
 // sums the pair forces of 512 >> split slots with all its lanes, hands them over in LDS
 // and finishes the slots with its first lanes. The next slots' first row entries are in
-// flight meanwhile, the first ones' while the tables are staged.
-template<int INTEG, bool ENERGY, bool ANALYTIC, int PMF>
+// flight meanwhile, the first ones' while the tables are staged. PRUNE: with pruned rows, as
+// in k_step (a template parameter: asking at run time costs the step of 20k beads 3%).
+template<int INTEG, bool ENERGY, bool ANALYTIC, int PMF, bool PRUNE>
 __global__ __launch_bounds__(kSplitBlock, 4) void k_step_split(
 	const float4* __restrict__ pos, float4* __restrict__ pos_next, float4* __restrict__ mom, float4* __restrict__ force,
 	uint64_t n, NbrList L, const NbTables* __restrict__ T_dev, const float* __restrict__ knots_g, uint32_t knot_words,
 	const marsmd_particle_types* __restrict__ types_dev, const marsmd_grid_view* __restrict__ grids, StepParams S,
-	int has_bonded, int store_force, PruneView PR, uint32_t split) {
+	int has_bonded, int store_force, const float4* __restrict__ pmf_in, PruneView PR, uint32_t split) {
 	extern __shared__ float lds_knots[]; // knot_words words (a multiple of 4), then the handed-over forces
 	__shared__ NbLds lds_nb;
 	__shared__ marsmd_particle_types lds_types;
@@ -456,12 +457,17 @@ __global__ __launch_bounds__(kSplitBlock, 4) void k_step_split(
 	const uint32_t lane = threadIdx.x & 63u;
 	const uint32_t first = (threadIdx.x - lane) >> split; // the wave's first slot of a tile
 	const TileRange R = xcd_tiles(uint32_t((n + per - 1) / per));
+	const bool track = PRUNE && PR.limit2 > 0.0f;
+	bool pruned = PRUNE;
+	if (track && PR.since > 0)
+		pruned = __uint_as_float(PR.disp[(PR.since - 1u) & 3u]) < PR.limit2;
+	const NbrList LL = pruned ? PR.list : L;
+	const uint32_t* const lane_slot = PRUNE ? PR.lane_slot : nullptr;
 	RowHead h{};
 	if (R.tile < R.end)
-		h = row_head(R.tile * per + mine, uint32_t(n), sub, pos, L);
+		h = row_head(R.tile * per + mine, uint32_t(n), sub, pos, LL, lane_slot, pruned || !PRUNE);
 	stage_step<INTEG>(*types_dev, S, lds_types, lds_steps);
 	stage_tables(T, knots_g, lds_knots, lds_nb);
-	const bool track = PR.lane_slot && PR.limit2 > 0.0f;
 	float disp2 = 0.0f;
 	uint32_t turn = 0;
 	for (uint32_t tile = R.tile; tile < R.end; tile += R.stride, turn ^= 1u) {
@@ -472,46 +478,54 @@ __global__ __launch_bounds__(kSplitBlock, 4) void k_step_split(
 		if ((lane >> 2) < (64u >> split))
 			reinterpret_cast<float*>(lds_force)[4u * (turn * per + first + (lane >> 2)) + (lane & 3u)] = f;
 		if (tile + R.stride < R.end)
-			h = row_head((tile + R.stride) * per + mine, uint32_t(n), sub, pos, L);
+			h = row_head((tile + R.stride) * per + mine, uint32_t(n), sub, pos, LL, lane_slot, pruned || !PRUNE);
 		if (PMF == kPmfCubic) // a quad per slot samples the grids
 			for (uint32_t k = threadIdx.x >> 2; k < per && tile * per + k < n; k += kSplitBlock / 4) {
-				const float4 p = pos[tile * per + k];
+				const uint32_t lt = tile * per + k;
+				const float4 p = pos[PRUNE ? lane_slot[lt] : lt];
 				const float4 g = position_dependent_force_t<true, true>(p.x, p.y, p.z, int(meta_type(fb(p.w))), lds_types,
 																		grids, S.ef);
 				if ((threadIdx.x & 3u) == 0u)
 					lds_pmf[turn * per + k] = g;
 			}
 		__syncthreads(); // (the other buffers' readers finished before it)
-		const uint32_t u = tile * per + threadIdx.x;
-		if (threadIdx.x < per && u < n) {
+		const uint32_t lt = tile * per + threadIdx.x; // lane position
+		if (threadIdx.x < per && lt < n) {
+			const uint32_t t = PRUNE ? lane_slot[lt] : lt; // slot
 			const uint32_t at = turn * per + threadIdx.x;
 			const float4 pn = step_finish<INTEG, ENERGY, PMF == kPmfCubic ? kPmfGiven : PMF>(
-				u, pos[u], lds_force[at], mom, force, lds_types, lds_steps, grids, S, has_bonded, store_force,
-				PMF == kPmfCubic ? lds_pmf[at] : float4{});
-			pos_next[u] = pn;
+				t, pos[t], lds_force[at], mom, force, lds_types, lds_steps, grids, S, has_bonded, store_force,
+				PMF == kPmfCubic ? lds_pmf[at] : PMF == kPmfGiven ? pmf_in[t] : float4{});
+			pos_next[t] = pn;
 			if (track)
-				disp2 = fmaxf(disp2, len2(wrap_diff_uniform(S.box, sub3(pn, PR.ref[u]))));
+				disp2 = fmaxf(disp2, len2(wrap_diff_uniform(S.box, sub3(pn, PR.ref[t]))));
 		}
 	}
 	if (track)
 		record_displacement(PR, disp2, lds_red);
 }
 
-using SplitStepFn = decltype(&k_step_split<MARSMD_INTEGRATOR_BROWNIAN, false, false, kPmfNone>);
-template<int I, bool E, bool A>
+using SplitStepFn = decltype(&k_step_split<MARSMD_INTEGRATOR_BROWNIAN, false, false, kPmfNone, false>);
+template<int I, bool E, bool A, bool P>
 SplitStepFn pick_split_pmf(int pmf) {
-	return pmf == kPmfCubic ? k_step_split<I, E, A, kPmfCubic>
-							: pmf == kPmfLinear ? k_step_split<I, E, A, kPmfLinear> : k_step_split<I, E, A, kPmfNone>;
+	return pmf == kPmfGiven		? k_step_split<I, E, A, kPmfGiven, P>
+		   : pmf == kPmfCubic	? k_step_split<I, E, A, kPmfCubic, P>
+		   : pmf == kPmfLinear	? k_step_split<I, E, A, kPmfLinear, P>
+								: k_step_split<I, E, A, kPmfNone, P>;
 }
-template<int I>
+template<int I, bool P>
 SplitStepFn pick_split_i(bool energy, bool an, int pmf) {
 	if (energy)
-		return an ? pick_split_pmf<I, true, true>(pmf) : pick_split_pmf<I, true, false>(pmf);
-	return an ? pick_split_pmf<I, false, true>(pmf) : pick_split_pmf<I, false, false>(pmf);
+		return an ? pick_split_pmf<I, true, true, P>(pmf) : pick_split_pmf<I, true, false, P>(pmf);
+	return an ? pick_split_pmf<I, false, true, P>(pmf) : pick_split_pmf<I, false, false, P>(pmf);
 }
-SplitStepFn pick_split(bool bd, bool energy, bool an, int pmf) {
-	return bd ? pick_split_i<MARSMD_INTEGRATOR_BROWNIAN>(energy, an, pmf)
-			  : pick_split_i<MARSMD_INTEGRATOR_LANGEVIN>(energy, an, pmf);
+template<bool P>
+SplitStepFn pick_split_p(bool bd, bool energy, bool an, int pmf) {
+	return bd ? pick_split_i<MARSMD_INTEGRATOR_BROWNIAN, P>(energy, an, pmf)
+			  : pick_split_i<MARSMD_INTEGRATOR_LANGEVIN, P>(energy, an, pmf);
+}
+SplitStepFn pick_split(bool bd, bool energy, bool an, int pmf, bool prune) {
+	return prune ? pick_split_p<true>(bd, energy, an, pmf) : pick_split_p<false>(bd, energy, an, pmf);
 }
 using StepFn = decltype(&k_step<MARSMD_INTEGRATOR_BROWNIAN, false, false, kPmfNone>);
 template<int I, bool E, bool A>
@@ -1068,14 +1082,22 @@ unsigned PatchImpl::lds_bytes() const {
 	return tables->nb.lds ? unsigned(std::max(tables->nb.total_knots, 2)) * 4u : 0u;
 }
 
+// Where the step kernels take the position-dependent force from (kPmf*); `given`: from a
+// kernel of its own.
+int PatchImpl::pmf_source(bool given, int interp) const {
+	if (num_grids == 0)
+		return kPmfNone;
+	return given ? kPmfGiven : interp == MARSMD_INTERP_LINEAR ? kPmfLinear : kPmfCubic;
+}
+
 // Tiles, block and dynamic LDS of the step kernel.
-PatchImpl::StepShape PatchImpl::step_shape(uint32_t split, int sampled) const {
+PatchImpl::StepShape PatchImpl::step_shape(uint32_t split, int pmf) const {
 	if (split == 0)
 		return StepShape{(n + kBlock - 1) / kBlock, kBlock, lds_bytes(), 0};
 	const uint64_t per = uint64_t(kSplitBlock) >> split;
 	const uint32_t words = (lds_bytes() / 4u + 3u) & ~3u;
 	// the knots, then the handed-over forces of two tiles (and their grid forces)
-	return StepShape{(n + per - 1) / per, kSplitBlock, 4u * words + (sampled == kPmfCubic ? 64u : 32u) * unsigned(per), words};
+	return StepShape{(n + per - 1) / per, kSplitBlock, 4u * words + (pmf == kPmfCubic ? 64u : 32u) * unsigned(per), words};
 }
 
 // Workgroups for a persistent launch over `tiles` tiles: as many as are resident at once
@@ -1378,17 +1400,16 @@ void PatchImpl::run(const marsmd_run_params& P, uint64_t first_step, uint64_t nu
 		const bool bd = P.integrator == MARSMD_INTEGRATOR_BROWNIAN;
 		const bool an = (tables->nb.enabled & kAnalyticTerms) != 0;
 		const uint32_t split = row_split(n, pl->max_neighbors, pl->nbr_entries);
-		// with grids, the position-dependent force may come from its own kernel (the split
-		// rows' step samples it itself: the same bits)
-		const bool pmf_in = split_pmf && num_grids > 0 && split == 0;
-		const int sampled = num_grids == 0 ? kPmfNone : P.interpolation == MARSMD_INTERP_LINEAR ? kPmfLinear : kPmfCubic;
-		const StepFn kern = pick_step(bd, energy, an, pmf_in ? kPmfGiven : sampled);
-		const SplitStepFn kern_split = pick_split(bd, energy, an, sampled);
-		const StepShape shape = step_shape(split, sampled);
+		prepare_prune(P.cutoff, P.pairlist_cutoff, s);
+		// with grids, the position-dependent force may come from its own kernel
+		const bool pmf_in = split_pmf && num_grids > 0;
+		const int pmf = pmf_source(pmf_in, P.interpolation);
+		const StepFn kern = pick_step(bd, energy, an, pmf);
+		const SplitStepFn kern_split = pick_split(bd, energy, an, pmf, prune_valid);
+		const StepShape shape = step_shape(split, pmf);
 		const unsigned grid = persistent_grid(split > 0 ? reinterpret_cast<const void*>(kern_split)
 														: reinterpret_cast<const void*>(kern),
 											  shape.tiles, shape.block, shape.lds);
-		prepare_prune(P.cutoff, P.pairlist_cutoff, s);
 		PruneView PR{};
 		if (prune_valid) {
 			PR.list = NbrList{prune_count.data(), prune_tile_base.data(), prune_nbr.data()};
@@ -1423,7 +1444,7 @@ void PatchImpl::run(const marsmd_run_params& P, uint64_t first_step, uint64_t nu
 			kern_split<<<grid, kSplitBlock, shape.lds, s>>>(pos[cur].data(), pnext, mom.data(), force.data(), n, pl->list(),
 													  tables->nb_dev(), tables->nb_knots(), shape.knot_words,
 													  tables->types_dev(), grids_dev.data(), S, has_bonded, store,
-													  PR, split);
+													  pmf_in ? pmf_buf.data() : nullptr, PR, split);
 		else
 			kern<<<grid, kBlock, shape.lds, s>>>(pos[cur].data(), pnext, mom.data(), force.data(), n, pl->list(),
 										   tables->nb_dev(), tables->nb_knots(), tables->types_dev(),
@@ -1510,17 +1531,18 @@ void PatchImpl::autotune(const marsmd_run_params& P, uint64_t first_step, uint64
 		double ms = 1e300;
 	};
 	std::vector<Cand> cands;
-	const int sampled = num_grids == 0 ? kPmfNone : P.interpolation == MARSMD_INTERP_LINEAR ? kPmfLinear : kPmfCubic;
 	const uint32_t split = pl->built ? row_split(n, pl->max_neighbors, pl->nbr_entries) : 0u;
 	for (bool sp : {false, true}) {
-		if (sp && (num_grids == 0 || split > 0)) // (split rows sample the grids themselves)
+		if (sp && num_grids == 0)
 			continue;
-		// each step kernel's own occupancy (the split one holds fewer registers), then less
-		const void* probe = split > 0 ? reinterpret_cast<const void*>(pick_split(bd, false, an, sampled))
-									  : reinterpret_cast<const void*>(pick_step(bd, false, an, sp ? kPmfGiven : sampled));
+		// each step kernel's own occupancy (one that samples no grid holds fewer registers),
+		// then less
+		const int pmf = pmf_source(sp, P.interpolation);
+		const void* probe = split > 0 ? reinterpret_cast<const void*>(pick_split(bd, false, an, pmf, prune_valid))
+									  : reinterpret_cast<const void*>(pick_step(bd, false, an, pmf));
 		const int saved = blocks_per_cu;
 		blocks_per_cu = 0;
-		const StepShape shape = step_shape(split, sampled);
+		const StepShape shape = step_shape(split, pmf);
 		(void)persistent_grid(probe, shape.tiles, shape.block, shape.lds);
 		blocks_per_cu = saved;
 		const int occ = occupancy[probe].second;

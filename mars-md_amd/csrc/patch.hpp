@@ -134,7 +134,8 @@ struct PatchImpl {
 		int block;
 		unsigned lds, knot_words;
 	};
-	StepShape step_shape(uint32_t split, int sampled) const;
+	int pmf_source(bool given, int interp) const;
+	StepShape step_shape(uint32_t split, int pmf) const;
 	unsigned persistent_grid(const void* kernel, uint64_t tiles, int block, unsigned lds);
 };
 
