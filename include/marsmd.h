@@ -520,18 +520,17 @@ marsmd_status marsmd_patch_autotune(marsmd_patch* p, const marsmd_run_params* pa
                                     marsmd_stream stream);
 /* Cell configuration of the Patch's pairlist walk: home cells (one wave's tile of home
  * particles) of the finest Morton level that holds home_target particles on average
- * (1 .. 4096), candidate cells fine_offset levels below (1 .. 4). Until it is set or
- * tuned the library chooses the cells from the particle count (and get_cells reports 24
- * and 2). The pair set does not depend on it; the order of neighbours in a row, and so the
- * FP32 summation order of the forces, does. Applies from the next build. No
- * counterpart in the reference (its cell grid is select_cell_grid's,
- * ZOrderPairlist.cpp:24-81). */
+ * (1 .. 4096), candidate cells fine_offset levels below (1 .. 4). 24 and 2, the default,
+ * stand for the library's own choice from the particle count. The pair set does not
+ * depend on it; the order of neighbours in a row, and so the FP32 summation order of the
+ * forces, does. Applies from the next build. No counterpart in the reference (its cell
+ * grid is select_cell_grid's, ZOrderPairlist.cpp:24-81). */
 marsmd_status marsmd_patch_set_cells(marsmd_patch* p, int32_t home_target, int32_t fine_offset);
 marsmd_status marsmd_patch_get_cells(marsmd_patch* p, int32_t* home_target, int32_t* fine_offset);
 /* Runs first_step+1 .. first_step+num_steps as marsmd_patch_run, after choosing the cell
- * configuration (home_target 8/12/16/24/48 x fine_offset 1/2/3), each timed re-walking
- * the last build's positions; the live list is then walked with the choice.
- * *walk_ms: the choice's walk time (0 when the home walk does not apply). */
+ * configuration (home_target 8/12/16/24/48 x fine_offset 1/2/3, among them the library's
+ * own choice), each timed re-walking the last build's positions; the live list is then
+ * walked with the choice. *walk_ms: the choice's walk time (0 when the home walk does not apply). */
 marsmd_status marsmd_patch_autotune_cells(marsmd_patch* p, const marsmd_run_params* params,
                                           uint64_t first_step, uint64_t num_steps, double* walk_ms,
                                           marsmd_stream stream);
@@ -624,9 +623,9 @@ marsmd_status marsmd_batch_autotune(marsmd_batch* b, const marsmd_run_params* pa
  * are the finest Morton cells that still hold home_target[b] particles on average,
  * the candidate cells lie fine_offset[b] Morton levels below them. The pair set does
  * not depend on it; the order of neighbours in a row, and so the FP32 summation order
- * of the forces, does. A bucket left at 24 and 2, the defaults, has its cells chosen by
- * the library from the particle counts. No counterpart in the reference (its cell
- * grid is ZOrderPairlist::select_cell_grid's, ZOrderPairlist.cpp:24-81). */
+ * of the forces, does. 24 and 2, the default, stand for the library's own choice from the
+ * particle counts. No counterpart in the reference (its cell grid is
+ * ZOrderPairlist::select_cell_grid's, ZOrderPairlist.cpp:24-81). */
 #define MARSMD_BATCH_BUCKETS 32
 typedef struct marsmd_batch_cells {
     int32_t home_target[MARSMD_BATCH_BUCKETS]; /* 1 .. 4096 */

@@ -789,7 +789,8 @@ void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<ui
 		int m = 0;
 		while (m < 10 && (uint64_t(1) << (3 * (m + 1))) <= 2 * std::max<uint64_t>(n, 1))
 			++m;
-		const WalkLevel lv = walk_level(n, m, cells_auto[size_t(bucket)] ? 0 : int(target), cell_fine[size_t(bucket)],
+		const int offset = cell_fine[size_t(bucket)];
+		const WalkLevel lv = walk_level(n, m, cells_auto(int(target), offset) ? 0 : int(target), offset,
 										kWalkFill * double(n) / double(total));
 		const int h = lv.h;
 		g.h = h;
@@ -865,7 +866,7 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 	// the plan depends on the cutoff, the cell configuration and the pair bookkeeping
 	// (boxes and sizes are fixed): planned again only when one of them changed, which
 	// keeps it off the GPU's idle time when a run starts with a rebuild
-	if (!(plan.valid && plan.rc == rc && plan.target == cell_target && plan.fine == cell_fine && plan.own == cells_auto &&
+	if (!(plan.valid && plan.rc == rc && plan.target == cell_target && plan.fine == cell_fine &&
 		  plan.ref == ref_max_pairs)) {
 		plan.valid = geom_uploaded = false; // until planned whole and uploaded
 		plan_geometry(rc, geom_host, items, plan.fine_total, plan.home_total);
@@ -873,7 +874,6 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 		plan.rc = rc;
 		plan.target = cell_target;
 		plan.fine = cell_fine;
-		plan.own = cells_auto;
 		plan.ref = ref_max_pairs;
 	}
 	const uint64_t fine_total = plan.fine_total, home_total = plan.home_total;
@@ -1282,9 +1282,6 @@ void BatchImpl::set_cells(const marsmd_batch_cells& c) {
 			raise(MARSMD_ERR_VALUE, "batch: fine_offset must be in [1, 4]");
 	}
 	for (int b = 0; b < kBatchBuckets; ++b) {
-		// a bucket set to what it already says keeps the library's own choice
-		cells_auto[size_t(b)] = cells_auto[size_t(b)] && cell_target[size_t(b)] == c.home_target[b] &&
-								cell_fine[size_t(b)] == c.fine_offset[b];
 		cell_target[size_t(b)] = c.home_target[b];
 		cell_fine[size_t(b)] = c.fine_offset[b];
 	}
@@ -1365,11 +1362,9 @@ void BatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, 
 	// one bucket at a time, the others held; a candidate must beat the incumbent by 1%
 	for (int b : present) {
 		int bt = cell_target[size_t(b)], bf = cell_fine[size_t(b)];
-		bool own = cells_auto[size_t(b)]; // the library's own choice, until a candidate beats it
-		cells_auto[size_t(b)] = false;
 		for (int t : targets)
 			for (int f : fines) {
-				if (!own && t == bt && f == bf)
+				if (t == bt && f == bf)
 					continue;
 				cell_target[size_t(b)] = t;
 				cell_fine[size_t(b)] = f;
@@ -1378,12 +1373,10 @@ void BatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, 
 					best = ms;
 					bt = t;
 					bf = f;
-					own = false;
 				}
 			}
 		cell_target[size_t(b)] = bt;
 		cell_fine[size_t(b)] = bf;
-		cells_auto[size_t(b)] = own;
 	}
 	*walk_out = best < 1e300 ? best : 0.0;
 	if (step < first_step + num_steps)

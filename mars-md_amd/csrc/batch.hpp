@@ -55,7 +55,6 @@ struct BatchImpl {
 		bool valid = false;
 		float rc = 0.0f;
 		std::vector<int> target, fine;
-		std::vector<uint8_t> own;
 		std::vector<uint64_t> ref;
 		uint64_t fine_total = 0, home_total = 0;
 	} plan;
@@ -90,10 +89,8 @@ struct BatchImpl {
 	DevArray<uint32_t> step_word;
 	// cell configuration per size bucket: the walk's home cells hold at least
 	// cell_target particles on average; its fine cells lie cell_fine levels below
-	std::vector<int> cell_target = std::vector<int>(size_t(kBatchBuckets), 24);
-	std::vector<int> cell_fine = std::vector<int>(size_t(kBatchBuckets), 2);
-	// buckets neither set nor tuned, whose cells walk_level chooses
-	std::vector<uint8_t> cells_auto = std::vector<uint8_t>(size_t(kBatchBuckets), 1);
+	std::vector<int> cell_target = std::vector<int>(size_t(kBatchBuckets), kCellsTarget);
+	std::vector<int> cell_fine = std::vector<int>(size_t(kBatchBuckets), kCellsOffset);
 	// scratch of the walk timing (the live list is untouched)
 	DevArray<uint8_t> t_geom;
 	DevArray<uint32_t> t_items, t_counts, t_nbr;

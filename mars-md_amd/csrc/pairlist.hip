@@ -810,14 +810,14 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 		return per && (1 << (mf - h)) + 2 * reach_of(mf, a) >= (1 << mf);
 	};
 	const bool wraps = box.periodic[0] && box.periodic[1] && box.periodic[2];
-	WalkLevel lv = walk_level(n, m, cells_auto ? 0 : home_target, fine_offset, kWalkFill, excl.offsets ? 2 : 4);
+	WalkLevel lv = walk_level(n, m, cells_auto() ? 0 : home_target, fine_offset, kWalkFill, excl.offsets ? 2 : 4);
 	// the level whose cells order the rows (its own when the cells were set)
-	const WalkLevel order = cells_auto ? walk_level(n, m, kRowTarget, kRowOffset, 0.0) : lv;
+	const WalkLevel order = cells_auto() ? walk_level(n, m, kRowTarget, kRowOffset, 0.0) : lv;
 	int full_axes = 0; // of the order level's stencil
 	for (int a = 0; a < 3; ++a)
 		full_axes += full_of(order.h, std::min(10, order.h + order.s), a) ? 1 : 0;
 	uint32_t lists = 1;
-	if (cells_auto && wraps) {
+	if (cells_auto() && wraps) {
 		if (full_axes == 3 && n <= kWholeBoxMax)
 			lv.s = -lv.h; // rows by slot: every particle is a candidate, in slot order
 		else if (full_axes > 0 || full_of(lv.h, lv.h, 0) || full_of(lv.h, lv.h, 1) || full_of(lv.h, lv.h, 2))

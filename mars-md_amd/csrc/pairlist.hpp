@@ -73,6 +73,12 @@ __host__ __device__ inline uint64_t nbr_slot_index(uint64_t tile_base, uint32_t 
 	return tile_base + uint64_t(k >> 2) * 256u + uint64_t(t & 63u) * 4u + (k & 3u);
 }
 
+// The cell configuration that leaves the choice to the library.
+constexpr int kCellsTarget = 24, kCellsOffset = 2;
+inline bool cells_auto(int home_target, int fine_offset) {
+	return home_target == kCellsTarget && fine_offset == kCellsOffset;
+}
+
 struct PairlistImpl {
 	uint64_t max_particles = 0;
 	uint64_t ref_max_pairs = 0;     // Pairlist::max_pairs_ bookkeeping (grows x1.25)
@@ -94,9 +100,10 @@ struct PairlistImpl {
 	DevArray<uint2> walk_cells;
 	uint32_t home_cap = 0;
 	// cell configuration of the home walk: home cells of the finest level holding at
-	// least home_target particles on average, candidate cells fine_offset levels below
-	int home_target = 24, fine_offset = 2;
-	bool cells_auto = true;         // neither set nor tuned: walk_level chooses
+	// least home_target particles on average, candidate cells fine_offset levels below; the
+	// defaults stand for the library's own choice (walk_level)
+	int home_target = kCellsTarget, fine_offset = kCellsOffset;
+	bool cells_auto() const { return mmd::cells_auto(home_target, fine_offset); }
 	// every exclusion is in both ends' rows and names a particle of the build: set by the
 	// Patch for its own CSR and builds only
 	bool excl_symmetric = false;

@@ -1468,7 +1468,6 @@ void PatchImpl::set_cells(int home_target, int fine_offset) {
 		raise(MARSMD_ERR_VALUE, "Patch: fine_offset must be in [1, 4]");
 	pl->home_target = home_target;
 	pl->fine_offset = fine_offset;
-	pl->cells_auto = false;
 }
 
 void PatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, uint64_t num_steps, hipStream_t s,
@@ -1487,11 +1486,10 @@ void PatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, 
 			return b;
 		};
 		int bt = pl->home_target, bf = pl->fine_offset;
-		bool own = pl->cells_auto; // the library's own choice, until a candidate beats it
 		best = measure();
 		for (int t : {8, 12, 16, 24, 48})
 			for (int f : {1, 2, 3}) {
-				if (!own && t == bt && f == bf)
+				if (t == bt && f == bf)
 					continue;
 				set_cells(t, f);
 				const double ms = measure();
@@ -1499,11 +1497,9 @@ void PatchImpl::autotune_cells(const marsmd_run_params& P, uint64_t first_step, 
 					best = ms;
 					bt = t;
 					bf = f;
-					own = false;
 				}
 			}
 		set_cells(bt, bf);
-		pl->cells_auto = own;
 		(void)pl->rewalk_ms(s); // the live list as the choice walks it
 	}
 	*walk_out = best > 0.0 ? best : 0.0;

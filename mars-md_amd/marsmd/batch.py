@@ -163,7 +163,7 @@ class Batch:
 
     def set_cells(self, cells: dict):
         """Cell configuration per size bucket, {bucket: (home_target, fine_offset)}; the
-        buckets not named keep theirs. Applies from the next build."""
+        buckets not named keep theirs; (24, 2) stands for the library's own choice. Applies from the next build."""
         cur = self.get_cells(all_buckets=True)
         cur.update({int(b): tuple(v) for b, v in cells.items()})
         c = api.BatchCells()

@@ -126,8 +126,8 @@ class Patch:
 
     def set_cells(self, home_target: int = 24, fine_offset: int = 2):
         """Cell configuration of the pairlist walk (home cells holding home_target
-        particles on average, candidate cells fine_offset levels finer); the pair set
-        does not depend on it. Applies from the next build."""
+        particles on average, candidate cells fine_offset levels finer; 24 and 2 stand for
+        the library's own choice); the pair set does not depend on it. Applies from the next build."""
         api.call("marsmd_patch_set_cells", self._h, int(home_target), int(fine_offset))
 
     def get_cells(self) -> tuple:
