@@ -54,8 +54,9 @@ struct RepGeom {
 	// the home-frame prefilter of the walk (see HomeParams)
 	int pre;
 	float pre_lo2, pre_hi2;
-	// the replica's fine-cell stencil in the batch's table (count 0: none)
-	uint32_t stencil_off, stencil_n;
+	// the replica's fine-cell stencil in the batch's table (count 0: none), one list for each
+	// position under the mask (see HomeParams)
+	uint32_t stencil_off, stencil_n, stencil_lists;
 };
 
 // A wrapped coordinate lies in [lo, hi] up to the rounding of PeriodicBox::wrap_scalar
@@ -186,6 +187,21 @@ __global__ void k_b_cell_ranges(const uint32_t* __restrict__ codes, uint64_t tot
 		home[G.home_off + hc].y = uint32_t(i + 1);
 }
 
+// The stencils' lists, one a workgroup. A stencil of more cells than are sorted has one list,
+// which is its own order.
+__global__ __launch_bounds__(256) void k_b_stencil_lists(const StencilList* __restrict__ lists,
+														 const int4* __restrict__ offsets,
+														 uint32_t* __restrict__ codes) {
+	__shared__ uint64_t keys[kStencilSortMax];
+	const StencilList l = lists[blockIdx.x];
+	if (l.n <= kStencilSortMax) {
+		stencil_list(offsets + l.first, l.n, int(l.level), l.position, codes + l.out, keys);
+		return;
+	}
+	for (uint32_t i = threadIdx.x; i < l.n; i += 256u)
+		codes[l.out + i] = stencil_offset_code(offsets[l.first + i], int(l.level));
+}
+
 // The home-cell walk over the work items of all replicas (item_off[r] = first item of
 // replica r, one item per home cell).
 __global__ __launch_bounds__(256, 6) void k_b_walk(const RepGeom* __restrict__ geom, const uint32_t* __restrict__ item_off,
@@ -242,6 +258,7 @@ __global__ __launch_bounds__(256, 6) void k_b_walk(const RepGeom* __restrict__ g
 		P.pre_hi2 = G.pre_hi2;
 		P.stencil_code = G.stencil_n ? stencils + G.stencil_off : nullptr;
 		P.stencil_n = G.stencil_n;
+		P.stencil_lists = G.stencil_lists;
 		const uint32_t cell = item - item_off[r];
 		const uint2 hr = P.home[cell];
 		const uint32_t from = uint32_t(__builtin_amdgcn_readfirstlane(int(hr.x)));
@@ -767,10 +784,10 @@ int batch_size_bucket(uint64_t n) {
 }
 
 // Per-replica geometry of a build with the cell configuration of each replica's size
-// bucket: home cells of the largest level h <= m - 1 holding at least `home_target`
-// particles on average, fine cells `fine_offset` levels below (at most level 10).
+// bucket (walk_grid; left to the library, the home cells of all replicas together occupy
+// the chip, and a replica's rows are in the order that its own size gives, as a Patch's).
 void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<uint32_t>& items,
-							  uint64_t& fine_total, uint64_t& home_total) {
+							  uint64_t& fine_total, uint64_t& home_total, hipStream_t s) {
 	const float rc2 = rc * rc;
 	gh.assign(R * sizeof(RepGeom), 0);
 	RepGeom* G = reinterpret_cast<RepGeom*>(gh.data());
@@ -785,29 +802,25 @@ void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<ui
 		g.n = uint32_t(n);
 		g.pid = pid[r];
 		const int bucket = batch_size_bucket(n);
-		const uint64_t target = uint64_t(std::max(1, cell_target[size_t(bucket)]));
 		int m = 0;
 		while (m < 10 && (uint64_t(1) << (3 * (m + 1))) <= 2 * std::max<uint64_t>(n, 1))
 			++m;
-		const int offset = cell_fine[size_t(bucket)];
-		const WalkLevel lv = walk_level(n, m, cells_auto(int(target), offset) ? 0 : int(target), offset,
-										kWalkFill * double(n) / double(total));
-		const int h = lv.h;
-		g.h = h;
-		g.mf = std::min(10, h + lv.s);
-		const int fine_cells = 1 << g.mf;
-		const int span = 1 << (g.mf - h);
-		const int k = 1024 / fine_cells;
 		for (int a = 0; a < 3; ++a) {
 			g.lo[a] = boxes[r].origin[a];
 			g.hi[a] = boxes[r].origin[a] + boxes[r].size[a];
-			const float extent = std::fmax(g.hi[a] - g.lo[a], 1e-6f);
-			const double W = double(extent) / 1023.0;
-			const double need = (double(rc) * (1.0 + 1e-6) + 1e-3) / W + 1.0;
-			g.reach[a] = std::max(1, int(std::min(std::ceil(need / double(k)), double(fine_cells))));
-			g.full[a] = span + 2 * g.reach[a] >= fine_cells ? 1 : 0;
-			g.cw[a] = float(double(extent) * k / 1023.0);
-			g.margin[a] = float(W * 1.001 + 1e-5 * double(extent) + 1e-3);
+		}
+		const bool per[3] = {true, true, true};
+		const WalkGrid w = walk_grid(n, m, cell_target[size_t(bucket)], cell_fine[size_t(bucket)],
+									 kWalkFill * double(n) / double(total), 4, g.lo, g.hi, per, double(rc), rc2);
+		const int h = w.h;
+		g.h = h;
+		g.mf = w.mf;
+		g.stencil_lists = w.lists - 1u;
+		for (int a = 0; a < 3; ++a) {
+			g.reach[a] = w.reach[a];
+			g.full[a] = w.full[a];
+			g.cw[a] = w.cw[a];
+			g.margin[a] = w.margin[a];
 		}
 		// the reference grid of this replica: when it misses seam pairs, the walk keeps
 		// exactly the pairs its stencil reaches
@@ -831,13 +844,22 @@ void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<ui
 										float(g.reach[1]), float(g.reach[2]),  float(g.full[0]),
 										float(g.full[1]),  float(g.full[2]),   g.cw[0],
 										g.cw[1],		   g.cw[2],			   g.margin[0],
-										g.margin[1],	   g.margin[2],		   rc2};
+										g.margin[1],	   g.margin[2],		   rc2,
+										float(w.lists)};
 		auto it = stencil_index.find(key);
 		if (it == stencil_index.end()) {
-			const std::vector<int4> st = home_stencil(h, g.mf - h, g.reach, g.full, g.cw, g.margin, rc2, 8192);
-			it = stencil_index.emplace(key, std::make_pair(uint32_t(stencils_host.size()), uint32_t(st.size()))).first;
-			for (const int4& o : st)
-				stencils_host.push_back(stencil_offset_code(o, g.mf));
+			const std::vector<int4> st = g.mf < h ? std::vector<int4>{make_int4(0, 0, 0, 0)}
+												  : home_stencil(h, g.mf - h, g.reach, g.full, g.cw, g.margin, rc2, 8192);
+			const uint32_t cells = uint32_t(st.size());
+			if (stencil_codes + uint64_t(cells) * w.lists >= (uint64_t(1) << 32))
+				raise(MARSMD_ERR_VALUE, "batch: stencils exceed 2^32 entries");
+			it = stencil_index.emplace(key, std::make_pair(uint32_t(stencil_codes), cells)).first;
+			for (uint32_t b = 0; b < (cells > 0 ? w.lists : 0u); ++b) {
+				stencil_lists_host.push_back(StencilList{uint32_t(stencil_cells_host.size()), cells,
+														 uint32_t(stencil_codes), uint32_t(g.mf), b});
+				stencil_codes += cells;
+			}
+			stencil_cells_host.insert(stencil_cells_host.end(), st.begin(), st.end());
 		}
 		g.stencil_off = it->second.first;
 		g.stencil_n = it->second.second;
@@ -851,11 +873,19 @@ void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<ui
 	}
 	if (fine_total >= (uint64_t(1) << 32))
 		raise(MARSMD_ERR_VALUE, "batch: cell tables exceed 2^32 entries");
-	if (stencils_host.size() > stencils_uploaded) { // new geometries (a synchronous upload, rare)
-		stencils.resize(stencils_host.size());
-		MMD_HIP(hipMemcpy(stencils.data(), stencils_host.data(), sizeof(uint32_t) * stencils_host.size(),
+	if (stencil_lists_host.size() > stencils_made) { // new geometries (synchronous uploads, rare)
+		stencils_made = 0; // until all are made
+		stencils.resize(stencil_codes);
+		stencil_cells.resize(stencil_cells_host.size());
+		stencil_lists.resize(stencil_lists_host.size());
+		MMD_HIP(hipMemcpy(stencil_cells.data(), stencil_cells_host.data(), sizeof(int4) * stencil_cells_host.size(),
 						  hipMemcpyHostToDevice));
-		stencils_uploaded = stencils_host.size();
+		MMD_HIP(hipMemcpy(stencil_lists.data(), stencil_lists_host.data(),
+						  sizeof(StencilList) * stencil_lists_host.size(), hipMemcpyHostToDevice));
+		k_b_stencil_lists<<<unsigned(stencil_lists_host.size()), 256, 0, s>>>(stencil_lists.data(),
+																			  stencil_cells.data(), stencils.data());
+		MMD_LAUNCH_CHECK();
+		stencils_made = stencil_lists_host.size();
 	}
 }
 
@@ -869,7 +899,7 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 	if (!(plan.valid && plan.rc == rc && plan.target == cell_target && plan.fine == cell_fine &&
 		  plan.ref == ref_max_pairs)) {
 		plan.valid = geom_uploaded = false; // until planned whole and uploaded
-		plan_geometry(rc, geom_host, items, plan.fine_total, plan.home_total);
+		plan_geometry(rc, geom_host, items, plan.fine_total, plan.home_total, s);
 		plan.valid = true;
 		plan.rc = rc;
 		plan.target = cell_target;
@@ -1298,7 +1328,7 @@ double BatchImpl::walk_ms(hipStream_t s) {
 	std::vector<uint8_t> gh;
 	std::vector<uint32_t> items;
 	uint64_t ft = 0, ht = 0;
-	plan_geometry(built_cutoff, gh, items, ft, ht);
+	plan_geometry(built_cutoff, gh, items, ft, ht, s);
 	t_geom.resize(R * sizeof(RepGeom));
 	MMD_HIP(hipMemcpyAsync(t_geom.data(), gh.data(), R * sizeof(RepGeom), hipMemcpyHostToDevice, s));
 	t_items.resize(R + 1);

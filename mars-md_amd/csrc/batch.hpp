@@ -17,6 +17,12 @@ struct StepParams;
 constexpr int kBatchBuckets = MARSMD_BATCH_BUCKETS;
 int batch_size_bucket(uint64_t n);
 
+// A stencil's list of codes for one position of a home cell (see stencil_list).
+struct StencilList {
+	uint32_t first, n, out; // its offsets, its codes
+	uint32_t level, position;
+};
+
 struct BatchImpl {
 	uint64_t R = 0, total = 0, base_seed = 0;
 	std::vector<uint64_t> off, count, pid;
@@ -45,11 +51,16 @@ struct BatchImpl {
 	uint32_t cap = 0, max_neighbors = 0;
 	std::vector<uint8_t> geom_host;     // host copies behind the asynchronous uploads
 	// fine-cell stencils of the home walk, one per distinct replica geometry (key: the
-	// walk parameters it depends on; value: offset and count in stencils)
+	// walk parameters it depends on; value: first code in stencils and cells of a list),
+	// each as its lists of codes in row order
 	std::map<std::vector<float>, std::pair<uint32_t, uint32_t>> stencil_index;
-	std::vector<uint32_t> stencils_host; // Morton codes of the offsets
+	std::vector<int4> stencil_cells_host;
+	std::vector<StencilList> stencil_lists_host;
+	uint64_t stencil_codes = 0; // of every list
+	DevArray<int4> stencil_cells;
+	DevArray<StencilList> stencil_lists;
 	DevArray<uint32_t> stencils;
-	size_t stencils_uploaded = 0;
+	size_t stencils_made = 0; // lists whose codes are in `stencils`
 	std::vector<uint32_t> items_host;
 	struct Plan { // what geom_host and items_host were planned from
 		bool valid = false;
@@ -126,7 +137,7 @@ struct BatchImpl {
 
   private:
 	void plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<uint32_t>& items, uint64_t& fine_total,
-					   uint64_t& home_total);
+					   uint64_t& home_total, hipStream_t s);
 	double walk_ms(hipStream_t s);
 	void build(float pairlist_cutoff, bool relabel, hipStream_t s);
 	bool needs_rebuild(float skin, hipStream_t s);

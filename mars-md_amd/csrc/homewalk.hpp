@@ -116,20 +116,19 @@ struct HomeParams {
 	uint32_t stencil_lists;
 };
 
-// The fine cells of the walk's enumeration that pass its gap test, as offsets (see
-// HomeParams::stencil); empty when there are more than max_cells of them. The test is
-// the walk's own: per axis not enumerated whole, the number of cells between the cell
-// and the home cell's span times the cell width, less twice the margin, floored at 0,
-// squared and summed, against rc^2.
-inline std::vector<int4> home_stencil(int h, int s, const int reach[3], const int full[3], const float cw[3],
-									  const float margin[3], float rc2, size_t max_cells) {
+// f(offset) for the fine cells of the walk's enumeration that pass its gap test, as offsets
+// (see HomeParams::stencil), until it returns false. The test is the walk's own: per axis
+// not enumerated whole, the number of cells between the cell and the home cell's span times
+// the cell width, less twice the margin, floored at 0, squared and summed, against rc^2.
+template<class F>
+inline void for_each_stencil_cell(int h, int s, const int reach[3], const int full[3], const float cw[3],
+								  const float margin[3], float rc2, F&& f) {
 	const int fine_cells = 1 << (h + s), span = 1 << s;
 	int lo[3], nax[3];
 	for (int a = 0; a < 3; ++a) {
 		lo[a] = full[a] ? 0 : -reach[a];
 		nax[a] = full[a] ? fine_cells : span + 2 * reach[a];
 	}
-	std::vector<int4> out;
 	for (int z = 0; z < nax[2]; ++z)
 		for (int y = 0; y < nax[1]; ++y)
 			for (int x = 0; x < nax[0]; ++x) {
@@ -142,12 +141,23 @@ inline std::vector<int4> home_stencil(int h, int s, const int reach[3], const in
 					const float g = std::fmax(0.0f, float(apart) * cw[a] - 2.0f * margin[a]);
 					gap2 += g * g;
 				}
-				if (gap2 <= rc2) {
-					if (out.size() == max_cells)
-						return {};
-					out.push_back(make_int4(o[0], o[1], o[2], 0));
-				}
+				if (gap2 <= rc2 && !f(make_int4(o[0], o[1], o[2], 0)))
+					return;
 			}
+}
+// All of them in Morton order; empty when there are more than max_cells.
+inline std::vector<int4> home_stencil(int h, int s, const int reach[3], const int full[3], const float cw[3],
+									  const float margin[3], float rc2, size_t max_cells) {
+	std::vector<int4> out;
+	bool fits = true;
+	for_each_stencil_cell(h, s, reach, full, cw, margin, rc2, [&](const int4& o) {
+		fits = out.size() < max_cells;
+		if (fits)
+			out.push_back(o);
+		return fits;
+	});
+	if (!fits)
+		return {};
 	// Morton order of the offsets: 64 consecutive candidates then come from a compact
 	// cluster of cells
 	auto key = [](const int4& c) {
@@ -183,20 +193,110 @@ inline WalkLevel walk_level(uint64_t n, int m, int target, int offset, double fi
 		++h;
 	return WalkLevel{h, 0};
 }
-// A Patch's rows list a particle's neighbours by the Morton order of their offsets from
-// the particle's cell at the level that holds kRowTarget particles per cell on average (by
-// slot where that level's stencil wraps onto itself on every axis), whatever level the
-// walk runs at: the FP32 sum over a row is then the same bits.
-constexpr int kRowTarget = 24, kRowOffset = 2;
+// Rows list a particle's neighbours by the Morton order of their offsets from the
+// particle's cell at the level that holds kRowTarget particles per cell on average (by slot
+// where that level's stencil wraps onto itself on every axis), whatever level the walk runs
+// at: the FP32 sum over a row is then the same bits. Where the cells were set, and in boxes
+// with an open axis, a row is in the order of the walk's own cells.
+constexpr int kRowTarget = kCellsTarget, kRowOffset = kCellsOffset;
 // particles up to which rows by slot come from walking the whole box (n / 64 candidate
 // blocks a home cell)
 constexpr uint64_t kWholeBoxMax = 16384;
+// cells of a stencil that is listed once for each position of a home cell in its cell of the
+// order level (see k_stencil_lists)
+constexpr uint32_t kStencilSortMax = 2048;
+
+// The cells of a walk: home cells of level h; fine cells of level mf with their enumeration
+// (mf < h: one fine cell, the whole box); the lists its stencil has
+// (HomeParams::stencil_lists + 1).
+struct WalkGrid {
+	int h, mf;
+	uint32_t lists;
+	int reach[3], full[3];
+	float cw[3], margin[3];
+};
+// The grid for n particles in the Morton domain [lo, hi), periodic where `per`, with build
+// levels up to m and the cell configuration given (see walk_level for fill and per_cell).
+inline WalkGrid walk_grid(uint64_t n, int m, int home_target, int fine_offset, double fill, uint64_t per_cell,
+						  const float lo[3], const float hi[3], const bool per[3], double rc, float rc2) {
+	const auto extent = [&](int a) { return std::fmax(hi[a] - lo[a], 1e-6f); };
+	// fine cells of level `mf` beyond a home cell that cover rc with the seam slack of the
+	// quantised top cell, and whether such a stencil wraps onto itself on the axis
+	const auto reach_of = [&](int mf, int a) {
+		const double W = double(extent(a)) / 1023.0;
+		const double need = (rc * (1.0 + 1e-6) + 1e-3) / W + (per[a] ? 1.0 : 0.0);
+		return std::max(1, int(std::min(std::ceil(need / double(1024 >> mf)), double(1 << mf))));
+	};
+	const auto full_of = [&](int h, int mf, int a) {
+		return per[a] && (1 << (mf - h)) + 2 * reach_of(mf, a) >= (1 << mf);
+	};
+	const auto grid_of = [&](const WalkLevel& lv) {
+		WalkGrid g{};
+		g.h = lv.h;
+		g.mf = std::min(10, lv.h + lv.s);
+		g.lists = 1;
+		for (int a = 0; a < 3; ++a) {
+			const double W = double(extent(a)) / 1023.0;
+			g.reach[a] = reach_of(g.mf, a);
+			g.full[a] = g.mf < g.h || full_of(g.h, g.mf, a) ? 1 : 0;
+			g.cw[a] = float(double(extent(a)) * (1024 >> g.mf) / 1023.0);
+			g.margin[a] = float(W * 1.001 + 1e-5 * double(extent(a)) + 1e-3);
+		}
+		return g;
+	};
+	const bool own = cells_auto(home_target, fine_offset);
+	WalkLevel lv = walk_level(n, m, own ? 0 : home_target, fine_offset, fill, per_cell);
+	if (!own || !(per[0] && per[1] && per[2]))
+		return grid_of(lv);
+	const WalkGrid order = grid_of(walk_level(n, m, kRowTarget, kRowOffset, 0.0));
+	const int full_axes = order.full[0] + order.full[1] + order.full[2];
+	if (full_axes == 3 && n <= kWholeBoxMax) {
+		lv.s = -lv.h; // rows by slot: every particle is a candidate, in slot order
+		return grid_of(lv);
+	}
+	WalkGrid g = grid_of(lv);
+	if (full_axes > 0 || g.full[0] || g.full[1] || g.full[2])
+		return order; // offsets and absolute cells mixed: the order level's own walk
+	if (g.h > order.h) {
+		uint32_t cells = 0;
+		for_each_stencil_cell(g.h, g.mf - g.h, g.reach, g.full, g.cw, g.margin, rc2,
+							  [&](const int4&) { return ++cells <= kStencilSortMax; });
+		if (cells > kStencilSortMax)
+			return order; // (more than 500 neighbours a particle)
+		g.lists = 1u << (3 * (g.h - order.h));
+	}
+	return g;
+}
 
 // An offset of home_stencil as the Morton code of its components modulo 2^level cells.
-inline uint32_t stencil_offset_code(const int4& o, int level) {
+__host__ __device__ inline uint32_t stencil_offset_code(const int4& o, int level) {
 	const uint32_t mask = (1u << level) - 1u;
 	return split_by3(uint32_t(o.z) & mask) | (split_by3(uint32_t(o.y) & mask) << 1) |
 		   (split_by3(uint32_t(o.x) & mask) << 2);
+}
+
+// List b of a stencil in row order: its n offsets (relative to a home cell of `level`) in the
+// Morton order of the cells' offsets from the home cell's ancestor of the order level,
+// within which the home cell lies at the position whose Morton code is b, as codes
+// (stencil_offset_code). Ranks by counting (a few hundred cells; no two keys are equal), by a
+// workgroup with `keys` in LDS.
+__device__ inline void stencil_list(const int4* __restrict__ offsets, uint32_t n, int level, uint32_t b,
+									uint32_t* __restrict__ codes, uint64_t* keys) {
+	const int p[3] = {int(compact_by3(b >> 2)), int(compact_by3(b >> 1)), int(compact_by3(b))};
+	for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+		const int4 o = offsets[i];
+		const uint32_t v[3] = {uint32_t(p[0] + o.x + 1024), uint32_t(p[1] + o.y + 1024), uint32_t(p[2] + o.z + 1024)};
+		keys[i] = (uint64_t(((v[0] >> 10) & 1u) << 2 | ((v[1] >> 10) & 1u) << 1 | ((v[2] >> 10) & 1u)) << 30) |
+				  (split_by3(v[0]) << 2 | split_by3(v[1]) << 1 | split_by3(v[2]));
+	}
+	__syncthreads();
+	for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
+		const uint64_t k = keys[i];
+		uint32_t rank = 0;
+		for (uint32_t j = 0; j < n; ++j)
+			rank += keys[j] < k ? 1u : 0u;
+		codes[rank] = stencil_offset_code(offsets[i], level);
+	}
 }
 
 // The prefilter's band for a domain [lo, hi) whose home cells (level h) have width

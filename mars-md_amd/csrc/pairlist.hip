@@ -198,33 +198,11 @@ __global__ void k_walk_cells(const uint32_t* __restrict__ codes, uint64_t n, int
 		home[c >> home_shift].y = uint32_t(i + 1);
 }
 
-// The walk's stencil lists in row order (see kRowTarget): list b holds the n offsets
-// (relative to a home cell of `level`) in the Morton order of the cells' offsets from the
-// home cell's ancestor `up` levels above, within which the home cell lies at the position
-// whose Morton code is b. Ranks by counting (a few hundred cells; no two keys are equal).
-constexpr uint32_t kStencilSortMax = 2048;
+// The walk's stencil lists in row order, one a workgroup (see stencil_list).
 __global__ __launch_bounds__(256) void k_stencil_lists(const int4* __restrict__ offsets, uint32_t n, int level,
 													   uint32_t* __restrict__ codes) {
 	__shared__ uint64_t keys[kStencilSortMax];
-	const uint32_t b = blockIdx.x;
-	const int p[3] = {int(compact_by3(b >> 2)), int(compact_by3(b >> 1)), int(compact_by3(b))};
-	for (uint32_t i = threadIdx.x; i < n; i += 256u) {
-		const int4 o = offsets[i];
-		const uint32_t v[3] = {uint32_t(p[0] + o.x + 1024), uint32_t(p[1] + o.y + 1024), uint32_t(p[2] + o.z + 1024)};
-		keys[i] = (uint64_t(((v[0] >> 10) & 1u) << 2 | ((v[1] >> 10) & 1u) << 1 | ((v[2] >> 10) & 1u)) << 30) |
-				  (split_by3(v[0]) << 2 | split_by3(v[1]) << 1 | split_by3(v[2]));
-	}
-	__syncthreads();
-	const uint32_t mask = (1u << level) - 1u;
-	for (uint32_t i = threadIdx.x; i < n; i += 256u) {
-		const uint64_t k = keys[i];
-		uint32_t rank = 0;
-		for (uint32_t j = 0; j < n; ++j)
-			rank += keys[j] < k ? 1u : 0u;
-		const int4 o = offsets[i];
-		codes[uint64_t(b) * n + rank] =
-			split_by3(uint32_t(o.x) & mask) << 2 | split_by3(uint32_t(o.y) & mask) << 1 | split_by3(uint32_t(o.z) & mask);
-	}
+	stencil_list(offsets, n, level, blockIdx.x, codes + uint64_t(blockIdx.x) * n, keys);
 }
 
 // BuildCellNeighborsKernel (ZOrderNeighbor.h:55-139), for the reference tables.
@@ -796,36 +774,13 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 	const int m = build_grid.m;
 	if (m < 1)
 		return false;
-	const double cut = std::sqrt(double(cutoff_squared));
-	// fine cells of level `mf` beyond a home cell that cover rc with the seam slack of the
-	// quantised top cell, and whether such a stencil wraps onto itself on the axis
-	const auto reach_of = [&](int mf, int a) {
-		const bool per = box.periodic[a] != 0 && box.size[a] > 0.0f;
-		const double W = double(std::fmax(domain_max[a] - domain_min[a], 1e-6f)) / 1023.0;
-		const double need = (cut * (1.0 + 1e-6) + 1e-3) / W + (per ? 1.0 : 0.0);
-		return std::max(1, int(std::min(std::ceil(need / double(1024 >> mf)), double(1 << mf))));
-	};
-	const auto full_of = [&](int h, int mf, int a) {
-		const bool per = box.periodic[a] != 0 && box.size[a] > 0.0f;
-		return per && (1 << (mf - h)) + 2 * reach_of(mf, a) >= (1 << mf);
-	};
-	const bool wraps = box.periodic[0] && box.periodic[1] && box.periodic[2];
-	WalkLevel lv = walk_level(n, m, cells_auto() ? 0 : home_target, fine_offset, kWalkFill, excl.offsets ? 2 : 4);
-	// the level whose cells order the rows (its own when the cells were set)
-	const WalkLevel order = cells_auto() ? walk_level(n, m, kRowTarget, kRowOffset, 0.0) : lv;
-	int full_axes = 0; // of the order level's stencil
-	for (int a = 0; a < 3; ++a)
-		full_axes += full_of(order.h, std::min(10, order.h + order.s), a) ? 1 : 0;
-	uint32_t lists = 1;
-	if (cells_auto() && wraps) {
-		if (full_axes == 3 && n <= kWholeBoxMax)
-			lv.s = -lv.h; // rows by slot: every particle is a candidate, in slot order
-		else if (full_axes > 0 || full_of(lv.h, lv.h, 0) || full_of(lv.h, lv.h, 1) || full_of(lv.h, lv.h, 2))
-			lv = order; // offsets and absolute cells mixed: the order level's own walk
-		else if (lv.h > order.h)
-			lists = 1u << (3 * (lv.h - order.h));
-	}
-	const int h = lv.h, mf = std::min(10, lv.h + lv.s);
+	const bool per[3] = {box.periodic[0] != 0 && box.size[0] > 0.0f, box.periodic[1] != 0 && box.size[1] > 0.0f,
+						 box.periodic[2] != 0 && box.size[2] > 0.0f};
+	const bool wraps = per[0] && per[1] && per[2];
+	const WalkGrid grid_cells = walk_grid(n, m, home_target, fine_offset, kWalkFill, excl.offsets ? 2 : 4, domain_min,
+										  domain_max, per, std::sqrt(double(cutoff_squared)), cutoff_squared);
+	const int h = grid_cells.h, mf = grid_cells.mf;
+	const uint32_t lists = grid_cells.lists;
 	const uint64_t tiles = (n + 63) / 64;
 	HomeParams P{};
 	P.spos = spos.data();
@@ -834,13 +789,11 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 	P.num_home = uint32_t(1) << (3 * h);
 	double volume = 1.0;
 	for (int a = 0; a < 3; ++a) {
-		const float extent = std::fmax(domain_max[a] - domain_min[a], 1e-6f);
-		const double W = double(extent) / 1023.0;
-		P.reach[a] = reach_of(mf, a);
-		P.full[a] = mf < h || full_of(h, mf, a) ? 1 : 0;
-		volume *= double(extent);
-		P.cw[a] = float(double(extent) * (1024 >> mf) / 1023.0);
-		P.margin[a] = float(W * 1.001 + 1e-5 * double(extent) + 1e-3);
+		P.reach[a] = grid_cells.reach[a];
+		P.full[a] = grid_cells.full[a];
+		P.cw[a] = grid_cells.cw[a];
+		P.margin[a] = grid_cells.margin[a];
+		volume *= double(std::fmax(domain_max[a] - domain_min[a], 1e-6f));
 	}
 	const uint64_t num_fine = uint64_t(1) << (3 * mf), num_home = uint64_t(1) << (3 * h);
 	walk_cells.resize(num_fine + num_home);
@@ -870,11 +823,11 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 									P.margin[1],	   P.margin[2],		   P.rc2,			  wraps ? 1.0f : 0.0f,
 									float(lists)};
 	if (key != stencil_key) {
-		stencil_key = key;
+		stencil_key.clear(); // until it is made
 		const std::vector<int4> cells = mf < h ? std::vector<int4>{make_int4(0, 0, 0, 0)}
 											   : home_stencil(h, P.s, P.reach, P.full, P.cw, P.margin, P.rc2, 8192);
 		stencil_n = uint32_t(cells.size());
-		stencil_lists = stencil_n <= kStencilSortMax ? lists : 1u;
+		stencil_lists = lists;
 		if (stencil_n > 0 && (!wraps || stencil_lists > 1)) {
 			stencil_dev.resize(stencil_n);
 			MMD_HIP(hipMemcpy(stencil_dev.data(), cells.data(), sizeof(int4) * stencil_n, hipMemcpyHostToDevice));
@@ -892,6 +845,7 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 					hipMemcpy(stencil_codes.data(), words.data(), sizeof(uint32_t) * stencil_n, hipMemcpyHostToDevice));
 			}
 		}
+		stencil_key = key;
 	}
 	if (stencil_n > 0) {
 		P.stencil_code = wraps ? stencil_codes.data() : nullptr;
