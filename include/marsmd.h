@@ -602,8 +602,9 @@ marsmd_status marsmd_batch_set_kernel_timing(marsmd_batch* b, int32_t enable);
 marsmd_status marsmd_batch_get_kernel_timing(marsmd_batch* b, double* total_ms, uint64_t* steps);
 
 /* Launch configuration of the batched step (no counterpart in the reference). Results
- * do not depend on it: each particle's step is one lane's work whatever the grid, and
- * a replayed segment launches the same kernels with the same arguments. */
+ * do not depend on it: each particle's sums are taken in the same order whatever lanes
+ * and workgroups take them, and a replayed segment launches the same kernels with the
+ * same arguments. */
 typedef struct marsmd_batch_launch {
     int32_t blocks_per_cu; /* persistent step-kernel workgroups per CU; 0: as many as fit */
     int32_t use_graph;     /* replay the steps between host decisions (rebuild checks,

@@ -364,8 +364,9 @@ __device__ __forceinline__ void b_stage_step(const BatchConsts& C, const StepPar
 
 // The fused step over every replica's particles, persistent over XCD-local tiles: the
 // replica of a slot gives its box and its seed mix. Bounded to 96 VGPRs (5 waves per
-// SIMD; no spills in the BD case, 2 dwords in the others): 160 -> 156.5 us at 512
-// replicas against 4 waves with 123 VGPRs.
+// SIMD; the analytical instances spill 16-21): 160 -> 156.5 us at 512 replicas against 4
+// waves with 123 VGPRs; with analytical terms 13 replicas of 40k beads take 188 us and 209
+// at 4 waves, 16 of them 246 and 243.
 template<int INTEG, bool ENERGY, bool ANALYTIC>
 __global__ __launch_bounds__(kBatchBlock, 5) void k_b_step(const float4* __restrict__ pos, float4* __restrict__ pos_next,
 														  float4* __restrict__ mom, float4* __restrict__ force,
@@ -1246,8 +1247,8 @@ void BatchImpl::run(const marsmd_run_params& P, uint64_t first_step, uint64_t nu
 void BatchImpl::autotune(const marsmd_run_params& P, uint64_t first_step, uint64_t num_steps, hipStream_t s,
 						 double* best_ms) {
 	// candidates: workgroups per CU from the occupancy down, each with and without
-	// segment replay; results do not depend on them (each particle's step is one lane's
-	// work, and a replay launches the same kernels with the same arguments)
+	// segment replay; results do not depend on them (each particle's sums are
+	// taken in one order, and a replay launches the same kernels with the same arguments)
 	const StepShape sh = step_shape();
 	(void)step_grid(reinterpret_cast<const void*>(pick_b_step(sh.split > 0, true, false, false)), sh);
 	std::vector<int> per_cu = {occupancy};

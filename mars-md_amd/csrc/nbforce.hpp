@@ -49,12 +49,17 @@ __device__ __forceinline__ uint32_t fb(float f) { return __float_as_uint(f); }
 // tabulated-only path carries none of the analytical code). `knots` points into LDS or
 // global memory, as the caller's instantiation says: a pointer that might be either
 // would be read with flat loads, whose waits also drain the position gathers in flight.
-// Returns what the pair adds to the slot's force and energy (+-0 from a pair that is skipped,
-// which leaves the sums' bits unchanged: they start at +0 and can never become -0).
-template<bool ANALYTIC>
-__device__ __forceinline__ float4 nb_pair_term(const float4& p, uint32_t ct, uint32_t tt, const float4& q,
-											   const NbTables& T, const float* __restrict__ knots, const NbLds& S,
-											   const DevBox& box, float cut_d, bool energy) {
+// Calls add(x, y, z, e) with what the pair adds to the slot's force and energy, unless it is
+// skipped (without ANALYTIC a skipped pair adds +-0, which leaves the sums' bits unchanged:
+// they start at +0 and can never become -0). The additions stand in the analytical terms'
+// branches: as a value merged behind them they cost the one-lane steps 9-12 VGPRs, at 5
+// waves 14-42 spilled ones instead of 4-9 (the batch's 54 instead of 16-21). Step, us, merged
+// and in the branches: 300k beads 139 and 137, with energies 153.5 and 147; 1M 379 and 376,
+// 417 and 404; 16 replicas of 40k 261 and 245, 280 and 268.
+template<bool ANALYTIC, class Add>
+__device__ __forceinline__ void nb_pair_add(const float4& p, uint32_t tt, const float4& q, const NbTables& T,
+											const float* __restrict__ knots, const NbLds& S, const DevBox& box,
+											float cut_d, bool energy, Add&& add) {
 	const uint32_t mj = fb(q.w);
 	const uint32_t tj = meta_type(mj);
 	// ct < cj, from the meta words (canonical index in the high bits; a pad entry is the
@@ -104,13 +109,13 @@ __device__ __forceinline__ float4 nb_pair_term(const float4& p, uint32_t ct, uin
 		// (force over distance once, then per axis: the product rounds in another order
 		// than fm * (r / d), a relative change of about 1e-7)
 		const float g = ((in_cut && d > 1e-6f) ? (t_is_x ? -fm : fm) : 0.0f) * inv;
-		return make_float4(g * r.x, g * r.y, g * r.z, energy && in_cut && !(d < 1e-6f) ? en * 0.5f : 0.0f);
+		add(g * r.x, g * r.y, g * r.z, energy && in_cut && !(d < 1e-6f) ? en * 0.5f : 0.0f);
+		return;
 	}
-	const float4 none = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 	const uint32_t tag = S.tag[(tx << 4) | ty];
 	const uint32_t terms = tag & T.enabled;
 	if (terms == 0u)
-		return none;
+		return;
 	const float3 r = wrap_diff(box, sub3(py, px));
 	const float r2 = len2(r);
 	const float d = sqrtf(r2);
@@ -122,7 +127,7 @@ __device__ __forceinline__ float4 nb_pair_term(const float4& p, uint32_t ct, uin
 		uz = inv * r.z;
 	}
 	if (d < 1e-6f || d > cut_d)
-		return none;
+		return;
 	float fm = 0.0f, en = 0.0f;
 	if (ANALYTIC && (terms & kAnalyticTerms)) {
 		const float4 cx = S.coef[tx], cy = S.coef[ty];
@@ -135,20 +140,32 @@ __device__ __forceinline__ float4 nb_pair_term(const float4& p, uint32_t ct, uin
 		en += v.e;
 	}
 	const float gx = fm * ux, gy = fm * uy, gz = fm * uz;
-	const float en_half = energy ? en * 0.5f : 0.0f;
-	return t_is_x ? make_float4(-gx, -gy, -gz, en_half) : make_float4(gx, gy, gz, en_half);
+	const float half = energy ? en * 0.5f : 0.0f;
+	if (t_is_x)
+		add(-gx, -gy, -gz, half);
+	else
+		add(gx, gy, gz, half);
 }
 template<bool ANALYTIC>
-__device__ __forceinline__ void nb_pair(const float4& p, uint32_t ct, uint32_t tt, const float4& q,
-										const NbTables& T, const float* __restrict__ knots, const NbLds& S,
-										const DevBox& box, float cut_d, bool energy, float& fx, float& fy,
-										float& fz, float& e) {
-	const float4 v = nb_pair_term<ANALYTIC>(p, ct, tt, q, T, knots, S, box, cut_d, energy);
-	fx += v.x;
-	fy += v.y;
-	fz += v.z;
-	if (energy)
-		e += v.w;
+__device__ __forceinline__ float4 nb_pair_term(const float4& p, uint32_t tt, const float4& q, const NbTables& T,
+											   const float* __restrict__ knots, const NbLds& S, const DevBox& box,
+											   float cut_d, bool energy) {
+	float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+	nb_pair_add<ANALYTIC>(p, tt, q, T, knots, S, box, cut_d, energy,
+						  [&](float x, float y, float z, float e) { v = make_float4(x, y, z, e); });
+	return v;
+}
+template<bool ANALYTIC>
+__device__ __forceinline__ void nb_pair(const float4& p, uint32_t tt, const float4& q, const NbTables& T,
+										const float* __restrict__ knots, const NbLds& S, const DevBox& box,
+										float cut_d, bool energy, float4& sum) {
+	nb_pair_add<ANALYTIC>(p, tt, q, T, knots, S, box, cut_d, energy, [&](float x, float y, float z, float e) {
+		sum.x += x;
+		sum.y += y;
+		sum.z += z;
+		if (energy)
+			sum.w += e;
+	});
 }
 
 // Position record of slot j, addressed by a 32-bit byte offset from the array base
@@ -166,12 +183,11 @@ __device__ __forceinline__ float4 nb_force_list(uint32_t t, const float4& p, con
 											   const NbrList& L, const NbTables& T, const float* __restrict__ knots,
 											   const NbLds& S, const DevBox& box, float cut_d, bool energy) {
 	const uint32_t mt = fb(p.w);
-	const uint32_t ct = meta_canon(mt);
 	const uint32_t tt = meta_type(mt);
-	float fx = 0.0f, fy = 0.0f, fz = 0.0f, e = 0.0f;
+	float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 	const uint32_t ng = (L.count[t] + 3u) >> 2;
 	if (ng == 0)
-		return make_float4(fx, fy, fz, e);
+		return sum;
 	const uint4* __restrict__ row = reinterpret_cast<const uint4*>(L.nbr + L.tile_base[t >> 6]) + (t & 63u);
 	// two register sets (a, b) take turns: while one group is evaluated the positions
 	// of the next are in flight in the other set, and the indices of the one after;
@@ -189,10 +205,10 @@ __device__ __forceinline__ float4 nb_force_list(uint32_t t, const float4& p, con
 			if (g + 2 < ng)
 				ja = row[uint64_t(g + 2) * 64u];
 		}
-		nb_pair<ANALYTIC>(p, ct, tt, a0, T, knots, S, box, cut_d, energy, fx, fy, fz, e);
-		nb_pair<ANALYTIC>(p, ct, tt, a1, T, knots, S, box, cut_d, energy, fx, fy, fz, e);
-		nb_pair<ANALYTIC>(p, ct, tt, a2, T, knots, S, box, cut_d, energy, fx, fy, fz, e);
-		nb_pair<ANALYTIC>(p, ct, tt, a3, T, knots, S, box, cut_d, energy, fx, fy, fz, e);
+		nb_pair<ANALYTIC>(p, tt, a0, T, knots, S, box, cut_d, energy, sum);
+		nb_pair<ANALYTIC>(p, tt, a1, T, knots, S, box, cut_d, energy, sum);
+		nb_pair<ANALYTIC>(p, tt, a2, T, knots, S, box, cut_d, energy, sum);
+		nb_pair<ANALYTIC>(p, tt, a3, T, knots, S, box, cut_d, energy, sum);
 		if (g + 1 >= ng)
 			break;
 		if (g + 2 < ng) {
@@ -203,14 +219,14 @@ __device__ __forceinline__ float4 nb_force_list(uint32_t t, const float4& p, con
 			if (g + 3 < ng)
 				jb = row[uint64_t(g + 3) * 64u];
 		}
-		nb_pair<ANALYTIC>(p, ct, tt, b0, T, knots, S, box, cut_d, energy, fx, fy, fz, e);
-		nb_pair<ANALYTIC>(p, ct, tt, b1, T, knots, S, box, cut_d, energy, fx, fy, fz, e);
-		nb_pair<ANALYTIC>(p, ct, tt, b2, T, knots, S, box, cut_d, energy, fx, fy, fz, e);
-		nb_pair<ANALYTIC>(p, ct, tt, b3, T, knots, S, box, cut_d, energy, fx, fy, fz, e);
+		nb_pair<ANALYTIC>(p, tt, b0, T, knots, S, box, cut_d, energy, sum);
+		nb_pair<ANALYTIC>(p, tt, b1, T, knots, S, box, cut_d, energy, sum);
+		nb_pair<ANALYTIC>(p, tt, b2, T, knots, S, box, cut_d, energy, sum);
+		nb_pair<ANALYTIC>(p, tt, b3, T, knots, S, box, cut_d, energy, sum);
 		if (g + 2 >= ng)
 			break;
 	}
-	return make_float4(fx, fy, fz, e);
+	return sum;
 }
 
 // LDS written by some lanes of this wave and read by others: order the accesses.
@@ -282,7 +298,6 @@ __device__ __forceinline__ float nb_force_split(const RowHead& h, uint32_t sub, 
 												float cut_d, bool energy, float* terms) {
 	const float4 p = h.p;
 	const uint32_t mt = fb(p.w);
-	const uint32_t ct = meta_canon(mt);
 	const uint32_t tt = meta_type(mt);
 	const uint32_t m = 1u << split, ng = h.ng, lane = threadIdx.x & 63u;
 	const uint32_t row = 4u * m + 4u, comp = (64u >> split) * row;
@@ -297,10 +312,10 @@ __device__ __forceinline__ float nb_force_split(const RowHead& h, uint32_t sub, 
 		j = h.self;
 		if (g0 + m + sub < ng)
 			j = h.row[uint64_t(g0 + m + sub) * 64u];
-		const float4 t0 = nb_pair_term<ANALYTIC>(p, ct, tt, q0, T, knots, S, box, cut_d, energy);
-		const float4 t1 = nb_pair_term<ANALYTIC>(p, ct, tt, q1, T, knots, S, box, cut_d, energy);
-		const float4 t2 = nb_pair_term<ANALYTIC>(p, ct, tt, q2, T, knots, S, box, cut_d, energy);
-		const float4 t3 = nb_pair_term<ANALYTIC>(p, ct, tt, q3, T, knots, S, box, cut_d, energy);
+		const float4 t0 = nb_pair_term<ANALYTIC>(p, tt, q0, T, knots, S, box, cut_d, energy);
+		const float4 t1 = nb_pair_term<ANALYTIC>(p, tt, q1, T, knots, S, box, cut_d, energy);
+		const float4 t2 = nb_pair_term<ANALYTIC>(p, tt, q2, T, knots, S, box, cut_d, energy);
+		const float4 t3 = nb_pair_term<ANALYTIC>(p, tt, q3, T, knots, S, box, cut_d, energy);
 		wave_lds_order(); // (the last round's reads)
 		*reinterpret_cast<float4*>(mine) = make_float4(t0.x, t1.x, t2.x, t3.x);
 		*reinterpret_cast<float4*>(mine + comp) = make_float4(t0.y, t1.y, t2.y, t3.y);

@@ -385,8 +385,10 @@ __device__ __forceinline__ void stage_step(const marsmd_particle_types& types, c
 
 // The fused step: nonbonded + bonded (from `force` when has_bonded) + PMF + integrator,
 // persistent over XCD-local tiles so the table knots are staged once per workgroup.
-// Bounded to 128 VGPRs (4 waves per SIMD; the tricubic sampler alone would take ~140
-// and leave 3): measured faster despite a few dwords of spill.
+// Bounded to 96 VGPRs (5 waves per SIMD: the tabulated term takes 76-80, the analytical ones
+// spill 4-9; at 4 waves without spills 520k beads with them take 215 us instead of 189, 1M
+// 392 instead of 377, 300k 135 and 137), with the tricubic sampler, which alone would take
+// about 140, to 128 (4 waves).
 template<int INTEG, bool ENERGY, bool ANALYTIC, int PMF>
 __global__ __launch_bounds__(kBlock, PMF == kPmfCubic ? 4 : 5) void k_step(const float4* __restrict__ pos, float4* __restrict__ pos_next,
 												 float4* __restrict__ mom, float4* __restrict__ force, uint64_t n,

@@ -146,3 +146,26 @@ def test_the_kernels_that_run(cuda, n, lanes_kernel, given):
     assert sum("k_pmf_force" in x for x in names) == (3 if given else 0), names
     # the fourth template argument: sampled linearly here (1) or given (3)
     assert all(re.search(r"<[^,]*, [^,]*, [^,]*, (\d)", x).group(1) == ("3" if given else "1") for x in steps), steps
+
+
+@pytest.mark.parametrize("energy", [0, 2])
+@pytest.mark.parametrize("case", ["brownian_table", "brownian_analytic", "langevin_analytic"])
+def test_batch_replicas_have_the_bits_of_patches(cuda, case, energy):
+    # 5 replicas together take one lane a row, each as a Patch four
+    from marsmd.batch import Batch
+
+    specs = []
+    for r, n in enumerate([24_000, 23_999, 20_011, 25_000, 24_001]):
+        spec = CASES[case](n=n, L=(n / 1.25e-4) ** (1.0 / 3.0))
+        spec.patch_id, spec.params.energy_period, spec.params.rebuild_period = r, energy, 3
+        spec.params.timestep /= 50.0
+        specs.append(spec)
+    assert sum(s.n for s in specs) > LIMIT
+    print("case:", case, energy, flush=True)
+    b = Batch(specs)
+    b.run(6)
+    for r, (spec, got) in enumerate(zip(specs, b.copy_particles_to_host())):
+        p = marsmd.Patch(spec)
+        p.run(6)
+        for k, want in _state(p).items():
+            assert np.array_equal(got[k].view(np.uint32), want), f"{k} of replica {r}"
