@@ -187,19 +187,13 @@ __global__ void k_b_cell_ranges(const uint32_t* __restrict__ codes, uint64_t tot
 		home[G.home_off + hc].y = uint32_t(i + 1);
 }
 
-// The stencils' lists, one a workgroup. A stencil of more cells than are sorted has one list,
-// which is its own order.
+// The stencils' lists in row order, one a workgroup (see stencil_list).
 __global__ __launch_bounds__(256) void k_b_stencil_lists(const StencilList* __restrict__ lists,
 														 const int4* __restrict__ offsets,
 														 uint32_t* __restrict__ codes) {
-	__shared__ uint64_t keys[kStencilSortMax];
+	__shared__ uint64_t keys[kStencilMax];
 	const StencilList l = lists[blockIdx.x];
-	if (l.n <= kStencilSortMax) {
-		stencil_list(offsets + l.first, l.n, int(l.level), l.position, codes + l.out, keys);
-		return;
-	}
-	for (uint32_t i = threadIdx.x; i < l.n; i += 256u)
-		codes[l.out + i] = stencil_offset_code(offsets[l.first + i], int(l.level));
+	stencil_list(offsets + l.first, l.n, int(l.level), l.position, l.by_slot != 0u, codes + l.out, keys);
 }
 
 // The home-cell walk over the work items of all replicas (item_off[r] = first item of
@@ -812,7 +806,7 @@ void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<ui
 		}
 		const bool per[3] = {true, true, true};
 		const WalkGrid w = walk_grid(n, m, cell_target[size_t(bucket)], cell_fine[size_t(bucket)],
-									 kWalkFill * double(n) / double(total), 4, g.lo, g.hi, per, double(rc), rc2);
+									 kWalkFill * double(n) / double(total), 0.0, 4, g.lo, g.hi, per, double(rc), rc2);
 		const int h = w.h;
 		g.h = h;
 		g.mf = w.mf;
@@ -846,18 +840,19 @@ void BatchImpl::plan_geometry(float rc, std::vector<uint8_t>& gh, std::vector<ui
 										float(g.full[1]),  float(g.full[2]),   g.cw[0],
 										g.cw[1],		   g.cw[2],			   g.margin[0],
 										g.margin[1],	   g.margin[2],		   rc2,
-										float(w.lists)};
+										float(w.lists),	   w.by_slot ? 1.0f : 0.0f};
 		auto it = stencil_index.find(key);
 		if (it == stencil_index.end()) {
 			const std::vector<int4> st = g.mf < h ? std::vector<int4>{make_int4(0, 0, 0, 0)}
-												  : home_stencil(h, g.mf - h, g.reach, g.full, g.cw, g.margin, rc2, 8192);
+												  : home_stencil(h, g.mf - h, g.reach, g.full, g.cw, g.margin, rc2, kStencilMax);
 			const uint32_t cells = uint32_t(st.size());
 			if (stencil_codes + uint64_t(cells) * w.lists >= (uint64_t(1) << 32))
 				raise(MARSMD_ERR_VALUE, "batch: stencils exceed 2^32 entries");
 			it = stencil_index.emplace(key, std::make_pair(uint32_t(stencil_codes), cells)).first;
 			for (uint32_t b = 0; b < (cells > 0 ? w.lists : 0u); ++b) {
 				stencil_lists_host.push_back(StencilList{uint32_t(stencil_cells_host.size()), cells,
-														 uint32_t(stencil_codes), uint32_t(g.mf), b});
+														 uint32_t(stencil_codes), uint32_t(g.mf), b,
+														 w.by_slot ? 1u : 0u});
 				stencil_codes += cells;
 			}
 			stencil_cells_host.insert(stencil_cells_host.end(), st.begin(), st.end());

@@ -20,7 +20,7 @@ int batch_size_bucket(uint64_t n);
 // A stencil's list of codes for one position of a home cell (see stencil_list).
 struct StencilList {
 	uint32_t first, n, out; // its offsets, its codes
-	uint32_t level, position;
+	uint32_t level, position, by_slot;
 };
 
 struct BatchImpl {

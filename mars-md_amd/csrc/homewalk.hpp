@@ -196,29 +196,33 @@ inline WalkLevel walk_level(uint64_t n, int m, int target, int offset, double fi
 // Rows list a particle's neighbours by the Morton order of their offsets from the
 // particle's cell at the level that holds kRowTarget particles per cell on average (by slot
 // where that level's stencil wraps onto itself on every axis), whatever level the walk runs
-// at: the FP32 sum over a row is then the same bits. Where the cells were set, and in boxes
-// with an open axis, a row is in the order of the walk's own cells.
+// at: the FP32 sum over a row is then the same bits. Where the cells were set, in boxes with
+// an open axis and where that stencil wraps on one or two axes only (which the order level
+// walks slowly: a build of 60k in 300 x 300 x 60 at cutoff 28 takes 6400 us there, 720 here), a
+// row is in the order of the walk's own cells.
 constexpr int kRowTarget = kCellsTarget, kRowOffset = kCellsOffset;
-// particles up to which rows by slot come from walking the whole box (n / 64 candidate
-// blocks a home cell)
-constexpr uint64_t kWholeBoxMax = 16384;
-// cells of a stencil that is listed once for each position of a home cell in its cell of the
-// order level (see k_stencil_lists)
-constexpr uint32_t kStencilSortMax = 2048;
+// cells of a stencil; a larger one is not listed, the walk then tests every cell of its reach
+constexpr uint32_t kStencilMax = 8192;
+
+// home levels at which a stencil may have a list for every home cell (512 of a few hundred)
+constexpr int kSlotListLevel = 3;
 
 // The cells of a walk: home cells of level h; fine cells of level mf with their enumeration
 // (mf < h: one fine cell, the whole box); the lists its stencil has
-// (HomeParams::stencil_lists + 1).
+// (HomeParams::stencil_lists + 1), by_slot: in the order of the cells themselves.
 struct WalkGrid {
 	int h, mf;
 	uint32_t lists;
+	bool by_slot;
 	int reach[3], full[3];
 	float cw[3], margin[3];
 };
 // The grid for n particles in the Morton domain [lo, hi), periodic where `per`, with build
-// levels up to m and the cell configuration given (see walk_level for fill and per_cell).
-inline WalkGrid walk_grid(uint64_t n, int m, int home_target, int fine_offset, double fill, uint64_t per_cell,
-						  const float lo[3], const float hi[3], const bool per[3], double rc, float rc2) {
+// levels up to m and the cell configuration given (see walk_level for fill and per_cell;
+// own_fill: the fill where rows follow the walk's own cells).
+inline WalkGrid walk_grid(uint64_t n, int m, int home_target, int fine_offset, double fill, double own_fill,
+						  uint64_t per_cell, const float lo[3], const float hi[3], const bool per[3], double rc,
+						  float rc2) {
 	const auto extent = [&](int a) { return std::fmax(hi[a] - lo[a], 1e-6f); };
 	// fine cells of level `mf` beyond a home cell that cover rc with the seam slack of the
 	// quantised top cell, and whether such a stencil wraps onto itself on the axis
@@ -244,25 +248,61 @@ inline WalkGrid walk_grid(uint64_t n, int m, int home_target, int fine_offset, d
 		}
 		return g;
 	};
-	const bool own = cells_auto(home_target, fine_offset);
-	WalkLevel lv = walk_level(n, m, own ? 0 : home_target, fine_offset, fill, per_cell);
-	if (!own || !(per[0] && per[1] && per[2]))
-		return grid_of(lv);
+	// whether the home frame of a cell of level h gives minimum images (home_prefilter_band)
+	const auto frames = [&](int h) {
+		for (int a = 0; a < 3; ++a)
+			if (per[a] && !(0.5f * extent(a) > extent(a) / float(1 << h) + float(rc) + 0.01f * extent(a) + 1.0f))
+				return false;
+		return true;
+	};
+	// The library's own level. Without the home frame each test takes the whole predicate and
+	// no candidate is dropped before, so one level finer where that has the frame and the
+	// cells to choose from (a build of 120k in 300 x 300 x 60 at cutoff 25: 2440 -> 725 us),
+	// or where its cells still hold 2 particles and leave out some of the box (the same at
+	// cutoff 27: 2440 -> 1510 us; 128 replicas of 900 that test all their particles anyway:
+	// 340 -> 432 us a step with a build, and with 0.6 particles a cell 512 of 300: 157 -> 288).
+	const auto own_level = [&](double f, bool prunes) {
+		WalkLevel l = walk_level(n, m, 0, 0, f, per_cell);
+		if (l.h < m && !frames(l.h) &&
+			((frames(l.h + 1) && double(uint64_t(1) << (3 * l.h)) <= f) || (prunes && (n >> (3 * l.h)) >= 16)))
+			++l.h;
+		return l;
+	};
+	if (!cells_auto(home_target, fine_offset))
+		return grid_of(walk_level(n, m, home_target, fine_offset, fill, per_cell));
+	if (!(per[0] && per[1] && per[2]))
+		return grid_of(own_level(own_fill, true));
 	const WalkGrid order = grid_of(walk_level(n, m, kRowTarget, kRowOffset, 0.0));
 	const int full_axes = order.full[0] + order.full[1] + order.full[2];
-	if (full_axes == 3 && n <= kWholeBoxMax) {
-		lv.s = -lv.h; // rows by slot: every particle is a candidate, in slot order
+	WalkLevel lv = own_level(full_axes == 1 || full_axes == 2 ? own_fill : fill, full_axes < 3);
+	WalkGrid g = grid_of(lv);
+	if (full_axes == 3) {
+		// rows by slot: every particle is a candidate, in slot order; where the walk fills the
+		// chip and its stencil does not wrap, the stencil's cells in their own order, a list
+		// for each home cell (2000 replicas of 500: a step with its build 488 -> 456 us)
+		if (lv.h <= kSlotListLevel && double(uint64_t(1) << (3 * lv.h)) > fill && !g.full[0] && !g.full[1] &&
+			!g.full[2]) {
+			g.lists = 1u << (3 * lv.h);
+			g.by_slot = true;
+			return g;
+		}
+		lv.s = -lv.h;
 		return grid_of(lv);
 	}
-	WalkGrid g = grid_of(lv);
-	if (full_axes > 0 || g.full[0] || g.full[1] || g.full[2])
-		return order; // offsets and absolute cells mixed: the order level's own walk
+	if (full_axes > 0)
+		return g;
+	if (g.full[0] || g.full[1] || g.full[2])
+		return order; // (offsets and absolute cells mixed)
 	if (g.h > order.h) {
+		uint64_t reached = 1;
+		for (int a = 0; a < 3; ++a)
+			reached *= uint64_t(1 << (g.mf - g.h)) + 2u * uint64_t(g.reach[a]);
 		uint32_t cells = 0;
-		for_each_stencil_cell(g.h, g.mf - g.h, g.reach, g.full, g.cw, g.margin, rc2,
-							  [&](const int4&) { return ++cells <= kStencilSortMax; });
-		if (cells > kStencilSortMax)
-			return order; // (more than 500 neighbours a particle)
+		if (reached > kStencilMax)
+			for_each_stencil_cell(g.h, g.mf - g.h, g.reach, g.full, g.cw, g.margin, rc2,
+								  [&](const int4&) { return ++cells <= kStencilMax; });
+		if (cells > kStencilMax)
+			return order;
 		g.lists = 1u << (3 * (g.h - order.h));
 	}
 	return g;
@@ -278,13 +318,17 @@ __host__ __device__ inline uint32_t stencil_offset_code(const int4& o, int level
 // List b of a stencil in row order: its n offsets (relative to a home cell of `level`) in the
 // Morton order of the cells' offsets from the home cell's ancestor of the order level,
 // within which the home cell lies at the position whose Morton code is b, as codes
-// (stencil_offset_code). Ranks by counting (a few hundred cells; no two keys are equal), by a
+// (stencil_offset_code); by_slot: b is the home cell, in the Morton order of the cells. Ranks by counting (a few hundred cells; no two keys are equal), by a
 // workgroup with `keys` in LDS.
-__device__ inline void stencil_list(const int4* __restrict__ offsets, uint32_t n, int level, uint32_t b,
+__device__ inline void stencil_list(const int4* __restrict__ offsets, uint32_t n, int level, uint32_t b, bool by_slot,
 									uint32_t* __restrict__ codes, uint64_t* keys) {
 	const int p[3] = {int(compact_by3(b >> 2)), int(compact_by3(b >> 1)), int(compact_by3(b))};
 	for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) {
 		const int4 o = offsets[i];
+		if (by_slot) {
+			keys[i] = stencil_offset_code(make_int4(p[0] + o.x, p[1] + o.y, p[2] + o.z, 0), level);
+			continue;
+		}
 		const uint32_t v[3] = {uint32_t(p[0] + o.x + 1024), uint32_t(p[1] + o.y + 1024), uint32_t(p[2] + o.z + 1024)};
 		keys[i] = (uint64_t(((v[0] >> 10) & 1u) << 2 | ((v[1] >> 10) & 1u) << 1 | ((v[2] >> 10) & 1u)) << 30) |
 				  (split_by3(v[0]) << 2 | split_by3(v[1]) << 1 | split_by3(v[2]));

@@ -200,9 +200,9 @@ __global__ void k_walk_cells(const uint32_t* __restrict__ codes, uint64_t n, int
 
 // The walk's stencil lists in row order, one a workgroup (see stencil_list).
 __global__ __launch_bounds__(256) void k_stencil_lists(const int4* __restrict__ offsets, uint32_t n, int level,
-													   uint32_t* __restrict__ codes) {
-	__shared__ uint64_t keys[kStencilSortMax];
-	stencil_list(offsets, n, level, blockIdx.x, codes + uint64_t(blockIdx.x) * n, keys);
+													   int by_slot, uint32_t* __restrict__ codes) {
+	__shared__ uint64_t keys[kStencilMax];
+	stencil_list(offsets, n, level, blockIdx.x, by_slot != 0, codes + uint64_t(blockIdx.x) * n, keys);
 }
 
 // BuildCellNeighborsKernel (ZOrderNeighbor.h:55-139), for the reference tables.
@@ -777,8 +777,9 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 	const bool per[3] = {box.periodic[0] != 0 && box.size[0] > 0.0f, box.periodic[1] != 0 && box.size[1] > 0.0f,
 						 box.periodic[2] != 0 && box.size[2] > 0.0f};
 	const bool wraps = per[0] && per[1] && per[2];
-	const WalkGrid grid_cells = walk_grid(n, m, home_target, fine_offset, kWalkFill, excl.offsets ? 2 : 4, domain_min,
-										  domain_max, per, std::sqrt(double(cutoff_squared)), cutoff_squared);
+	const WalkGrid grid_cells = walk_grid(n, m, home_target, fine_offset, kWalkFill, kWalkFill, excl.offsets ? 2 : 4,
+										  domain_min, domain_max, per, std::sqrt(double(cutoff_squared)),
+										  cutoff_squared);
 	const int h = grid_cells.h, mf = grid_cells.mf;
 	const uint32_t lists = grid_cells.lists;
 	const uint64_t tiles = (n + 63) / 64;
@@ -821,11 +822,11 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 									float(P.reach[2]), float(P.full[0]),   float(P.full[1]),  float(P.full[2]),
 									P.cw[0],		   P.cw[1],			   P.cw[2],			  P.margin[0],
 									P.margin[1],	   P.margin[2],		   P.rc2,			  wraps ? 1.0f : 0.0f,
-									float(lists)};
+									float(lists),	   grid_cells.by_slot ? 1.0f : 0.0f};
 	if (key != stencil_key) {
 		stencil_key.clear(); // until it is made
 		const std::vector<int4> cells = mf < h ? std::vector<int4>{make_int4(0, 0, 0, 0)}
-											   : home_stencil(h, P.s, P.reach, P.full, P.cw, P.margin, P.rc2, 8192);
+											   : home_stencil(h, P.s, P.reach, P.full, P.cw, P.margin, P.rc2, kStencilMax);
 		stencil_n = uint32_t(cells.size());
 		stencil_lists = lists;
 		if (stencil_n > 0 && (!wraps || stencil_lists > 1)) {
@@ -835,7 +836,8 @@ bool PairlistImpl::walk_home(hipStream_t s, bool& outside) {
 		if (stencil_n > 0 && wraps) {
 			stencil_codes.resize(uint64_t(stencil_n) * stencil_lists);
 			if (stencil_lists > 1) {
-				k_stencil_lists<<<stencil_lists, 256, 0, s>>>(stencil_dev.data(), stencil_n, mf, stencil_codes.data());
+				k_stencil_lists<<<stencil_lists, 256, 0, s>>>(stencil_dev.data(), stencil_n, mf, grid_cells.by_slot ? 1 : 0,
+															  stencil_codes.data());
 				MMD_LAUNCH_CHECK();
 			} else {
 				std::vector<uint32_t> words;

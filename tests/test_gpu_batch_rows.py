@@ -43,3 +43,26 @@ def test_a_replica_keeps_its_bits(cuda, sizes, density, integrator):
         for k in KEYS:
             assert np.array_equal(together[r][k], alone[k]), f"{k} of {s.n} beads in a batch"
             assert np.array_equal(together[r][k], patch[k]), f"{k} of {s.n} beads against a Patch"
+
+
+@pytest.mark.parametrize("replicas", [3, 40, 200])
+@pytest.mark.parametrize("n,density", [(500, 1e-4), (300, 1e-4), (1600, 8e-4)])
+def test_a_replica_keeps_its_bits_in_a_crowd(cuda, n, density, replicas):
+    # more replicas, coarser cells each: whole boxes, then a list for each home cell
+    base = configs.config3(replicas=1, n_min=n, n_max=n, density=density, seed=29)[0]
+    specs = []
+    for r in range(replicas):
+        s = dataclasses.replace(base, patch_id=r, params=dataclasses.replace(
+            base.params, timestep=base.params.timestep / 100.0, rebuild_period=5))
+        s.positions = configs.uniform_positions(n, base.box.size[0], 100 + r)
+        specs.append(s)
+    print("case:", n, density, replicas, flush=True)
+    b = Batch(specs)
+    b.run(7)
+    together = b.copy_particles_to_host()
+    for r in (0, replicas - 1):
+        p = marsmd.Patch(specs[r])
+        p.run(7)
+        patch = p.copy_particles_to_host()
+        for k in KEYS:
+            assert np.array_equal(together[r][k], patch[k]), f"{k} of replica {r}"
