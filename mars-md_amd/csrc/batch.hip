@@ -1062,18 +1062,26 @@ BatchImpl::StepShape BatchImpl::step_shape() const {
 	return sh;
 }
 
+// Workgroups per CU of a step kernel (its instances hold different LDS and registers).
+int BatchImpl::step_occupancy(const void* kernel, const StepShape& sh) {
+	auto it = occupancy.find(kernel);
+	if (it == occupancy.end() || it->second.first != sh.lds) {
+		int occ = 0;
+		MMD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, kernel, int(sh.block), sh.lds));
+		it = occupancy.insert_or_assign(kernel, std::make_pair(sh.lds, std::max(occ, 1))).first;
+	}
+	return it->second.second;
+}
+
 unsigned BatchImpl::step_grid(const void* kernel, const StepShape& sh) {
-	if (occupancy == 0 || occupancy_lds != sh.lds || occupancy_block != sh.block) {
-		MMD_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occupancy, kernel, int(sh.block), sh.lds));
-		occupancy = std::max(occupancy, 1);
-		occupancy_lds = sh.lds;
-		occupancy_block = sh.block;
+	const int occ = step_occupancy(kernel, sh);
+	if (num_cus == 0) {
 		int dev = 0;
 		MMD_HIP(hipGetDevice(&dev));
 		MMD_HIP(hipDeviceGetAttribute(&num_cus, hipDeviceAttributeMultiprocessorCount, dev));
 		num_cus = std::max(num_cus, 1);
 	}
-	const int per_cu = blocks_per_cu > 0 ? std::min(blocks_per_cu, occupancy) : occupancy;
+	const int per_cu = blocks_per_cu > 0 ? std::min(blocks_per_cu, occ) : occ;
 	uint64_t g = std::min<uint64_t>(uint64_t(per_cu) * uint64_t(num_cus), (sh.tiles + 7) / 8 * 8);
 	return unsigned(std::max<uint64_t>((g + 7) / 8 * 8, 8));
 }
@@ -1245,9 +1253,11 @@ void BatchImpl::autotune(const marsmd_run_params& P, uint64_t first_step, uint64
 	// segment replay; results do not depend on them (each particle's sums are
 	// taken in one order, and a replay launches the same kernels with the same arguments)
 	const StepShape sh = step_shape();
-	(void)step_grid(reinterpret_cast<const void*>(pick_b_step(sh.split > 0, true, false, false)), sh);
-	std::vector<int> per_cu = {occupancy};
-	for (int v : {occupancy - 1, occupancy / 2, 1})
+	const bool bd = P.integrator == MARSMD_INTEGRATOR_BROWNIAN;
+	const bool an = (tables->enabled & kAnalyticTerms) != 0;
+	const int occ = step_occupancy(reinterpret_cast<const void*>(pick_b_step(sh.split > 0, bd, false, an)), sh);
+	std::vector<int> per_cu = {occ};
+	for (int v : {occ - 1, occ / 2, 1})
 		if (v >= 1 && std::find(per_cu.begin(), per_cu.end(), v) == per_cu.end())
 			per_cu.push_back(v);
 	struct Cand {

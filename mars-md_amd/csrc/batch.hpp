@@ -85,8 +85,8 @@ struct BatchImpl {
 	std::vector<hipEvent_t> timing_events;
 	std::vector<uint64_t> timing_steps;
 	size_t timing_used = 0;
-	int occupancy = 0, num_cus = 0; // of the step kernel launched with
-	unsigned occupancy_lds = 0, occupancy_block = 0;
+	std::map<const void*, std::pair<unsigned, int>> occupancy; // of a step kernel, with its dynamic LDS
+	int num_cus = 0;
 	// launch configuration: persistent step-kernel workgroups per CU (0: as many as
 	// fit) and whether runs of steps that need no host decision replay as hipGraphs
 	int blocks_per_cu = 0;
@@ -148,6 +148,7 @@ struct BatchImpl {
 		uint32_t split = 0, knot_words = 0;
 	};
 	StepShape step_shape() const;
+	int step_occupancy(const void* kernel, const StepShape& shape);
 	unsigned step_grid(const void* kernel, const StepShape& shape);
 	// count consecutive steps from `first` with the current list; `store` keeps the
 	// forces of the last one
