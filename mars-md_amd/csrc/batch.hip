@@ -577,16 +577,6 @@ struct SegmentKey {
 	StepParams S;
 };
 
-// Ready for a walk: the cell tables cleared and the uniform rows' bases.
-__global__ void k_b_walk_setup(uint2* __restrict__ cells, uint64_t num_cells, uint32_t* __restrict__ tile_base,
-							   uint64_t tiles, uint32_t row) {
-	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (i < num_cells)
-		cells[i] = make_uint2(0u, 0u);
-	if (i <= tiles)
-		tile_base[i] = uint32_t(i * row);
-}
-
 } // namespace
 
 BatchImpl::BatchImpl(const marsmd_batch_desc& d) : tables(new NbTables{}) {
@@ -976,7 +966,7 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 		const double mean = double(total) / vol * 4.0 / 3.0 * 3.141592653589793 * double(rc) * rc * rc;
 		cap = uint32_t(std::min(1.6 * mean + 16.0, 4096.0) + 3) & ~3u;
 	}
-	k_b_walk_setup<<<grid_for(std::max(num_fine + num_home, tiles + 1), 256), 256, 0, s>>>(
+	k_walk_setup<<<grid_for(std::max(num_fine + num_home, tiles + 1), 256), 256, 0, s>>>(
 		fine, num_fine + num_home, tile_base.data(), tiles, 64u * cap);
 	MMD_LAUNCH_CHECK();
 	k_b_cell_ranges<<<grid_for(total, 256), 256, 0, s>>>(codes.data(), total, rep_of_slot.data(), gd, fine, home,
@@ -991,7 +981,7 @@ void BatchImpl::build(float pairlist_cutoff, bool relabel, hipStream_t s) {
 		if (storage > nbr.count)
 			nbr.resize(storage + storage / 8 + 1024);
 		if (attempt > 0) { // larger rows
-			k_b_walk_setup<<<grid_for(tiles + 1, 256), 256, 0, s>>>(nullptr, 0, tile_base.data(), tiles, 64u * cap);
+			k_walk_setup<<<grid_for(tiles + 1, 256), 256, 0, s>>>(nullptr, 0, tile_base.data(), tiles, 64u * cap);
 			MMD_LAUNCH_CHECK();
 		}
 		k_b_walk<<<grid, 256, 0, s>>>(gd, item_off.data(), uint32_t(R), uint32_t(num_items), pos[cur].data(),

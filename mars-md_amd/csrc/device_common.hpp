@@ -763,4 +763,11 @@ __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
 	return dpp_add<0x143, 0xc>(v); // row_bcast:31 into rows 2 and 3
 }
 
+// LDS written by some lanes of this wave and read by others: order the accesses.
+__device__ __forceinline__ void wave_lds_sync() {
+	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+	__builtin_amdgcn_wave_barrier();
+	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 } // namespace mmd

@@ -420,12 +420,6 @@ __device__ __forceinline__ uint32_t bits_below(uint64_t m) {
 __device__ __forceinline__ void set_lane(uint32_t& v, uint32_t x, uint32_t i) {
 	asm("v_writelane_b32 %0, %1, %2" : "+v"(v) : "s"(x), "{m0}"(i));
 }
-// LDS written by some lanes of this wave and read by others: order the accesses.
-__device__ __forceinline__ void wave_lds_sync() {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // LDS of one wave of the walk.
 struct WalkLds {
@@ -808,6 +802,17 @@ __global__ __launch_bounds__(256, 6) void k_walk_home(HomeParams P, uint32_t* __
 			}
 		}
 	}
+}
+
+// Ready for a walk: the cell tables cleared and the uniform rows' bases
+// (tile_base[w] = w * row for w in [0, tiles], rows of `row` entries per tile).
+__global__ void k_walk_setup(uint2* __restrict__ cells, uint64_t num_cells, uint32_t* __restrict__ tile_base,
+							 uint64_t tiles, uint32_t row) {
+	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+	if (i < num_cells)
+		cells[i] = make_uint2(0u, 0u);
+	if (i <= tiles)
+		tile_base[i] = uint32_t(i * row);
 }
 
 } // namespace

@@ -229,13 +229,6 @@ __device__ __forceinline__ float4 nb_force_list(uint32_t t, const float4& p, con
 	return sum;
 }
 
-// LDS written by some lanes of this wave and read by others: order the accesses.
-__device__ __forceinline__ void wave_lds_order() {
-	__builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-	__builtin_amdgcn_wave_barrier();
-	__builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // The same sum with each slot's row dealt to m = 2^split adjacent lanes (4 or 8; this one's
 // index `sub`): a round takes m groups of 4 entries, lane k evaluates group k's
 // pairs and leaves their terms in LDS, and then four lanes per slot, one a component, add
@@ -316,13 +309,13 @@ __device__ __forceinline__ float nb_force_split(const RowHead& h, uint32_t sub, 
 		const float4 t1 = nb_pair_term<ANALYTIC>(p, tt, q1, T, knots, S, box, cut_d, energy);
 		const float4 t2 = nb_pair_term<ANALYTIC>(p, tt, q2, T, knots, S, box, cut_d, energy);
 		const float4 t3 = nb_pair_term<ANALYTIC>(p, tt, q3, T, knots, S, box, cut_d, energy);
-		wave_lds_order(); // (the last round's reads)
+		wave_lds_sync(); // (the last round's reads)
 		*reinterpret_cast<float4*>(mine) = make_float4(t0.x, t1.x, t2.x, t3.x);
 		*reinterpret_cast<float4*>(mine + comp) = make_float4(t0.y, t1.y, t2.y, t3.y);
 		*reinterpret_cast<float4*>(mine + 2u * comp) = make_float4(t0.z, t1.z, t2.z, t3.z);
 		if (energy)
 			*reinterpret_cast<float4*>(mine + 3u * comp) = make_float4(t0.w, t1.w, t2.w, t3.w);
-		wave_lds_order();
+		wave_lds_sync();
 		if (adds) {
 			for (uint32_t k = 0; k < m; k += 4) {
 				float4 v[4];

@@ -456,17 +456,6 @@ __global__ __launch_bounds__(kStatBlock) void k_count_stats(const uint32_t* __re
 	}
 }
 
-// Ready for a walk: the cell tables cleared and the uniform rows' bases
-// (tile_base[w] = w * row for w in [0, tiles], rows of `row` entries per tile).
-__global__ void k_walk_setup(uint2* __restrict__ cells, uint64_t num_cells, uint32_t* __restrict__ tile_base,
-							 uint64_t tiles, uint32_t row) {
-	const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-	if (i < num_cells)
-		cells[i] = make_uint2(0u, 0u);
-	if (i <= tiles)
-		tile_base[i] = uint32_t(i * row);
-}
-
 __global__ void k_half_counts(NbrList L, uint64_t n, uint32_t* __restrict__ half) {
 	const uint64_t t = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
 	if (t >= n)
