@@ -198,8 +198,8 @@ inline WalkLevel walk_level(uint64_t n, int m, int target, int offset, double fi
 // where that level's stencil wraps onto itself on every axis), whatever level the walk runs
 // at: the FP32 sum over a row is then the same bits. Where the cells were set, in boxes with
 // an open axis and where that stencil wraps on one or two axes only (which the order level
-// walks slowly: a build of 60k in 300 x 300 x 60 at cutoff 28 takes 6400 us there, 720 here), a
-// row is in the order of the walk's own cells.
+// walks slowly: a build of 60k in 300 x 300 x 60 at cutoff 28 takes 6360 us there, 1060 here),
+// a row is in the order of the walk's own cells.
 constexpr int kRowTarget = kCellsTarget, kRowOffset = kCellsOffset;
 // cells of a stencil; a larger one is not listed, the walk then tests every cell of its reach
 constexpr uint32_t kStencilMax = 8192;
@@ -318,8 +318,9 @@ __host__ __device__ inline uint32_t stencil_offset_code(const int4& o, int level
 // List b of a stencil in row order: its n offsets (relative to a home cell of `level`) in the
 // Morton order of the cells' offsets from the home cell's ancestor of the order level,
 // within which the home cell lies at the position whose Morton code is b, as codes
-// (stencil_offset_code); by_slot: b is the home cell, in the Morton order of the cells. Ranks by counting (a few hundred cells; no two keys are equal), by a
-// workgroup with `keys` in LDS.
+// (stencil_offset_code); by_slot: b is the home cell, and the cells are in their own Morton
+// order. Ranks by counting (a few hundred cells; no two keys are equal), by a workgroup with
+// `keys` in LDS.
 __device__ inline void stencil_list(const int4* __restrict__ offsets, uint32_t n, int level, uint32_t b, bool by_slot,
 									uint32_t* __restrict__ codes, uint64_t* keys) {
 	const int p[3] = {int(compact_by3(b >> 2)), int(compact_by3(b >> 1)), int(compact_by3(b))};

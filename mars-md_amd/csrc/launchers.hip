@@ -572,9 +572,9 @@ void launch_resolve_pair_tables(const int32_t* pairs, const int32_t* types, cons
 }
 
 // From 2^18 pairs on the sums in LDS pay for lists that run along their particles and cost
-// one in random order about 1%; below, a workgroup's 2048 pairs leave too few workgroups. Microseconds without and with, in pairlist, sorted
-// and random order: 2^17 pairs 46, 39, 38 and 25, 43, 42; 2^18 pairs 86, 74, 74 and
-// 29, 60, 75.
+// one in random order about 1%; below, a workgroup's 2048 pairs leave too few workgroups.
+// Microseconds without and with, in pairlist, sorted and random order: 2^17 pairs 46, 39, 38
+// and 25, 43, 42; 2^18 pairs 86, 74, 74 and 29, 60, 75.
 static bool pair_sums(uint64_t np) { return np >= (uint64_t(1) << 18); }
 static unsigned pair_block(uint64_t np) { return pair_sums(np) ? kPairBlock : 256; }
 static unsigned pair_grid(uint64_t np) {

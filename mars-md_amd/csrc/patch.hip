@@ -390,14 +390,11 @@ __device__ __forceinline__ void stage_step(const marsmd_particle_types& types, c
 // 392 instead of 377, 300k 135 and 137), with the tricubic sampler, which alone would take
 // about 140, to 128 (4 waves).
 template<int INTEG, bool ENERGY, bool ANALYTIC, int PMF>
-__global__ __launch_bounds__(kBlock, PMF == kPmfCubic ? 4 : 5) void k_step(const float4* __restrict__ pos, float4* __restrict__ pos_next,
-												 float4* __restrict__ mom, float4* __restrict__ force, uint64_t n,
-												 NbrList L, const NbTables* __restrict__ T_dev,
-												 const float* __restrict__ knots_g,
-												 const marsmd_particle_types* __restrict__ types_dev,
-												 const marsmd_grid_view* __restrict__ grids, StepParams S,
-												 int has_bonded, int store_force, const float4* __restrict__ pmf_in,
-												 PruneView PR) {
+__global__ __launch_bounds__(kBlock, PMF == kPmfCubic ? 4 : 5) void k_step(
+	const float4* __restrict__ pos, float4* __restrict__ pos_next, float4* __restrict__ mom, float4* __restrict__ force,
+	uint64_t n, NbrList L, const NbTables* __restrict__ T_dev, const float* __restrict__ knots_g,
+	const marsmd_particle_types* __restrict__ types_dev, const marsmd_grid_view* __restrict__ grids, StepParams S,
+	int has_bonded, int store_force, const float4* __restrict__ pmf_in, PruneView PR) {
 	extern __shared__ float lds_knots[];
 	__shared__ NbLds lds_nb;
 	__shared__ marsmd_particle_types lds_types;

@@ -141,6 +141,8 @@ def test_the_kernels_that_run(cuda, n, lanes_kernel, given):
         p.run(3, first_step=1)
         cuda.cuda.synchronize()
     names = [e.name for e in prof.events()]
+    if not any("mmd::" in x for x in names):
+        pytest.skip("the profiler records no kernels here")
     steps = [x for x in names if "k_step<" in x or "k_step_split<" in x]
     assert len(steps) == 3 and all(lanes_kernel in x for x in steps), names
     assert sum("k_pmf_force" in x for x in names) == (3 if given else 0), names
